@@ -90,6 +90,18 @@ int jfx_contract_f32(const float* A, int M, int K, const float* X, float* Y, lon
 int jfx_split_matrix(const double* A, int M, int K, int mode, int nslices, unsigned short* slices,
                      double* rowscale, hipStream_t stream);
 
+/* Per-axis contraction by operators whose even and odd parts decouple (any Q):
+ * mode 1 evaluates a parity basis on a symmetric mesh, A[M-1-m, k] = sgn
+ * (-1)^k A[m, k]; mode 2 projects from it, A[m, K-1-k] = sgn (-1)^m A[m, k];
+ * mode 3 has A[m, k] = 0 unless m + k is even (sgn 1) or odd (sgn -1), and with
+ * bp, bq >= 0 also zero outside -bp <= k - m <= bq; mode 0 has no structure.
+ * The operator is read as MFMA fragments that jfx_par_prepare writes (dtype 0
+ * FP64, 1 FP32; jfx_par_frag_elems values, 0 = sizes not taken). */
+long long jfx_par_frag_elems(int M, int K, int mode);
+int jfx_par_prepare(int dtype, const double* A, int M, int K, int mode, int sgn, void* frag, hipStream_t stream);
+int jfx_contract_par(int dtype, const void* frag, int M, int K, int mode, int sgn, int bp, int bq, const void* X,
+                     void* Y, long long P, long long Q, hipStream_t stream);
+
 /* BF16 float-split contraction on FP32 data: nslices 2 -> 3 products,
  * 3 -> 6 products, FP32 accumulation.  Same reference interface as above. */
 int jfx_contract_bf16x(const unsigned short* Aslices, int nslices, int M, int K, const float* X,

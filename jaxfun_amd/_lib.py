@@ -36,6 +36,10 @@ SIGNATURES: dict[str, tuple] = {
     "jfx_contract_f64": (c_int, [c_vp, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),
     "jfx_contract_f32": (c_int, [c_vp, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),
     "jfx_split_matrix": (c_int, [c_vp, c_int, c_int, c_int, c_int, c_vp, c_vp, c_vp]),
+    "jfx_par_frag_elems": (c_ll, [c_int, c_int, c_int]),
+    "jfx_par_prepare": (c_int, [c_int, c_vp, c_int, c_int, c_int, c_int, c_vp, c_vp]),
+    "jfx_contract_par": (c_int, [c_int, c_vp, c_int, c_int, c_int, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll,
+                                 c_vp]),
     "jfx_contract_bf16x": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),
     "jfx_contract_ozaki": (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),
     "jfx_split_matrix_i8": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_vp, c_vp]),

@@ -230,7 +230,7 @@ class Composite(OrthogonalSpace):
         if key not in self._ops:
             L = self.scalar_product_operator(N).A64.clone()
             K.band_lu_solve(self.mass_lu(), self.bandwidth, self.bandwidth, L, 0)
-            self._ops[key] = K.AxisOperator(L)
+            self._ops[key] = K.AxisOperator(L, K.projects_parity() if self.has_parity() else None)
         return self._ops[key]
 
     def to_orthogonal(self, c):
@@ -241,7 +241,8 @@ class Composite(OrthogonalSpace):
         ST = self._ops.get("ST")
         if ST is None:
             ST = self._ops["ST"] = K.AxisOperator(
-                torch.tensor(self.stencil_matrix().T.copy(), dtype=torch.float64, device=K.device()))
+                torch.tensor(self.stencil_matrix().T.copy(), dtype=torch.float64, device=K.device()),
+                K.host_structure(np.asarray(self.stencil_matrix()).T))
         return K.apply_along(ST, c, c.ndim - 1, "f64")
 
     def from_orthogonal(self, a):

@@ -171,7 +171,8 @@ def test_operator(v, i: int, Nq: int) -> K.AxisOperator:
         df = float(v.orthogonal.domain_factor)
         Pi = v.orthogonal.vandermonde(x, i)
         T = K.scale_transpose(Pi.contiguous(), w.contiguous(), None, df ** (i - 1))
-        v._ops[key] = K.AxisOperator(_stencil_apply(v, T, 0).contiguous())
+        v._ops[key] = K.AxisOperator(_stencil_apply(v, T, 0).contiguous(),
+                                     K.projects_parity((-1) ** i) if v.has_parity() else None)
     return v._ops[key]
 
 

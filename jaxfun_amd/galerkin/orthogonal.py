@@ -185,13 +185,27 @@ class OrthogonalSpace:
         V = self.orthogonal.vandermonde(X, k)
         return self._apply_stencil_cols(V)
 
+    def has_parity(self) -> bool:
+        """Basis function n is even or odd with n on a symmetric reference
+        interval (and Gauss meshes are symmetric): Legendre, Chebyshev and
+        Jacobi families with alpha = beta, under a stencil that couples equal
+        parities only."""
+        key = "has_parity"
+        if key not in self._ops:
+            V = self.orthogonal
+            ok = V.family in ("legendre", "chebyshev") or (hasattr(V, "alpha") and V.alpha == V.beta)
+            # stencil: {shift: coefficients} of phi_n = sum_o c_o psi_{n+o}, None for lifting functions
+            self._ops[key] = ok and self.stencil is not None and all(o % 2 == 0 for o in self.stencil)
+        return self._ops[key]
+
     def _stencil_dev(self):
         S = self.stencil_matrix()
         if S is None:
             return None
         key = "S"
         if key not in self._ops:
-            self._ops[key] = K.AxisOperator(torch.tensor(S, dtype=torch.float64, device=K.device()))
+            self._ops[key] = K.AxisOperator(torch.tensor(S, dtype=torch.float64, device=K.device()),
+                                            K.host_structure(np.asarray(S)))
         return self._ops[key]
 
     def _apply_stencil_cols(self, V: torch.Tensor) -> torch.Tensor:
@@ -211,7 +225,8 @@ class OrthogonalSpace:
         if key not in self._ops:
             X = self._points(kind, N)
             V = self.orthogonal._vander(X, k, float(self.domain_factor) ** k)
-            self._ops[key] = K.AxisOperator(self._apply_stencil_cols(V))
+            par = K.evaluates_parity((-1) ** k) if kind == MeshKind.QUADRATURE and self.has_parity() else None
+            self._ops[key] = K.AxisOperator(self._apply_stencil_cols(V), par)
         return self._ops[key]
 
     def _weighted_vt(self, N: int) -> torch.Tensor:
@@ -227,7 +242,8 @@ class OrthogonalSpace:
         if key not in self._ops:
             WVt = self._weighted_vt(N)
             S = self._stencil_dev()
-            self._ops[key] = K.AxisOperator(WVt if S is None else K.apply_along(S, WVt, 0, "f64"))
+            self._ops[key] = K.AxisOperator(WVt if S is None else K.apply_along(S, WVt, 0, "f64"),
+                                            K.projects_parity() if self.has_parity() else None)
         return self._ops[key]
 
     def forward_operator(self, N: int | None = None) -> K.AxisOperator:
@@ -238,7 +254,8 @@ class OrthogonalSpace:
             x, w = self.quad_points_and_weights(N)
             V = self.orthogonal._vander(x, 0)
             invh = torch.tensor(1.0 / self.norm_squared(), dtype=torch.float64, device=x.device)
-            self._ops[key] = K.AxisOperator(K.scale_transpose(V, w, invh, 1.0))
+            self._ops[key] = K.AxisOperator(K.scale_transpose(V, w, invh, 1.0),
+                                            K.projects_parity() if self.has_parity() else None)
         return self._ops[key]
 
     # ------------------------------------------------------------ 1D transforms

@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import math
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -400,8 +401,49 @@ def dense_lu_solve(LU: torch.Tensor, perm: torch.Tensor, B: torch.Tensor) -> tor
 # ---------------------------------------------------------------- per-axis contraction
 
 
+PAR_KEYS = {"f64": "par_f64", "f32": "par_f32"}
+PAR_DENSE, PAR_EVAL, PAR_PROJ, PAR_MIX = range(4)  # operator structures of csrc/contract_par.hip
+
+
+def evaluates_parity(sgn: int = 1) -> tuple:
+    """Structure of a (mesh x modes) operator on a symmetric mesh:
+    A[M-1-m, k] = sgn (-1)^k A[m, k]."""
+    return (PAR_EVAL, sgn, -1, -1)
+
+
+def projects_parity(sgn: int = 1) -> tuple:
+    """Structure of a (modes x mesh) operator: A[m, K-1-k] = sgn (-1)^m A[m, k]."""
+    return (PAR_PROJ, sgn, -1, -1)
+
+
+def mixes_parity(sgn: int = 1, p: int = -1, q: int = -1) -> tuple:
+    """Structure of a (modes x modes) operator that couples equal (sgn = 1) or
+    opposite (sgn = -1) parities only, with ``p`` lower and ``q`` upper bands
+    (-1: all)."""
+    return (PAR_MIX, sgn, p, q)
+
+
+def host_structure(A: np.ndarray) -> tuple | None:
+    """:func:`mixes_parity` of a host matrix whose entries vanish exactly on
+    every second diagonal, else None."""
+    if np.iscomplexobj(A) or A.ndim != 2 or 0 in A.shape or not np.all(np.isfinite(A)):
+        return None
+    r, c = np.nonzero(A)
+    if r.size == 0:
+        return None
+    d = c - r
+    odd = (d & 1).astype(bool)
+    if odd.any() and not odd.all():
+        return None
+    return mixes_parity(-1 if odd.any() else 1, max(0, int(-d.min())), max(0, int(d.max())))
+
+
 class AxisOperator:
     """A constant (M x K) matrix applied along one axis, prepared per precision.
+
+    ``parity``: its structure (:func:`evaluates_parity`, :func:`projects_parity`,
+    :func:`mixes_parity`), which FP64 and FP32 contractions use to halve their
+    products; the caller vouches for it up to rounding.
 
     ``f64`` uses the FP64 matrix; ``f32`` an FP32 copy; ``bf16x3``/``bf16x6``
     2/3 bf16 float slices; ``ozakiS`` S fixed-point digit slices with
@@ -410,12 +452,42 @@ class AxisOperator:
     reference caches factorizations on its matrix objects.
     """
 
-    def __init__(self, A: torch.Tensor):
+    def __init__(self, A: torch.Tensor, parity: tuple | None = None):
         if A.dtype != torch.float64:
             A = A.to(torch.float64)
         self.A64 = A.contiguous()
         self.M, self.K = self.A64.shape
+        self.parity = parity
         self._prep: dict[str, tuple] = {}
+
+    def t(self) -> "AxisOperator":
+        """The transposed operator, its structure transposed with it."""
+        par = self.parity
+        if par is not None:
+            mode, sgn, p, q = par
+            par = ({PAR_EVAL: PAR_PROJ, PAR_PROJ: PAR_EVAL, PAR_MIX: PAR_MIX}[mode], sgn, q, p)
+        return AxisOperator(self.A64.t().contiguous(), par)
+
+    def fragments(self, prec: str):
+        """MFMA fragments of ``csrc/contract_par.hip`` and their structure
+        ``(fragments, mode, sgn, p, q)`` for ``prec`` f64 or f32, or None where
+        the sizes are not taken.  A first use inside a graph capture gives None
+        too: the capture would record the preparation instead of running it."""
+        key = PAR_KEYS[prec]
+        fr = self._prep.get(key, 0)
+        if fr != 0:
+            return fr
+        mode, sgn, p, q = self.parity or (PAR_DENSE, 1, -1, -1)
+        n = _lib.load().jfx_par_frag_elems(self.M, self.K, mode)
+        if n == 0:
+            self._prep[key] = None
+            return None
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        f = torch.empty(n, dtype=io_dtype(prec), device=self.A64.device)
+        _lib.call("jfx_par_prepare", 0 if prec == "f64" else 1, _p(self.A64), self.M, self.K, mode, sgn, _p(f), _s())
+        self._prep[key] = (f, mode, sgn, p, q)
+        return self._prep[key]
 
     def _padded(self):
         """Zero-pad K to a multiple of 32 (the slice row stride the kernels read)."""
@@ -506,6 +578,11 @@ def _apply_complex(op: ComplexAxisOperator, X: torch.Tensor, axis: int) -> torch
     return Y
 
 
+def _use_fragments(op: AxisOperator, Q: int) -> bool:
+    """Whether FP64/FP32 contractions of ``op`` run from MFMA fragments."""
+    return op.parity is not None or not (Q == 1 or Q % 64 == 0)
+
+
 def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
                 out: torch.Tensor | None = None) -> torch.Tensor:
     """``Y = A`` applied along ``axis`` of X: Y[p, m, q] = sum_k A[m, k] X[p, k, q].
@@ -543,6 +620,12 @@ def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
         _req(out, dt, "out")
         if list(out.shape) != shape:
             raise ValueError("apply_along: bad out shape")
+    if prec in ("f64", "f32") and P * Q > 0 and _use_fragments(op, Q):
+        fr = op.fragments(prec)
+        if fr is not None:
+            _lib.call("jfx_contract_par", 0 if prec == "f64" else 1, _p(fr[0]), op.M, K, fr[1], fr[2], fr[3], fr[4],
+                      _p(X), _p(Y), P, Q, _s())
+            return Y
     prep = op.prepared(prec)
     if prec == "f64":
         _lib.call("jfx_contract_f64", _p(prep[0]), op.M, K, _p(X), _p(Y), P, Q, _s())

@@ -74,7 +74,8 @@ class BaseMatrix:
 
     def operator(self):
         if self._op is None:
-            self._op = K.ComplexAxisOperator(self.todense()) if self.is_complex else K.AxisOperator(self.todense())
+            self._op = K.ComplexAxisOperator(self.todense()) if self.is_complex else \
+                K.AxisOperator(self.todense(), K.host_structure(self._host_data))
         return self._op
 
     def diagonal_or_none(self) -> np.ndarray | None:

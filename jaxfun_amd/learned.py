@@ -131,17 +131,17 @@ class VarCoeffPoisson2D:
         self.TB = test_operator(S, 0, N)
         self.TD = test_operator(S, 1, N)
         self.F = S.forward_operator(N)
-        self.FT = K.AxisOperator(self.F.A64.t().contiguous())
-        self.BT = K.AxisOperator(self.B.A64.t().contiguous())
+        self.FT = self.F.t()
+        self.BT = self.B.t()
         x, w = S.quad_points_and_weights(N)
         self.w2 = (w[:, None] * w[None, :]).contiguous()
-        self.Vg = K.AxisOperator(K.vandermonde("legendre", x, gmodes))          # (Q, gm)
-        self.VgT = K.AxisOperator(self.Vg.A64.t().contiguous())                # (gm, Q)
+        self.Vg = K.AxisOperator(K.vandermonde("legendre", x, gmodes), K.evaluates_parity())  # (Q, gm)
+        self.VgT = self.Vg.t()                                                 # (gm, Q)
         h = 2.0 / (2 * np.arange(N) + 1.0)
         SH = np.zeros((N - 2, N))
         SH[np.arange(N - 2), np.arange(N - 2)] = h[:N - 2]
         SH[np.arange(N - 2), np.arange(2, N)] = -h[2:]
-        self.SH = K.AxisOperator(torch.tensor(SH, device=K.device()))         # S diag(h)
+        self.SH = K.AxisOperator(torch.tensor(SH, device=K.device()), K.host_structure(SH))  # S diag(h)
         v, u = TestFunction(self.T), TrialFunction(self.T)
         self.L = inner(Div(Grad(u)) * v, sparse=True).scale(-1.0).fd_factor()  # (grad v, grad u)
 
