@@ -102,6 +102,17 @@ int jfx_par_prepare(int dtype, const double* A, int M, int K, int mode, int sgn,
 int jfx_contract_par(int dtype, const void* frag, int M, int K, int mode, int sgn, int bp, int bq, const void* X,
                      void* Y, long long P, long long Q, hipStream_t stream);
 
+/* Both axes of (K0 x K1) slabs in one launch, all dims <= 128, operators of one
+ * mode (1, 2 or 3) given by their FP64 fragments:
+ * Y[b] = alpha A0 X[b] A1^T, then / E (epi 1), * E (2) or * E[b] (3), then added to
+ * Y (accum).  jfx_plane_fd_par: Y[b] = V0 ((W0 X[b] W1^T) / E) V1^T with mode-3
+ * operators (sgn 1). */
+int jfx_plane_par(int mode, const double* F0, int M0, int K0, int sgn0, int bp0, int bq0, const double* F1, int M1,
+                  int K1, int sgn1, int bp1, int bq1, const double* X, double* Y, const double* E, int epi,
+                  double alpha, int accum, long long B, hipStream_t stream);
+int jfx_plane_fd_par(const double* W0, const double* W1, const double* V0, const double* V1, const double* X,
+                     double* Y, const double* E, long long B, int n0, int n1, hipStream_t stream);
+
 /* BF16 float-split contraction on FP32 data: nslices 2 -> 3 products,
  * 3 -> 6 products, FP32 accumulation.  Same reference interface as above. */
 int jfx_contract_bf16x(const unsigned short* Aslices, int nslices, int M, int K, const float* X,

@@ -32,11 +32,9 @@
 // the parity order) times 16 columns, see lds_stride().
 // `band`: operators with A[m, k] = 0 outside -bp <= k - m <= bq skip the k-steps
 // a row block does not touch (mass matrices: 5 of 16; triangular stiffness: half).
-#include "jfx_common.h"
+#include "par_blocks.h"
 
 namespace jfx {
-
-enum { MODE_DENSE = 0, MODE_EVAL = 1, MODE_PROJ = 2, MODE_MIX = 3 };
 
 constexpr int PAR_MAXRB = 32;   // 16-row blocks of a part (M <= 1024 structured, 512 dense)
 constexpr int PAR_MAXK = 512;
@@ -411,6 +409,44 @@ static bool par_dims(int M, int K, int mode, ParDims& d) {
   return d.nrb <= PAR_MAXRB && K <= PAR_MAXK;
 }
 
+// k-steps [lo, hi) (even numbers) in which row block rb of part h is not zero
+static void par_range(const ParDims& d, int mode, int sgn, int bp, int bq, int h, int rb, short& lo, short& hi) {
+  int k0 = 0, k1 = d.Kh - 1;
+  if (mode == MODE_MIX && bp >= 0 && bq >= 0) {
+    // rows 2 m + r, columns 2 k + h: -bp <= 2 (k - m) + h - r <= bq
+    const int r = sgn < 0 ? 1 - h : h, m0 = 16 * rb, m1 = m0 + 15 < d.Mh - 1 ? m0 + 15 : d.Mh - 1;
+    k0 = m0 + (r - h - bp >= 0 ? (r - h - bp + 1) / 2 : -((bp + h - r) / 2));
+    k1 = m1 + (r - h + bq >= 0 ? (r - h + bq) / 2 : -((h - r - bq + 1) / 2));
+    if (k0 < 0) k0 = 0;
+    if (k1 > d.Kh - 1) k1 = d.Kh - 1;
+  }
+  lo = (short)(k0 <= k1 ? 2 * (k0 / 8) : 0);
+  hi = (short)(k0 <= k1 ? 2 * (k1 / 8 + 1) : 0);
+}
+
+// Descriptor of a structured operator for the slab kernels (at most 128 rows:
+// four half row blocks); k-step ranges cover both parts.
+bool par_op(const double* frag, int M, int K, int mode, int sgn, int bp, int bq, ParOp& o) {
+  ParDims d;
+  if (!par_dims(M, K, mode, d) || d.nrb > 4 || K > SLAB_MAX || (sgn != 1 && sgn != -1)) return false;
+  o.f = frag;
+  o.M = M;
+  o.K = K;
+  o.S = d.S;
+  o.nrb = d.nrb;
+  o.sgn = sgn;
+  for (int rb = 0; rb < 4; ++rb) o.lo[rb] = o.hi[rb] = 0;
+  for (int rb = 0; rb < d.nrb; ++rb) {
+    short lo[2], hi[2];
+    for (int h = 0; h < 2; ++h) par_range(d, mode, sgn, bp, bq, h, rb, lo[h], hi[h]);
+    if (lo[0] >= hi[0]) lo[0] = lo[1], hi[0] = hi[1];
+    if (lo[1] >= hi[1]) lo[1] = lo[0], hi[1] = hi[0];
+    o.lo[rb] = (signed char)(lo[0] < lo[1] ? lo[0] : lo[1]);
+    o.hi[rb] = (signed char)(hi[0] > hi[1] ? hi[0] : hi[1]);
+  }
+  return true;
+}
+
 template <typename T, int MODE, bool QONE, int NB, int JB>
 static int launch_par3(const T* Af, const T* X, T* Y, const ParMap& pm, hipStream_t st) {
   const int kz = par_kz(MODE, pm.K, pm.S);
@@ -472,19 +508,7 @@ static int launch_par(const T* Af, int M, int K, int mode, int sgn, int bp, int 
   pm.nt = run % (128 / (int)sizeof(T)) == 0 && ((uintptr_t)Y & 127) == 0 &&
           pm.ncols * M * (long long)sizeof(T) >= (64LL << 20);
   for (int h = 0; h < 2; ++h)
-    for (int rb = 0; rb < d.nrb; ++rb) {
-      int k0 = 0, k1 = d.Kh - 1;
-      if (mode == MODE_MIX && bp >= 0 && bq >= 0) {
-        // rows 2 m + r, columns 2 k + h: -bp <= 2 (k - m) + h - r <= bq
-        const int r = sgn < 0 ? 1 - h : h, m0 = 16 * rb, m1 = m0 + 15 < d.Mh - 1 ? m0 + 15 : d.Mh - 1;
-        k0 = m0 + (r - h - bp >= 0 ? (r - h - bp + 1) / 2 : -((bp + h - r) / 2));
-        k1 = m1 + (r - h + bq >= 0 ? (r - h + bq) / 2 : -((h - r - bq + 1) / 2));
-        if (k0 < 0) k0 = 0;
-        if (k1 > d.Kh - 1) k1 = d.Kh - 1;
-      }
-      pm.lo[h][rb] = (short)(k0 <= k1 ? 2 * (k0 / 8) : 0);
-      pm.hi[h][rb] = (short)(k0 <= k1 ? 2 * (k1 / 8 + 1) : 0);
-    }
+    for (int rb = 0; rb < d.nrb; ++rb) par_range(d, mode, sgn, bp, bq, h, rb, pm.lo[h][rb], pm.hi[h][rb]);
   switch (mode) {
     case MODE_DENSE: return launch_par2<T, MODE_DENSE>(Af, X, Y, pm, st);
     case MODE_EVAL: return launch_par2<T, MODE_EVAL>(Af, X, Y, pm, st);

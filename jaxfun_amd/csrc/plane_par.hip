@@ -1,0 +1,206 @@
+// Fused two-axis FP64 contractions of 2D slabs by operators with decoupled even
+// and odd parts (contract_par.hip):
+//     Y[b] = alpha A0 X[b] A1^T,  optionally / E, * E or * E[b],  optionally + Y[b]
+// and the fast-diagonalisation solve  Y[b] = V0 ((W0 X[b] W1^T) / E) V1^T.
+//
+// A slab is read once and written once; the intermediate stays in LDS
+// (par_blocks.h).  One workgroup per slab: 4 waves up to 64 x 64 (37 KB of LDS,
+// four workgroups per CU), 16 waves for larger slabs (139 KB at 128 x 128).
+#include "par_blocks.h"
+
+namespace jfx {
+
+struct SlabMap {
+  ParOp o0, o1;  // axis 0 (M0 x K0), axis 1 (M1 x K1)
+  const double* E;
+  int epi;  // 0 none, 1 divide by E, 2 multiply by E, 3 multiply by E[b]
+  int accum;
+  double alpha;
+};
+
+template <int MODE, int NW>
+__global__ __launch_bounds__(64 * NW) void plane_par_kernel(const double* __restrict__ X, double* __restrict__ Y,
+                                                            SlabMap sm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  double* S = reinterpret_cast<double*>(smem);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int K0 = sm.o0.K, K1 = sm.o1.K, M0 = sm.o0.M, M1 = sm.o1.M;
+  const long long b = blockIdx.x;
+  slab_stage<64 * NW>(X + b * K0 * K1, K0, K1, S);
+  __syncthreads();
+  Acc4 acc;
+  acc_zero(acc);
+  const WaveA wa = wave_a(w, K0, sm.o1);
+  if (wa.on) phase_a<MODE>(S, slab_ldx(K1), sm.o1, wa, acc);
+  __syncthreads();
+  const int LDT = slab_ldt(M1);
+  if (wa.on) store_t<MODE>(S, LDT, sm.o1, wa, acc);
+  __syncthreads();
+  double* Yb = Y + b * M0 * M1;
+  const double* E = sm.epi == 3 ? sm.E + b * M0 * M1 : sm.E;
+  const int nit = items_b(sm.o0, M1);
+  for (int it = w; it < nit; it += NW) {
+    const ItemB ib = item_b(it, sm.o0, M1);
+    acc_zero(acc);
+    phase_b<MODE>(S, LDT, sm.o0, ib, acc);
+    each_b<MODE>(sm.o0, ib, M1, acc, [&](int m, int c, double v) {
+      const int i = m * M1 + c;
+      v *= sm.alpha;
+      if (sm.epi == 1)
+        v /= E[i];
+      else if (sm.epi)
+        v *= E[i];
+      if (sm.accum) v += Yb[i];
+      Yb[i] = v;
+    });
+  }
+}
+
+struct FdMap {
+  ParOp w0, w1, v0, v1;
+  const double* E;
+};
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void plane_fd_par_kernel(const double* __restrict__ X, double* __restrict__ Y,
+                                                               FdMap fm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  double* S = reinterpret_cast<double*>(smem);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = fm.w0.K, n1 = fm.w1.K;
+  const long long b = blockIdx.x;
+  const int LDX = slab_ldx(n1), LDT = slab_ldt(n1);
+  slab_stage<64 * NW>(X + b * n0 * n1, n0, n1, S);
+  __syncthreads();
+  Acc4 acc;
+  const WaveA wa = wave_a(w, n0, fm.w1);
+  const bool onb = w < items_b(fm.w0, n1);  // NW covers every item
+  const ItemB ib = item_b(w, fm.w0, n1);
+  acc_zero(acc);
+  if (wa.on) phase_a<MODE_MIX>(S, LDX, fm.w1, wa, acc);
+  __syncthreads();
+  if (wa.on) store_t<MODE_MIX>(S, LDT, fm.w1, wa, acc);
+  __syncthreads();
+  acc_zero(acc);
+  if (onb) phase_b<MODE_MIX>(S, LDT, fm.w0, ib, acc);
+  __syncthreads();
+  // G / E back into LDS as the second pass's input, zero padded like a staged slab
+  if (onb)
+    each_b<MODE_MIX>(fm.w0, ib, n1, acc, [&](int m, int c, double v) { S[m * LDX + c] = v / fm.E[m * n1 + c]; });
+  {
+    const int C = slab_pad(n1), R = slab_pad(n0), nz = C - n1;
+    if (nz)
+      for (int e = threadIdx.x; e < n0 * nz; e += 64 * NW) {
+        const int i = e / nz;
+        S[i * LDX + n1 + (e - i * nz)] = 0.0;
+      }
+    for (int e = threadIdx.x; e < (R - n0) * C; e += 64 * NW) {
+      const int i = e / C;
+      S[(n0 + i) * LDX + (e - i * C)] = 0.0;
+    }
+  }
+  __syncthreads();
+  acc_zero(acc);
+  if (wa.on) phase_a<MODE_MIX>(S, LDX, fm.v1, wa, acc);
+  __syncthreads();
+  if (wa.on) store_t<MODE_MIX>(S, LDT, fm.v1, wa, acc);
+  __syncthreads();
+  acc_zero(acc);
+  if (onb) {
+    phase_b<MODE_MIX>(S, LDT, fm.v0, ib, acc);
+    double* Yb = Y + b * n0 * n1;
+    each_b<MODE_MIX>(fm.v0, ib, n1, acc, [&](int m, int c, double v) { Yb[m * n1 + c] = v; });
+  }
+}
+
+bool par_op(const double* frag, int M, int K, int mode, int sgn, int bp, int bq, ParOp& o);
+
+// waves that phase A of (K0 rows) x (operator o1) needs, 4 or 16
+static int slab_waves(int K0, const ParOp& o0, const ParOp& o1) {
+  const int a = (slab_pad(K0) / 16) * ((o1.nrb + 1) / 2), b = o0.nrb * ((slab_pad(o1.M) / 16 + 1) / 2);
+  const int n = a > b ? a : b;
+  return n <= 4 ? 4 : n <= 8 ? 8 : 16;
+}
+
+template <typename K>
+static int slab_shm(K kern, size_t shm) {
+  if (shm > 64 * 1024)
+    JFX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+  return JFX_OK;
+}
+
+template <int MODE, int NW>
+static int launch_plane(const double* X, double* Y, const SlabMap& sm, long long B, hipStream_t st) {
+  const size_t shm = (size_t)slab_lds(sm.o0.K, sm.o1.K, sm.o1.M) * sizeof(double);
+  const int rc = slab_shm(plane_par_kernel<MODE, NW>, shm);
+  if (rc) return rc;
+  hipLaunchKernelGGL((plane_par_kernel<MODE, NW>), dim3((unsigned)B), dim3(64 * NW), shm, st, X, Y, sm);
+  JFX_LAUNCH_CHECK();
+  return JFX_OK;
+}
+
+template <int MODE>
+static int launch_plane_w(const double* X, double* Y, const SlabMap& sm, long long B, hipStream_t st) {
+  switch (slab_waves(sm.o0.K, sm.o0, sm.o1)) {
+    case 4: return launch_plane<MODE, 4>(X, Y, sm, B, st);
+    case 8: return launch_plane<MODE, 8>(X, Y, sm, B, st);
+    default: return launch_plane<MODE, 16>(X, Y, sm, B, st);
+  }
+}
+
+template <int NW>
+static int launch_fd(const double* X, double* Y, const FdMap& fm, long long B, hipStream_t st) {
+  const size_t shm = (size_t)slab_lds(fm.w0.K, fm.w1.K, fm.w1.M) * sizeof(double);
+  const int rc = slab_shm(plane_fd_par_kernel<NW>, shm);
+  if (rc) return rc;
+  hipLaunchKernelGGL(plane_fd_par_kernel<NW>, dim3((unsigned)B), dim3(64 * NW), shm, st, X, Y, fm);
+  JFX_LAUNCH_CHECK();
+  return JFX_OK;
+}
+
+}  // namespace jfx
+
+using namespace jfx;
+
+extern "C" {
+
+int jfx_plane_par(int mode, const double* F0, int M0, int K0, int sgn0, int bp0, int bq0, const double* F1, int M1,
+                  int K1, int sgn1, int bp1, int bq1, const double* X, double* Y, const double* E, int epi,
+                  double alpha, int accum, long long B, hipStream_t stream) {
+  if (!F0 || !F1 || !X || !Y || (epi && !E)) return set_error("plane_par: null pointer"), JFX_EARG;
+  if (epi < 0 || epi > 3) return set_error("plane_par: epi must be 0..3"), JFX_EARG;
+  SlabMap sm;
+  if (mode < MODE_EVAL || mode > MODE_MIX || !par_op(F0, M0, K0, mode, sgn0, bp0, bq0, sm.o0) ||
+      !par_op(F1, M1, K1, mode, sgn1, bp1, bq1, sm.o1) || M0 > SLAB_MAX || K0 > SLAB_MAX || M1 > SLAB_MAX ||
+      K1 > SLAB_MAX || B < 0 || B > 0x7fffffffLL)
+    return set_error("plane_par: sizes (%d x %d), (%d x %d), %lld slabs, mode %d", M0, K0, M1, K1, B, mode), JFX_ESHAPE;
+  if (B == 0) return JFX_OK;
+  sm.E = E;
+  sm.epi = epi;
+  sm.alpha = alpha;
+  sm.accum = accum;
+  switch (mode) {
+    case MODE_EVAL: return launch_plane_w<MODE_EVAL>(X, Y, sm, B, stream);
+    case MODE_PROJ: return launch_plane_w<MODE_PROJ>(X, Y, sm, B, stream);
+    default: return launch_plane_w<MODE_MIX>(X, Y, sm, B, stream);
+  }
+}
+
+int jfx_plane_fd_par(const double* W0, const double* W1, const double* V0, const double* V1, const double* X,
+                     double* Y, const double* E, long long B, int n0, int n1, hipStream_t stream) {
+  if (!W0 || !W1 || !V0 || !V1 || !X || !Y || !E) return set_error("plane_fd_par: null pointer"), JFX_EARG;
+  FdMap fm;
+  if (!par_op(W0, n0, n0, MODE_MIX, 1, -1, -1, fm.w0) || !par_op(W1, n1, n1, MODE_MIX, 1, -1, -1, fm.w1) ||
+      !par_op(V0, n0, n0, MODE_MIX, 1, -1, -1, fm.v0) || !par_op(V1, n1, n1, MODE_MIX, 1, -1, -1, fm.v1) ||
+      n0 > SLAB_MAX || n1 > SLAB_MAX || B < 0 || B > 0x7fffffffLL)
+    return set_error("plane_fd_par: %lld slabs of %d x %d", B, n0, n1), JFX_ESHAPE;
+  if (B == 0) return JFX_OK;
+  fm.E = E;
+  switch (slab_waves(n0, fm.w0, fm.w1)) {
+    case 4: return launch_fd<4>(X, Y, fm, B, stream);
+    case 8: return launch_fd<8>(X, Y, fm, B, stream);
+    default: return launch_fd<16>(X, Y, fm, B, stream);
+  }
+}
+
+}  // extern "C"

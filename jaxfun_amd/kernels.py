@@ -666,6 +666,43 @@ def plane_ok(op0: AxisOperator, op1: AxisOperator, prec: str) -> bool:
     return prec in PLANE_PRECISIONS and max(op0.M, op0.K, op1.M, op1.K) <= 128
 
 
+def _slab_fragments(ops):
+    """FP64 fragments of structured operators for the fused slab kernels
+    (csrc/plane_par.hip): one structure, at most 128 rows and columns; else None."""
+    mode = None
+    out = []
+    for o in ops:
+        if type(o) is not AxisOperator or o.parity is None or o.M > 128 or o.K > 128:
+            return None
+        if mode is not None and o.parity[0] != mode:
+            return None
+        mode = o.parity[0]
+        fr = o.fragments("f64")
+        if fr is None:
+            return None
+        out.append(fr)
+    return out
+
+
+def slab_pays(op0, op1, nslabs: int) -> bool | None:
+    """Whether ``nslabs`` slabs run faster through the fused FP64 slab kernel than
+    axis by axis; None where that kernel does not take the operators.  A slab is
+    one workgroup's work: up to 64 x 64 always (256 slabs 12.0 us, per axis
+    16.5 us; one 10.2 / 14.9 us), larger ones when they occupy half the CUs
+    (128 x 128: 256 slabs 36 us, per axis 47 us; 64 slabs 28 us, per axis 20 us)."""
+    if any(type(o) is not AxisOperator or o.parity is None or max(o.M, o.K) > 128 for o in (op0, op1)) or \
+            op0.parity[0] != op1.parity[0]:
+        return None
+    return max(op0.M, op0.K, op1.M, op1.K) <= 64 or 2 * nslabs >= num_cus()
+
+
+def plane_fd_par_ok(ops) -> bool:
+    """The fused FP64 solve of operators that couple equal parities applies
+    (W0, W1, V0, V1 square, up to 128, the two axes of any sizes)."""
+    return all(type(o) is AxisOperator and o.parity == (PAR_MIX, 1, -1, -1) and o.M == o.K <= 128 for o in ops) and \
+        ops[0].M == ops[2].M and ops[1].M == ops[3].M
+
+
 def plane_fd_ok(ops, prec: str) -> bool:
     """The fused 2D solve applies: four real n x n operators, n <= 64 (FP64) or 128 (bf16x6)."""
     if prec not in ("f64", "bf16x6"):
@@ -684,6 +721,16 @@ def plane_fd(W0: AxisOperator, W1: AxisOperator, V0: AxisOperator, V1: AxisOpera
     dt = io_dtype(prec)
     _req(X, dt, "X")
     _req(E, dt, "E")
+    if prec == "f64" and plane_fd_par_ok([W0, W1, V0, V1]):
+        fr = _slab_fragments([W0, W1, V0, V1])
+        if fr is not None:
+            shape = (W0.M, W1.M)
+            if tuple(X.shape[-2:]) != shape or tuple(E.shape) != shape:
+                raise ValueError("plane_fd: operators, array or divisor do not fit the fused solve")
+            Y = torch.empty_like(X)
+            _lib.call("jfx_plane_fd_par", _p(fr[0][0]), _p(fr[1][0]), _p(fr[2][0]), _p(fr[3][0]), _p(X), _p(Y), _p(E),
+                      math.prod(X.shape[:-2]), W0.M, W1.M, _s())
+            return Y
     n = W0.M
     if not plane_fd_ok([W0, W1, V0, V1], prec) or tuple(X.shape[-2:]) != (n, n) or tuple(E.shape) != (n, n):
         raise ValueError("plane_fd: operators, array or divisor do not fit the fused solve")
@@ -740,6 +787,12 @@ def plane(op0: AxisOperator, op1: AxisOperator, X: torch.Tensor, prec: str = "f6
                   op1.M, op1.K, _s())
         return Y
     if prec == "f64":
+        fr = _slab_fragments((op0, op1))
+        if fr is not None:
+            (f0, md, s0, p0, q0), (f1, _, s1, p1, q1) = fr
+            _lib.call("jfx_plane_par", md, _p(f0), op0.M, op0.K, s0, p0, q0, _p(f1), op1.M, op1.K, s1, p1, q1, _p(X),
+                      _p(Y), _p(E), mode, float(alpha), acc, B, _s())
+            return Y
         _lib.call("jfx_plane_contract", 0, _p(op0.A64), _p(op1.A64), _p(None), _p(None), _p(X), _p(Y), _p(E),
                   mode, float(alpha), acc, B, op0.M, op0.K, op1.M, op1.K, _s())
     else:

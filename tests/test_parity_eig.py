@@ -1,0 +1,61 @@
+"""Eigenpairs of Dirichlet mass and stiffness pairs, diagonalised one parity at a
+time (la/tpmatrix.py axis_eig), against the fast-diagonalisation solve refined in
+extended precision."""
+
+import numpy as np
+import pytest
+
+from jaxfun_amd.la import tpmatrix as T
+
+
+def _pair(family, N):
+    n, k = N - 2, np.arange(N)
+    S = np.eye(n, N) - np.eye(n, N, 2)
+    if family == "legendre":
+        return S @ np.diag(2.0 / (2 * k + 1)) @ S.T, -np.diag(4.0 * np.arange(n) + 6.0)
+    h = np.full(N, np.pi / 2)
+    h[0] = np.pi
+    off = k[None, :] - k[:, None]
+    A = np.where((off >= 2) & (off % 2 == 0), k[None, :] * (k[None, :]**2 - k[:, None]**2) * np.pi / 2, 0.0)
+    return S @ np.diag(h) @ S.T, S @ A @ S.T
+
+
+def _solve_error(eig, M, K, F):
+    lam, V, W = eig
+    D = lam[:, None] + lam[None, :]
+
+    def once(R):
+        return V @ ((W @ R @ W.T) / D) @ V.T
+
+    X = once(F)
+    Y, Ml, Kl = (a.astype(np.longdouble) for a in (X, M, K))
+    for _ in range(3):
+        Y = Y + once((F - (Kl @ Y @ Ml.T + Ml @ Y @ Kl.T)).astype(np.float64))
+    return float(np.linalg.norm(X - Y) / np.linalg.norm(Y))
+
+
+@pytest.mark.parametrize("family", ["legendre", "chebyshev"])
+@pytest.mark.parametrize("N", [5, 6, 16, 33, 50, 64, 65, 100, 128])
+def test_parity_blocks(family, N):
+    M, K = _pair(family, N)
+    n = N - 2
+    lam, V, W = T.axis_eig(K, M)
+    assert np.all(np.diff(lam) >= 0)
+    order = T._parity_order(V, W)
+    assert order is not None
+    Vp, Wp = V[:, order], W[order]
+    odd = np.add.outer(np.arange(n), np.arange(n)) % 2 == 1
+    assert not Vp[odd].any() and not Wp[odd].any()
+    f = np.random.default_rng(N).standard_normal((n, n)) * np.outer((1.0 + np.arange(n))**-2, (1.0 + np.arange(n))**-2)
+    err, whole = _solve_error((lam, V, W), M, K, f), _solve_error(T._axis_eig(K, M), M, K, f)
+    assert err <= 1.2 * whole + 4e-16  # no further off than the pair diagonalised as a whole
+
+
+def test_pairs_without_parity_are_left_whole():
+    rng = np.random.default_rng(0)
+    A = rng.standard_normal((7, 7))
+    A = A + A.T
+    lam, V, W = T.axis_eig(A, np.eye(7))
+    ref = T._axis_eig(A, np.eye(7))
+    assert all(np.array_equal(a, b) for a, b in zip((lam, V, W), ref))
+    assert T._parity_order(V, W) is None
