@@ -140,6 +140,13 @@ def check(rc: int, what: str = "") -> None:
     raise JfxError(text)
 
 
+_bound: dict = {}  # entry points by name, once loaded
+
+
 def call(name: str, *args) -> None:
-    rc = getattr(load(), name)(*args)
-    check(rc, name)
+    fn = _bound.get(name)
+    if fn is None:
+        fn = _bound[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc != JFX_OK:
+        check(rc, name)

@@ -26,14 +26,24 @@ def device() -> torch.device:
 
 
 def _p(t: torch.Tensor | None):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    """Device address for a pointer argument (None: null)."""
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _s():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device, as an address.  The raw query
+    builds no Stream object (0.3 against 2 us per launch)."""
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _req(t: torch.Tensor, dtype: torch.dtype, name: str) -> None:
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous():
+        return
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a CUDA/HIP torch tensor")
     if t.dtype != dtype:
@@ -607,13 +617,16 @@ def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
         return Y
     dt = io_dtype(prec)
     _req(X, dt, "X")
-    axis = axis % X.ndim
-    K = X.shape[axis]
+    shape = list(X.shape)
+    axis = axis % len(shape)
+    K = shape[axis]
     if K != op.K:
         raise ValueError(f"apply_along: axis {axis} has length {K}, operator expects {op.K}")
-    P = math.prod(X.shape[:axis])
-    Q = math.prod(X.shape[axis + 1:])
-    shape = list(X.shape)
+    P = Q = 1
+    for n in shape[:axis]:
+        P *= n
+    for n in shape[axis + 1:]:
+        Q *= n
     shape[axis] = op.M
     Y = torch.empty(shape, dtype=dt, device=X.device) if out is None else out
     if out is not None:
