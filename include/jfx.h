@@ -105,13 +105,29 @@ int jfx_contract_par(int dtype, const void* frag, int M, int K, int mode, int sg
 /* Both axes of (K0 x K1) slabs in one launch, all dims <= 128, operators of one
  * mode (1, 2 or 3) given by their FP64 fragments:
  * Y[b] = alpha A0 X[b] A1^T, then / E (epi 1), * E (2) or * E[b] (3), then added to
- * Y (accum).  jfx_plane_fd_par: Y[b] = V0 ((W0 X[b] W1^T) / E) V1^T with mode-3
- * operators (sgn 1). */
+ * Y (accum).  jfx_plane_fd_par: Y[b] = scale[b] V0 ((W0 X[b] W1^T) / E) V1^T with
+ * mode-3 operators (sgn 1); scale may be null. */
 int jfx_plane_par(int mode, const double* F0, int M0, int K0, int sgn0, int bp0, int bq0, const double* F1, int M1,
                   int K1, int sgn1, int bp1, int bq1, const double* X, double* Y, const double* E, int epi,
                   double alpha, int accum, long long B, hipStream_t stream);
 int jfx_plane_fd_par(const double* W0, const double* W1, const double* V0, const double* V1, const double* X,
-                     double* Y, const double* E, long long B, int n0, int n1, hipStream_t stream);
+                     double* Y, const double* E, const double* scale, long long B, int n0, int n1,
+                     hipStream_t stream);
+
+/* Weak -div(k grad u) on (n x n) slabs over a (Q x Q) mesh, n, Q <= 128, FP64:
+ * Y[b] = TD (k[b] * (D U[b] B^T)) TB^T + TB (k[b] * (B U[b] D^T)) TD^T with fragments of
+ * mode-1 operators B, D (Q x n) and mode-2 operators TB, TD (n x Q) and their signs. */
+int jfx_weak_par(const double* FB, int sB, const double* FD, int sD, const double* FTB, int sTB, const double* FTD,
+                 int sTD, int n, int Q, const double* U, const double* k, double* Y, long long B, hipStream_t stream);
+
+/* Fused PCG steps over `batch` systems of n values, FP64.  jfx_pcg_step: for active
+ * systems a = rz / (p, q), x += a p, r -= a q, then the stopping test of jfx_pcg_check
+ * with count = 1; *left is increased by the number of systems that stay active.
+ * jfx_pcg_direction: for active systems s = (r, z), p = z + (s / rz) p, rz = s. */
+int jfx_pcg_step(double* x, double* r, const double* p, const double* q, const double* rz, const double* bb,
+                 double tol2, int* active, int* iters, int* left, int batch, long long n, hipStream_t stream);
+int jfx_pcg_direction(double* p, const double* z, const double* r, double* rz, const int* active, int batch,
+                      long long n, hipStream_t stream);
 
 /* BF16 float-split contraction on FP32 data: nslices 2 -> 3 products,
  * 3 -> 6 products, FP32 accumulation.  Same reference interface as above. */

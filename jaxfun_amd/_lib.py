@@ -42,7 +42,11 @@ SIGNATURES: dict[str, tuple] = {
                                  c_vp]),
     "jfx_plane_par": (c_int, [c_int, c_vp, c_int, c_int, c_int, c_int, c_int, c_vp, c_int, c_int, c_int, c_int, c_int,
                               c_vp, c_vp, c_vp, c_int, c_dbl, c_int, c_ll, c_vp]),
-    "jfx_plane_fd_par": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_ll, c_int, c_int, c_vp]),
+    "jfx_plane_fd_par": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_ll, c_int, c_int, c_vp]),
+    "jfx_weak_par": (c_int, [c_vp, c_int, c_vp, c_int, c_vp, c_int, c_vp, c_int, c_int, c_int, c_vp, c_vp, c_vp, c_ll,
+                             c_vp]),
+    "jfx_pcg_step": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_dbl, c_vp, c_vp, c_vp, c_int, c_ll, c_vp]),
+    "jfx_pcg_direction": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_ll, c_vp]),
     "jfx_contract_bf16x": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),
     "jfx_contract_ozaki": (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),
     "jfx_split_matrix_i8": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_vp, c_vp]),

@@ -40,11 +40,26 @@ __host__ __device__ inline int slab_lds(int K0, int K1, int M1) {
 
 typedef double d2 __attribute__((ext_vector_type(2)));
 
+// Zeros around a (K0 x K1) slab in LDS, rows and columns up to multiples of 16.
+template <int NT>
+__device__ __forceinline__ void slab_zero_pad(int K0, int K1, double* Xs) {
+  const int LDX = slab_ldx(K1), R = slab_pad(K0), C = slab_pad(K1), tid = threadIdx.x;
+  const int nz = C - K1;
+  if (nz)
+    for (int e = tid; e < K0 * nz; e += NT) {
+      const int i = e / nz;
+      Xs[i * LDX + K1 + (e - i * nz)] = 0.0;
+    }
+  for (int e = tid; e < (R - K0) * C; e += NT) {
+    const int i = e / C;
+    Xs[(K0 + i) * LDX + (e - i * C)] = 0.0;
+  }
+}
+
 // X (K0 x K1, contiguous) into LDS, rows LDX apart, zero padded to 16s.
 template <int NT>
 __device__ __forceinline__ void slab_stage(const double* __restrict__ X, int K0, int K1, double* Xs) {
-  const int LDX = slab_ldx(K1), R = slab_pad(K0), C = slab_pad(K1);
-  const int tid = threadIdx.x;
+  const int LDX = slab_ldx(K1), tid = threadIdx.x;
   constexpr int U = 8;
   if (K1 % 2 == 0 && ((uintptr_t)X & 15) == 0) {
     const unsigned kh = K1 / 2;
@@ -78,16 +93,7 @@ __device__ __forceinline__ void slab_stage(const double* __restrict__ X, int K0,
       }
     }
   }
-  const int nz = C - K1;  // columns K1.. of the rows that exist
-  if (nz)
-    for (int e = tid; e < K0 * nz; e += NT) {
-      const int i = e / nz;
-      Xs[i * LDX + K1 + (e - i * nz)] = 0.0;
-    }
-  for (int e = tid; e < (R - K0) * C; e += NT) {
-    const int i = e / C;
-    Xs[(K0 + i) * LDX + (e - i * C)] = 0.0;
-  }
+  slab_zero_pad<NT>(K0, K1, Xs);
 }
 
 // even and odd operand of k-step s from a row of X (element stride 1)

@@ -1,7 +1,7 @@
 // Fused two-axis FP64 contractions of 2D slabs by operators with decoupled even
 // and odd parts (contract_par.hip):
 //     Y[b] = alpha A0 X[b] A1^T,  optionally / E, * E or * E[b],  optionally + Y[b]
-// and the fast-diagonalisation solve  Y[b] = V0 ((W0 X[b] W1^T) / E) V1^T.
+// and the fast-diagonalisation solve  Y[b] = scale[b] V0 ((W0 X[b] W1^T) / E) V1^T.
 //
 // A slab is read once and written once; the intermediate stays in LDS
 // (par_blocks.h).  One workgroup per slab: 4 waves up to 64 x 64 (37 KB of LDS,
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(64 * NW) void plane_par_kernel(const double* __rest
 
 struct FdMap {
   ParOp w0, w1, v0, v1;
-  const double* E;
+  const double *E, *scale;  // scale: one factor per slab, or null
 };
 
 template <int NW>
@@ -87,18 +87,7 @@ __global__ __launch_bounds__(64 * NW) void plane_fd_par_kernel(const double* __r
   // G / E back into LDS as the second pass's input, zero padded like a staged slab
   if (onb)
     each_b<MODE_MIX>(fm.w0, ib, n1, acc, [&](int m, int c, double v) { S[m * LDX + c] = v / fm.E[m * n1 + c]; });
-  {
-    const int C = slab_pad(n1), R = slab_pad(n0), nz = C - n1;
-    if (nz)
-      for (int e = threadIdx.x; e < n0 * nz; e += 64 * NW) {
-        const int i = e / nz;
-        S[i * LDX + n1 + (e - i * nz)] = 0.0;
-      }
-    for (int e = threadIdx.x; e < (R - n0) * C; e += 64 * NW) {
-      const int i = e / C;
-      S[(n0 + i) * LDX + (e - i * C)] = 0.0;
-    }
-  }
+  slab_zero_pad<64 * NW>(n0, n1, S);
   __syncthreads();
   acc_zero(acc);
   if (wa.on) phase_a<MODE_MIX>(S, LDX, fm.v1, wa, acc);
@@ -109,14 +98,15 @@ __global__ __launch_bounds__(64 * NW) void plane_fd_par_kernel(const double* __r
   if (onb) {
     phase_b<MODE_MIX>(S, LDT, fm.v0, ib, acc);
     double* Yb = Y + b * n0 * n1;
-    each_b<MODE_MIX>(fm.v0, ib, n1, acc, [&](int m, int c, double v) { Yb[m * n1 + c] = v; });
+    const double f = fm.scale ? fm.scale[b] : 1.0;
+    each_b<MODE_MIX>(fm.v0, ib, n1, acc, [&](int m, int c, double v) { Yb[m * n1 + c] = v * f; });
   }
 }
 
 bool par_op(const double* frag, int M, int K, int mode, int sgn, int bp, int bq, ParOp& o);
 
 // waves that phase A of (K0 rows) x (operator o1) needs, 4 or 16
-static int slab_waves(int K0, const ParOp& o0, const ParOp& o1) {
+int slab_waves(int K0, const ParOp& o0, const ParOp& o1) {
   const int a = (slab_pad(K0) / 16) * ((o1.nrb + 1) / 2), b = o0.nrb * ((slab_pad(o1.M) / 16 + 1) / 2);
   const int n = a > b ? a : b;
   return n <= 4 ? 4 : n <= 8 ? 8 : 16;
@@ -187,7 +177,8 @@ int jfx_plane_par(int mode, const double* F0, int M0, int K0, int sgn0, int bp0,
 }
 
 int jfx_plane_fd_par(const double* W0, const double* W1, const double* V0, const double* V1, const double* X,
-                     double* Y, const double* E, long long B, int n0, int n1, hipStream_t stream) {
+                     double* Y, const double* E, const double* scale, long long B, int n0, int n1,
+                     hipStream_t stream) {
   if (!W0 || !W1 || !V0 || !V1 || !X || !Y || !E) return set_error("plane_fd_par: null pointer"), JFX_EARG;
   FdMap fm;
   if (!par_op(W0, n0, n0, MODE_MIX, 1, -1, -1, fm.w0) || !par_op(W1, n1, n1, MODE_MIX, 1, -1, -1, fm.w1) ||
@@ -196,6 +187,7 @@ int jfx_plane_fd_par(const double* W0, const double* W1, const double* V0, const
     return set_error("plane_fd_par: %lld slabs of %d x %d", B, n0, n1), JFX_ESHAPE;
   if (B == 0) return JFX_OK;
   fm.E = E;
+  fm.scale = scale;
   switch (slab_waves(n0, fm.w0, fm.w1)) {
     case 4: return launch_fd<4>(X, Y, fm, B, stream);
     case 8: return launch_fd<8>(X, Y, fm, B, stream);

@@ -657,6 +657,29 @@ def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
     return Y
 
 
+def weak_laplacian(B: AxisOperator, D: AxisOperator, TB: AxisOperator, TD: AxisOperator, k: torch.Tensor,
+                   U: torch.Tensor) -> torch.Tensor | None:
+    """``TD (k * (D U B^T)) TB^T + TB (k * (B U D^T)) TD^T`` per slab of U (FP64) in one
+    launch (csrc/weak_par.hip), or None where its operators do not fit: B, D
+    evaluate a parity basis and its derivative, TB, TD project, all up to 128."""
+    n, Q = B.K, B.M
+    if max(n, Q) > 128 or any(o.parity is None or o.parity[0] != md or (o.M, o.K) != sz for o, md, sz in (
+            (B, PAR_EVAL, (Q, n)), (D, PAR_EVAL, (Q, n)), (TB, PAR_PROJ, (n, Q)), (TD, PAR_PROJ, (n, Q)))):
+        return None
+    fr = [o.fragments("f64") for o in (B, D, TB, TD)]
+    if any(f is None for f in fr):
+        return None
+    _req(U, torch.float64, "U")
+    _req(k, torch.float64, "k")
+    nb = math.prod(U.shape[:-2])
+    if tuple(U.shape[-2:]) != (n, n) or tuple(k.shape) != tuple(U.shape[:-2]) + (Q, Q):
+        raise ValueError(f"weak_laplacian: U {tuple(U.shape)} and k {tuple(k.shape)} do not fit n = {n}, Q = {Q}")
+    Y = torch.empty_like(U)
+    _lib.call("jfx_weak_par", _p(fr[0][0]), fr[0][2], _p(fr[1][0]), fr[1][2], _p(fr[2][0]), fr[2][2], _p(fr[3][0]),
+              fr[3][2], n, Q, _p(U), _p(k), _p(Y), nb, _s())
+    return Y
+
+
 PLANE_PRECISIONS = ("f64", "bf16x6", "i8x5", "i8x6")
 
 
@@ -729,8 +752,9 @@ def plane_fd_ok(ops, prec: str) -> bool:
 
 
 def plane_fd(W0: AxisOperator, W1: AxisOperator, V0: AxisOperator, V1: AxisOperator, X: torch.Tensor,
-             E: torch.Tensor, prec: str = "f64") -> torch.Tensor:
-    """``Y[b] = V0 ((W0 X[b] W1^T) / E) V1^T`` over the last two axes in one kernel."""
+             E: torch.Tensor, prec: str = "f64", scale: torch.Tensor | None = None) -> torch.Tensor:
+    """``Y[b] = V0 ((W0 X[b] W1^T) / E) V1^T`` over the last two axes in one kernel,
+    times ``scale[b]`` if given (FP64 operators that couple equal parities)."""
     dt = io_dtype(prec)
     _req(X, dt, "X")
     _req(E, dt, "E")
@@ -741,9 +765,16 @@ def plane_fd(W0: AxisOperator, W1: AxisOperator, V0: AxisOperator, V1: AxisOpera
             if tuple(X.shape[-2:]) != shape or tuple(E.shape) != shape:
                 raise ValueError("plane_fd: operators, array or divisor do not fit the fused solve")
             Y = torch.empty_like(X)
+            B = math.prod(X.shape[:-2])
+            if scale is not None:
+                _req(scale, torch.float64, "scale")
+                if scale.numel() != B:
+                    raise ValueError(f"plane_fd: {scale.numel()} scales for {B} slabs")
             _lib.call("jfx_plane_fd_par", _p(fr[0][0]), _p(fr[1][0]), _p(fr[2][0]), _p(fr[3][0]), _p(X), _p(Y), _p(E),
-                      math.prod(X.shape[:-2]), W0.M, W1.M, _s())
+                      _p(scale), B, W0.M, W1.M, _s())
             return Y
+    if scale is not None:
+        raise ValueError("plane_fd: scale needs FP64 operators that couple equal parities")
     n = W0.M
     if not plane_fd_ok([W0, W1, V0, V1], prec) or tuple(X.shape[-2:]) != (n, n) or tuple(E.shape) != (n, n):
         raise ValueError("plane_fd: operators, array or divisor do not fit the fused solve")
@@ -763,8 +794,8 @@ def plane(op0: AxisOperator, op1: AxisOperator, X: torch.Tensor, prec: str = "f6
           epi: tuple | None = None, alpha: float = 1.0, out: torch.Tensor | None = None,
           accumulate: bool = False) -> torch.Tensor:
     """``Y[b] = alpha A0 X[b] A1^T`` over the last two axes of X in one kernel
-    (optionally ``/ E`` or ``* E`` with ``epi=("div"|"mul", E)``); with
-    ``accumulate`` the result is added to ``out``."""
+    (optionally ``/ E`` or ``* E`` with ``epi=("div"|"mul", E)``, or ``* E[b]`` with
+    ``epi=("mul_each", E)``); with ``accumulate`` the result is added to ``out``."""
     dt = io_dtype(prec)
     _req(X, dt, "X")
     if X.shape[-2] != op0.K or X.shape[-1] != op1.K:
@@ -784,11 +815,13 @@ def plane(op0: AxisOperator, op1: AxisOperator, X: torch.Tensor, prec: str = "f6
         Y = out
     mode, E = 0, None
     if epi is not None:
-        mode = {"div": 1, "mul": 2}[epi[0]]
+        mode = {"div": 1, "mul": 2, "mul_each": 3}[epi[0]]
         E = epi[1]
         _req(E, dt, "E")
-        if tuple(E.shape) != (op0.M, op1.M):
+        if tuple(E.shape) != (tuple(shape) if mode == 3 else (op0.M, op1.M)):
             raise ValueError("plane: epilogue shape mismatch")
+        if mode == 3 and (prec != "f64" or slab_pays(op0, op1, B) is None):
+            raise ValueError("plane: a factor per slab needs FP64 operators with decoupled parities")
     acc = 1 if accumulate else 0
     if prec.startswith("i8x"):
         if mode or accumulate or alpha != 1.0:

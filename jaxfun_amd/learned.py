@@ -148,18 +148,31 @@ class VarCoeffPoisson2D:
     def _ap(self, op, X, axis):
         return K.apply_along(op, X.contiguous(), axis, "f64")
 
+    def _ap2(self, op, X, factor: torch.Tensor | None = None):
+        """op along both axes of (batch, K, K), times ``factor`` (batch, M, M): one
+        launch where the slab kernel pays off."""
+        X = X.contiguous()
+        if K.slab_pays(op, op, X.shape[0]):
+            return K.plane(op, op, X, "f64", epi=None if factor is None else ("mul_each", factor))
+        Y = self._ap(op, self._ap(op, X, 1), 2)
+        return Y if factor is None else mul_bcast(Y, factor)
+
     def kfield(self, ghat: torch.Tensor) -> torch.Tensor:
         """k = exp(g) at the (Q, Q) quadrature mesh for ghat (batch, gm, gm)."""
-        g = self._ap(self.Vg, self._ap(self.Vg, ghat, 1), 2)
+        g = self._ap2(self.Vg, ghat)
         k = torch.empty_like(g)
         _lib.call("jfx_exp", K._p(g), K._p(k), 1.0, g.numel(), K._s())
         return k
 
     def rhs(self, fhat: torch.Tensor) -> torch.Tensor:
         """b = (S (x) S)(diag(h) fhat diag(h)) for orthogonal Legendre forcing coefficients."""
-        return self._ap(self.SH, self._ap(self.SH, fhat, 1), 2)
+        return self._ap2(self.SH, fhat)
 
     def apply(self, kq: torch.Tensor, U: torch.Tensor) -> torch.Tensor:
+        if U.ndim == 3 and tuple(kq.shape) == (U.shape[0], self.Q, self.Q):
+            Y = K.weak_laplacian(self.B, self.Dx, self.TB, self.TD, kq, U.contiguous())
+            if Y is not None:
+                return Y
         ux = self._ap(self.Dx, self._ap(self.B, U, 2), 1)
         uy = self._ap(self.B, self._ap(self.Dx, U, 2), 1)
         a = self._ap(self.TB, self._ap(self.TD, mul_bcast(ux, kq), 1), 2)
@@ -177,6 +190,9 @@ class VarCoeffPoisson2D:
         inv = (1.0 / kbar).contiguous()
 
         def P(R):
+            if R.ndim == 3 and R.shape[0] == inv.numel() and R.dtype == torch.float64 and \
+                    K.plane_fd_par_ok([*self.L.W, *self.L.V]):
+                return K.plane_fd(*self.L.W, *self.L.V, R.contiguous(), self.L.D(torch.float64), scale=inv)
             Z = self.L.solve(R)
             out = torch.empty_like(Z)
             _lib.call("jfx_scale_batch", K._p(Z), K._p(inv), K._p(out), Z.shape[0], Z[0].numel(), K._s())
@@ -185,30 +201,30 @@ class VarCoeffPoisson2D:
 
     def scaled_parts(self, s: torch.Tensor, R: torch.Tensor):
         """Forward pass of P_s R, returning intermediates for the backward pass."""
-        FtR = self._ap(self.FT, self._ap(self.FT, R, 1), 2)     # (b, Q, Q)
+        FtR = self._ap2(self.FT, R)                             # (b, Q, Q)
         a = mul_bcast(FtR, s)
-        c = self._ap(self.BT, self._ap(self.BT, a, 1), 2)       # (b, n, n)
+        c = self._ap2(self.BT, a)                               # (b, n, n)
         d = self.L.solve(c)
-        e = self._ap(self.B, self._ap(self.B, d, 1), 2)         # (b, Q, Q)
+        e = self._ap2(self.B, d)                                # (b, Q, Q)
         y = mul_bcast(e, s)
-        z = self._ap(self.F, self._ap(self.F, y, 1), 2)
+        z = self._ap2(self.F, y)
         return z, (FtR, e)
 
     def scaled_precond(self, s: torch.Tensor):
         def P(R):
-            return self.scaled_parts(s, R)[0]
+            if tuple(s.shape) != (R.shape[0], self.Q, self.Q):  # one field for several systems
+                return self.scaled_parts(s, R)[0]
+            a = self._ap2(self.FT, R, s)
+            return self._ap2(self.F, self._ap2(self.B, self.L.solve(self._ap2(self.BT, a)), s))
         return P
 
     def scaled_backward(self, s, parts, gz):
         """d loss / d s given d loss / d z (P_s's two s-products; L symmetric)."""
         FtR, e = parts
-        gy = self._ap(self.FT, self._ap(self.FT, gz, 1), 2)
-        gs = mul_bcast(gy, e)
+        gy = self._ap2(self.FT, gz)
         ge = mul_bcast(gy, s)
-        gd = self._ap(self.BT, self._ap(self.BT, ge, 1), 2)
-        gc = self.L.solve(gd)
-        ga = self._ap(self.B, self._ap(self.B, gc, 1), 2)
-        return K.lincomb([(1.0, gs), (1.0, mul_bcast(ga, FtR))])
+        ga = self._ap2(self.B, self.L.solve(self._ap2(self.BT, ge)))
+        return K.sum_products([(1.0, gy, e), (1.0, ga, FtR)])
 
     def sigma_field(self, sig_hat: torch.Tensor) -> torch.Tensor:
         """s = exp(sigma) on the mesh from (batch, gm, gm) low-mode coefficients."""
@@ -220,6 +236,9 @@ def batched_dot(x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     out = torch.empty(x.shape[0], dtype=torch.float64, device=x.device)
     _lib.call("jfx_batched_dot", K._p(x), K._p(y), K._p(out), x.shape[0], x[0].numel(), K._s())
     return out
+
+
+_LEFT_SLOTS = 1024  # counters of active systems, reused in turn
 
 
 def pcg(apply, b: torch.Tensor, precond, x0: torch.Tensor | None = None, rtol: float = 1e-10,
@@ -246,21 +265,30 @@ def pcg(apply, b: torch.Tensor, precond, x0: torch.Tensor | None = None, rtol: f
     z = precond(r)
     p = K.lincomb([(1.0, z)])
     rz = batched_dot(r, z)
+    # left[i]: systems still active after iteration i.  The host reads it while the
+    # next iteration's operator and update are queued, so the device never waits for
+    # the host; systems that have stopped do not change, so a queued iteration too
+    # many changes nothing.
+    left = torch.zeros(_LEFT_SLOTS, dtype=torch.int32, device=b.device)
+    host = torch.empty(2, dtype=torch.int32, pin_memory=True)
+    ev = [torch.cuda.Event(), torch.cuda.Event()]
     for it in range(maxiter):
+        slot = it % _LEFT_SLOTS
+        if it and slot == 0:
+            left.zero_()
         q = apply(p)
-        pq = batched_dot(p, q)
-        _lib.call("jfx_pcg_update_xr", K._p(x), K._p(r), K._p(p), K._p(q), K._p(rz), K._p(pq), K._p(active), B,
-                  n, K._s())
-        rr = batched_dot(r, r)
-        _lib.call("jfx_pcg_check", K._p(rr), K._p(bb), rtol * rtol, K._p(active), K._p(iters), B, 1, K._s())
+        _lib.call("jfx_pcg_step", K._p(x), K._p(r), K._p(p), K._p(q), K._p(rz), K._p(bb), rtol * rtol, K._p(active),
+                  K._p(iters), left.data_ptr() + 4 * slot, B, n, K._s())
+        host[it % 2].copy_(left[slot], non_blocking=True)
+        ev[it % 2].record()
+        if it and it % check_every == 0:  # after iteration it - 1
+            ev[(it - 1) % 2].synchronize()
+            if int(host[(it - 1) % 2]) == 0:
+                break
         if snap_out is not None and it + 1 in snapshots:
             snap_out[it + 1] = (x.clone(), r.clone())
-        if (it + 1) % check_every == 0 and int(active.sum().item()) == 0:
-            break
         z = precond(r)
-        rz_new = batched_dot(r, z)
-        _lib.call("jfx_pcg_update_p", K._p(p), K._p(z), K._p(rz_new), K._p(rz), K._p(active), B, n, K._s())
-        rz = rz_new
+        _lib.call("jfx_pcg_direction", K._p(p), K._p(z), K._p(r), K._p(rz), K._p(active), B, n, K._s())
     if breakdown == "raise":
         nbad = int((iters < 0).sum().item())
         if nbad:
@@ -350,7 +378,7 @@ class LearnedPreconditioner:
         _lib.call("jfx_scale_batch", K._p(Md), K._p(w), K._p(gz), Bn, diff[0].numel(), K._s())
         gs = op.scaled_backward(s, parts, gz)
         gsig = mul_bcast(gs, s)
-        gsh = op._ap(op.VgT, op._ap(op.VgT, gsig, 1), 2)
+        gsh = op._ap2(op.VgT, gsig)
         grads = self.net.backward(hs, _f32(mul_bcast(gsh, self.D).reshape(Bn, -1)))
         return float(per.mean().item()), grads
 
