@@ -122,10 +122,12 @@ int jfx_weak_par(const double* FB, int sB, const double* FD, int sD, const doubl
 
 /* Fused PCG steps over `batch` systems of n values, FP64.  jfx_pcg_step: for active
  * systems a = rz / (p, q), x += a p, r -= a q, then the stopping test of jfx_pcg_check
- * with count = 1; *left is increased by the number of systems that stay active.
+ * with count = 1; *left (a zeroed int) counts the systems that stay active in its low
+ * 16 bits, and the count is stored to host_left (pinned host memory or null) when all are done.
  * jfx_pcg_direction: for active systems s = (r, z), p = z + (s / rz) p, rz = s. */
 int jfx_pcg_step(double* x, double* r, const double* p, const double* q, const double* rz, const double* bb,
-                 double tol2, int* active, int* iters, int* left, int batch, long long n, hipStream_t stream);
+                 double tol2, int* active, int* iters, int* left, int* host_left, int batch, long long n,
+                 hipStream_t stream);
 int jfx_pcg_direction(double* p, const double* z, const double* r, double* rz, const int* active, int batch,
                       long long n, hipStream_t stream);
 

@@ -45,7 +45,7 @@ SIGNATURES: dict[str, tuple] = {
     "jfx_plane_fd_par": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_ll, c_int, c_int, c_vp]),
     "jfx_weak_par": (c_int, [c_vp, c_int, c_vp, c_int, c_vp, c_int, c_vp, c_int, c_int, c_int, c_vp, c_vp, c_vp, c_ll,
                              c_vp]),
-    "jfx_pcg_step": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_dbl, c_vp, c_vp, c_vp, c_int, c_ll, c_vp]),
+    "jfx_pcg_step": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_dbl, c_vp, c_vp, c_vp, c_vp, c_int, c_ll, c_vp]),
     "jfx_pcg_direction": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_ll, c_vp]),
     "jfx_contract_bf16x": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),
     "jfx_contract_ozaki": (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),

@@ -239,24 +239,17 @@ __device__ __forceinline__ double block_sum(double s, double* red) {
 // vectors read once from HBM and the second time from L2.  256 systems of 3844
 // values: 7.3 + 6.3 + 7.3 + 2.0 us and a 3-kernel count before, 10 us now.
 constexpr int PCG_W = 8;
-__global__ __launch_bounds__(64 * PCG_W) void pcg_step_kernel(double* __restrict__ x, double* __restrict__ r,
-                                                              const double* __restrict__ p,
-                                                              const double* __restrict__ q,
-                                                              const double* __restrict__ rz,
-                                                              const double* __restrict__ bb, double tol2,
-                                                              int* __restrict__ active, int* __restrict__ iters,
-                                                              int* __restrict__ left, long long n) {
-  __shared__ double red[2][PCG_W];
-  const long long b = blockIdx.x;
-  if (!active[b]) return;  // uniform; thread 0 writes active[b] behind two barriers
-  x += b * n;
-  r += b * n;
-  p += b * n;
-  q += b * n;
+// One active system; returns (thread 0) whether it goes on.
+__device__ __forceinline__ int pcg_step_system(double* __restrict__ x, double* __restrict__ r,
+                                               const double* __restrict__ p, const double* __restrict__ q, double rz,
+                                               double stop, int* active, int* iters, double (*red)[PCG_W],
+                                               long long n) {
   double s = 0.0;
+#pragma unroll 4
   for (long long i = threadIdx.x; i < n; i += 64 * PCG_W) s += p[i] * q[i];
-  const double a = rz[b] / block_sum<PCG_W>(s, red[0]);
+  const double a = rz / block_sum<PCG_W>(s, red[0]);
   double t = 0.0;
+#pragma unroll 4
   for (long long i = threadIdx.x; i < n; i += 64 * PCG_W) {
     x[i] += a * p[i];
     const double v = r[i] - a * q[i];
@@ -264,17 +257,38 @@ __global__ __launch_bounds__(64 * PCG_W) void pcg_step_kernel(double* __restrict
     t += v * v;
   }
   const double rr = block_sum<PCG_W>(t, red[1]);
+  if (threadIdx.x != 0) return 0;
+  if (!isfinite(rr)) {  // breakdown: the system stops and is marked with iters = -1
+    *active = 0;
+    *iters = -1;
+    return 0;
+  }
+  *iters += 1;
+  if (rr > stop) return 1;
+  *active = 0;
+  return 0;
+}
+
+__global__ __launch_bounds__(64 * PCG_W) void pcg_step_kernel(double* __restrict__ x, double* __restrict__ r,
+                                                              const double* __restrict__ p,
+                                                              const double* __restrict__ q,
+                                                              const double* __restrict__ rz,
+                                                              const double* __restrict__ bb, double tol2,
+                                                              int* __restrict__ active, int* __restrict__ iters,
+                                                              unsigned* __restrict__ left,
+                                                              int* __restrict__ host_left, long long n) {
+  __shared__ double red[2][PCG_W];
+  const long long b = blockIdx.x;
+  int on = active[b];  // uniform; thread 0 writes active[b] behind two barriers
+  if (on) on = pcg_step_system(x + b * n, r + b * n, p + b * n, q + b * n, rz[b], tol2 * bb[b], active + b, iters + b,
+                               red, n);
+  // *left: workgroups that are done (high half) and systems that go on (low
+  // half) in one atomic, so that the last workgroup knows the count without a
+  // fence (13 us with one, 9 us without)
   if (threadIdx.x == 0) {
-    if (!isfinite(rr)) {  // breakdown: the system stops and is marked with iters = -1
-      active[b] = 0;
-      iters[b] = -1;
-    } else {
-      iters[b] += 1;
-      if (rr > tol2 * bb[b])
-        atomicAdd(left, 1);
-      else
-        active[b] = 0;
-    }
+    const unsigned old = atomicAdd(left, 0x10000u | (unsigned)on);
+    if (host_left && (old >> 16) == gridDim.x - 1)
+      __hip_atomic_store(host_left, (int)((old & 0xffffu) + on), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -290,9 +304,11 @@ __global__ __launch_bounds__(64 * PCG_W) void pcg_direction_kernel(double* __res
   z += b * n;
   r += b * n;
   double s = 0.0;
+#pragma unroll 4
   for (long long i = threadIdx.x; i < n; i += 64 * PCG_W) s += r[i] * z[i];
   s = block_sum<PCG_W>(s, red);
   const double beta = s / rz[b];
+#pragma unroll 4
   for (long long i = threadIdx.x; i < n; i += 64 * PCG_W) p[i] = z[i] + beta * p[i];
   __syncthreads();  // every thread has read rz[b]
   if (threadIdx.x == 0) rz[b] = s;
@@ -420,12 +436,12 @@ int jfx_pcg_check(const double* rr, const double* bb, double tol2, int* active, 
 }
 
 int jfx_pcg_step(double* x, double* r, const double* p, const double* q, const double* rz, const double* bb,
-                 double tol2, int* active, int* iters, int* left, int batch, long long n, hipStream_t stream) {
+                 double tol2, int* active, int* iters, int* left, int* host_left, int batch, long long n, hipStream_t stream) {
   if (!x || !r || !p || !q || !rz || !bb || !active || !iters || !left || batch < 0 || batch > 65535 || n < 0)
     return set_error("pcg_step: bad arguments"), JFX_EARG;
   if (batch == 0) return JFX_OK;
   hipLaunchKernelGGL(pcg_step_kernel, dim3(batch), dim3(64 * PCG_W), 0, stream, x, r, p, q, rz, bb, tol2, active, iters,
-                     left, n);
+                     (unsigned*)left, host_left, n);
   JFX_LAUNCH_CHECK();
   return JFX_OK;
 }

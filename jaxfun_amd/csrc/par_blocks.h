@@ -3,10 +3,13 @@
 //
 // One workgroup of NW waves holds a slab in LDS and applies one operator along
 // each axis:  T = X A1^T (rows x M1),  Y = A0 T (M0 x M1).
-//   phase A  a wave owns 16 rows of X and two half column blocks of T, even and
-//            odd part (4 accumulators): all of T sits in the workgroup's
-//            registers, so T overwrites X in LDS
-//   phase B  a wave owns a half row block of Y and two column blocks
+//   phase A  a wave owns 16 rows of X and JW half column blocks of T, even and odd
+//            part: all of T sits in the workgroup's registers, so T overwrites X
+//   phase B  a wave owns a half row block of Y and JW column blocks
+// Up to 64 x 64 (JW = 1) a wave loads all its fragments of a phase before the
+// barrier in front of it: with one slab per CU a phase is as long as its loads
+// take, and an L2 round trip per k-step was most of it.  Larger slabs (JW = 2, 16
+// waves) have no registers for that and load two k-steps ahead.
 // Rows of X are 16-byte pairs (even k, odd k) for EVAL and MIX; LDX = 2 (mod 16)
 // puts 16 rows on distinct banks.  T is read in rows 2 apart, 16 columns wide;
 // LDT = 8 (mod 16) does the same there.  Rows past the slab and columns past K1
@@ -40,10 +43,20 @@ __host__ __device__ inline int slab_lds(int K0, int K1, int M1) {
 
 typedef double d2 __attribute__((ext_vector_type(2)));
 
+// Thread and lane index as opaque values: addresses computed from them are not
+// shared between phases, which would hold hundreds of them in registers.
+__device__ __forceinline__ int own_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+__device__ __forceinline__ int own_lane() { return own_tid() & 63; }
+
 // Zeros around a (K0 x K1) slab in LDS, rows and columns up to multiples of 16.
 template <int NT>
 __device__ __forceinline__ void slab_zero_pad(int K0, int K1, double* Xs) {
-  const int LDX = slab_ldx(K1), R = slab_pad(K0), C = slab_pad(K1), tid = threadIdx.x;
+  const int LDX = slab_ldx(K1), R = slab_pad(K0), C = slab_pad(K1);
+  const int tid = own_tid();
   const int nz = C - K1;
   if (nz)
     for (int e = tid; e < K0 * nz; e += NT) {
@@ -59,7 +72,8 @@ __device__ __forceinline__ void slab_zero_pad(int K0, int K1, double* Xs) {
 // X (K0 x K1, contiguous) into LDS, rows LDX apart, zero padded to 16s.
 template <int NT>
 __device__ __forceinline__ void slab_stage(const double* __restrict__ X, int K0, int K1, double* Xs) {
-  const int LDX = slab_ldx(K1), tid = threadIdx.x;
+  const int LDX = slab_ldx(K1);
+  const int tid = own_tid();
   constexpr int U = 8;
   if (K1 % 2 == 0 && ((uintptr_t)X & 15) == 0) {
     const unsigned kh = K1 / 2;
@@ -125,91 +139,131 @@ __device__ __forceinline__ void col_operands(const double* T, int LDT, int c, in
   }
 }
 
-typedef v4d Acc4[2][2];  // [part][block]
-
-__device__ __forceinline__ void acc_zero(Acc4& a) {
+template <int JW>
+struct Acc {
+  v4d v[2][JW];  // [part][block]
+  __device__ __forceinline__ void zero() {
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) a[h][j] = v4d{0, 0, 0, 0};
-}
-
-// Waves of phase A: (row block, pair of half column blocks); -1: idle.
-struct WaveA {
-  int rb, cb[2];
-  bool on, on1;
+      for (int j = 0; j < JW; ++j) v[h][j] = v4d{0, 0, 0, 0};
+  }
 };
-__device__ __forceinline__ WaveA wave_a(int w, int K0, const ParOp& o) {
-  const int ncg = (o.nrb + 1) >> 1, nrow = slab_pad(K0) >> 4;
-  WaveA a;
-  a.rb = w / ncg;
-  const int cg = w - a.rb * ncg;
-  a.on = a.rb < nrow;
-  a.cb[0] = 2 * cg;
-  a.on1 = 2 * cg + 1 < o.nrb;
-  a.cb[1] = a.on1 ? 2 * cg + 1 : 2 * cg;  // a copy whose results are not stored
-  return a;
-}
 
-template <int MODE>
-__device__ __forceinline__ void phase_a(const double* Xs, int LDX, const ParOp& o, const WaveA& wa, Acc4& acc) {
-  const int lane = threadIdx.x & 63, kk = lane >> 4, cl = lane & 15;
+// Fragments of NB blocks of one operator, both parts: every k-step up to SMAX
+// (slabs up to 64: 8), or with SMAX = 2 the step pair in use.
+template <int NB, int SMAX>
+struct Frag {
+  const double* p[2][NB];
+  int lo, hi, S;
+  double v[SMAX][2][NB];
+
+  // unconditional (steps past the last are clamped), so that no earlier value of
+  // v stays live through a branch
+  __device__ __forceinline__ void load(int s0) {
+#pragma unroll
+    for (int u = 0; u < SMAX; ++u) {
+      const int s = SMAX == 2 || s0 + u < S ? s0 + u : S - 1;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) v[u][h][j] = p[h][j][s * 64];
+    }
+  }
+  // blocks rb[] of o; the first loads are issued here, ahead of the barrier
+  __device__ __forceinline__ void init(const ParOp& o, const int (&rb)[NB]) {
+    const int lane = own_lane();
+    lo = o.lo[rb[0]];
+    hi = o.hi[rb[0]];
+    S = o.S;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      lo = o.lo[rb[j]] < lo ? o.lo[rb[j]] : lo;
+      hi = o.hi[rb[j]] > hi ? o.hi[rb[j]] : hi;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) p[h][j] = o.f + ((h * o.nrb + rb[j]) * o.S) * 64 + lane;
+    }
+    load(SMAX == 2 ? lo : 0);  // lo < S, also of an empty range
+  }
+  // f(k-step, fragments of that step) over the steps that are not zero
+  template <typename F>
+  __device__ __forceinline__ void each(F&& f) {
+    if constexpr (SMAX == 2) {
+      for (int s = lo; s < hi; s += 2) {
+        Frag n = *this;
+        n.load(s + 2 < hi ? s + 2 : s);
+        f(s, v[0]);
+        f(s + 1, v[1]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) v[u][h][j] = n.v[u][h][j];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < SMAX; ++s)
+        if (s >= lo && s < hi) f(s, v[s]);
+    }
+  }
+};
+template <int JW>
+constexpr int frag_steps() { return JW == 1 ? 8 : 2; }
+
+// A wave's share of phase A: a row block and JW half column blocks.
+template <int JW>
+struct WaveA {
+  int rb, cb[JW];
+  bool on, ok[JW];
+  Frag<JW, frag_steps<JW>()> f;
+
+  __device__ __forceinline__ void init(int w, int K0, const ParOp& o) {
+    const int ncg = (o.nrb + JW - 1) / JW, nrow = slab_pad(K0) >> 4;
+    rb = w / ncg;
+    const int cg = w - rb * ncg;
+    on = rb < nrow;
+#pragma unroll
+    for (int j = 0; j < JW; ++j) {
+      ok[j] = JW * cg + j < o.nrb;
+      cb[j] = ok[j] ? JW * cg + j : JW * cg;  // a copy whose results are not stored
+    }
+  }
+  __device__ __forceinline__ void prefetch(const ParOp& o) { f.init(o, cb); }
+};
+
+template <int MODE, int JW>
+__device__ __forceinline__ void phase_a(const double* Xs, int LDX, const ParOp& o, WaveA<JW>& wa, Acc<JW>& acc) {
+  const int lane = own_lane(), kk = lane >> 4, cl = lane & 15;
   const double* row = Xs + (16 * wa.rb + cl) * LDX;
   const double sg = o.sgn;
-  int lo = o.lo[wa.cb[0]], hi = o.hi[wa.cb[0]];
-  lo = o.lo[wa.cb[1]] < lo ? o.lo[wa.cb[1]] : lo;
-  hi = o.hi[wa.cb[1]] > hi ? o.hi[wa.cb[1]] : hi;
-  const double* p[2][2];
+  const int K = o.K;
+  wa.f.each([&](int s, const double(&a)[2][JW]) {
+    double e, d;
+    row_operands<MODE>(row, s, kk, K, sg, e, d);
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) p[h][j] = o.f + ((h * o.nrb + wa.cb[j]) * o.S) * 64 + lane;
-  double a[2][2][2], n[2][2][2];  // [step][part][block]
-  auto ld = [&](int s, double(&d)[2][2][2]) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) d[u][h][j] = p[h][j][(s + u) * 64];
-  };
-  if (lo < hi) ld(lo, a);
-  for (int s = lo; s < hi; s += 2) {
-    if (s + 2 < hi) ld(s + 2, n);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      double e, d;
-      row_operands<MODE>(row, s + u, kk, o.K, sg, e, d);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[0][j] = mfma_f64(e, a[u][0][j], acc[0][j]);
-        acc[1][j] = mfma_f64(d, a[u][1][j], acc[1][j]);
-      }
+    for (int j = 0; j < JW; ++j) {
+      acc.v[0][j] = mfma_f64(e, a[0][j], acc.v[0][j]);
+      acc.v[1][j] = mfma_f64(d, a[1][j], acc.v[1][j]);
     }
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) a[u][h][j] = n[u][h][j];
-  }
+  });
 }
 
 // T (rows 16 rb.., M1 columns) into LDS, rows LDT apart
-template <int MODE>
-__device__ __forceinline__ void store_t(double* T, int LDT, const ParOp& o, const WaveA& wa, const Acc4& acc) {
-  const int lane = threadIdx.x & 63, cl = lane & 15;
+template <int MODE, int JW>
+__device__ __forceinline__ void store_t(double* T, int LDT, const ParOp& o, const WaveA<JW>& wa, const Acc<JW>& acc) {
+  const int lane = own_lane(), cl = lane & 15;
   const double sg = o.sgn;
   const int M = o.M, Mh = (M + 1) >> 1;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    if (j == 1 && !wa.on1) break;
+  for (int j = 0; j < JW; ++j) {
+    if (!wa.ok[j]) break;
     const int m = 16 * wa.cb[j] + cl;
     if (m >= Mh) continue;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       double* d = T + (16 * wa.rb + mfma16_row_f64(lane, r)) * LDT;
-      const double e = acc[0][j][r], q = acc[1][j][r];
+      const double e = acc.v[0][j][r], q = acc.v[1][j][r];
       if constexpr (MODE == MODE_EVAL) {
         d[m] = e + q;
         d[M - 1 - m] = M - 1 - m == m ? e + q : sg * (e - q);
@@ -221,76 +275,73 @@ __device__ __forceinline__ void store_t(double* T, int LDT, const ParOp& o, cons
   }
 }
 
-// Items of phase B: (half row block of A0, pair of column blocks of T)
-__device__ __forceinline__ int items_b(const ParOp& o, int M1) {
-  return o.nrb * (((slab_pad(M1) >> 4) + 1) >> 1);
+// A wave's share of phase B: a half row block of A0 and JW column blocks of T.
+template <int JW>
+__host__ __device__ __forceinline__ int items_b(const ParOp& o, int M1) {
+  return o.nrb * (((slab_pad(M1) >> 4) + JW - 1) / JW);
 }
+template <int JW>
 struct ItemB {
-  int rb, c[2];
-  bool on1;
-};
-__device__ __forceinline__ ItemB item_b(int it, const ParOp& o, int M1) {
-  const int ncb = slab_pad(M1) >> 4, ncg = (ncb + 1) >> 1;
-  ItemB b;
-  b.rb = it / ncg;
-  const int cg = it - b.rb * ncg;
-  b.c[0] = 32 * cg;
-  b.on1 = 2 * cg + 1 < ncb;
-  b.c[1] = b.on1 ? 32 * cg + 16 : 32 * cg;
-  return b;
-}
+  int rb, c[JW];
+  bool on, ok[JW];
+  Frag<1, frag_steps<JW>()> f;
 
-template <int MODE>
-__device__ __forceinline__ void phase_b(const double* T, int LDT, const ParOp& o, const ItemB& b, Acc4& acc) {
-  const int lane = threadIdx.x & 63, kk = lane >> 4, cl = lane & 15;
-  const double sg = o.sgn;
-  const int lo = o.lo[b.rb], hi = o.hi[b.rb];
-  const double* p0 = o.f + (b.rb * o.S) * 64 + lane;
-  const double* p1 = p0 + o.nrb * o.S * 64;
-  double a[2][2], n[2][2];  // [step][part]
-  auto ld = [&](int s, double(&d)[2][2]) {
+  __device__ __forceinline__ void init(int it, const ParOp& o, int M1) {
+    const int ncb = slab_pad(M1) >> 4, ncg = (ncb + JW - 1) / JW;
+    rb = it / ncg;
+    const int cg = it - rb * ncg;
+    on = rb < o.nrb;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      d[u][0] = p0[(s + u) * 64];
-      d[u][1] = p1[(s + u) * 64];
-    }
-  };
-  if (lo < hi) ld(lo, a);
-  for (int s = lo; s < hi; s += 2) {
-    if (s + 2 < hi) ld(s + 2, n);
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        double e, d;
-        col_operands<MODE>(T, LDT, b.c[j] + cl, s + u, kk, o.K, sg, e, d);
-        acc[0][j] = mfma_f64(a[u][0], e, acc[0][j]);
-        acc[1][j] = mfma_f64(a[u][1], d, acc[1][j]);
-      }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      a[u][0] = n[u][0];
-      a[u][1] = n[u][1];
+    for (int j = 0; j < JW; ++j) {
+      ok[j] = JW * cg + j < ncb;
+      c[j] = 16 * (ok[j] ? JW * cg + j : JW * cg);
     }
   }
+  __device__ __forceinline__ void prefetch(const ParOp& o) {
+    const int r[1] = {on ? rb : 0};
+    f.init(o, r);
+  }
+};
+
+template <int MODE, int JW>
+__device__ __forceinline__ void phase_b(const double* T, int LDT, const ParOp& o, ItemB<JW>& b, Acc<JW>& acc) {
+  const int lane = own_lane(), kk = lane >> 4, cl = lane & 15;
+  const double sg = o.sgn;
+  const int K = o.K;
+  b.f.each([&](int s, const double(&a)[2][1]) {
+#pragma unroll
+    for (int j = 0; j < JW; ++j) {
+      double e, d;
+      col_operands<MODE>(T, LDT, b.c[j] + cl, s, kk, K, sg, e, d);
+      acc.v[0][j] = mfma_f64(a[0][0], e, acc.v[0][j]);
+      acc.v[1][j] = mfma_f64(a[1][0], d, acc.v[1][j]);
+    }
+  });
+}
+
+// waves that cover phase A of (K0 rows) x o1 and phase B of o0
+template <int JW>
+inline int slab_items(int K0, const ParOp& o0, const ParOp& o1) {
+  const int a = (slab_pad(K0) / 16) * ((o1.nrb + JW - 1) / JW), b = items_b<JW>(o0, o1.M);
+  return a > b ? a : b;
 }
 
 // f(m, c, value) for every element of the item inside (M x M1)
-template <int MODE, typename F>
-__device__ __forceinline__ void each_b(const ParOp& o, const ItemB& b, int M1, const Acc4& acc, F&& f) {
-  const int lane = threadIdx.x & 63, cl = lane & 15;
+template <int MODE, int JW, typename F>
+__device__ __forceinline__ void each_b(const ParOp& o, const ItemB<JW>& b, int M1, const Acc<JW>& acc, F&& f) {
+  const int lane = own_lane(), cl = lane & 15;
   const double sg = o.sgn;
   const int M = o.M, Mh = (M + 1) >> 1;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    if (j == 1 && !b.on1) break;
+  for (int j = 0; j < JW; ++j) {
+    if (!b.ok[j]) break;
     const int c = b.c[j] + cl;
     if (c >= M1) continue;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = 16 * b.rb + mfma16_row_f64(lane, r);
       if (m >= Mh) continue;
-      const double e = acc[0][j][r], q = acc[1][j][r];
+      const double e = acc.v[0][j][r], q = acc.v[1][j][r];
       if constexpr (MODE == MODE_EVAL) {
         f(m, c, e + q);
         if (M - 1 - m != m) f(M - 1 - m, c, sg * (e - q));

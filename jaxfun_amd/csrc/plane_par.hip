@@ -4,8 +4,8 @@
 // and the fast-diagonalisation solve  Y[b] = scale[b] V0 ((W0 X[b] W1^T) / E) V1^T.
 //
 // A slab is read once and written once; the intermediate stays in LDS
-// (par_blocks.h).  One workgroup per slab: 4 waves up to 64 x 64 (37 KB of LDS,
-// four workgroups per CU), 16 waves for larger slabs (139 KB at 128 x 128).
+// (par_blocks.h).  One workgroup per slab: up to 8 waves for 64 x 64 (37 KB of
+// LDS), 16 for larger slabs (139 KB at 128 x 128, one workgroup per CU).
 #include "par_blocks.h"
 
 namespace jfx {
@@ -18,7 +18,7 @@ struct SlabMap {
   double alpha;
 };
 
-template <int MODE, int NW>
+template <int MODE, int NW, int JW>
 __global__ __launch_bounds__(64 * NW) void plane_par_kernel(const double* __restrict__ X, double* __restrict__ Y,
                                                             SlabMap sm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -26,34 +26,36 @@ __global__ __launch_bounds__(64 * NW) void plane_par_kernel(const double* __rest
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int K0 = sm.o0.K, K1 = sm.o1.K, M0 = sm.o0.M, M1 = sm.o1.M;
   const long long b = blockIdx.x;
+  WaveA<JW> wa;
+  ItemB<JW> ib;
+  Acc<JW> acc;
+  wa.init(w, K0, sm.o1);
+  ib.init(w, sm.o0, M1);
+  wa.prefetch(sm.o1);
   slab_stage<64 * NW>(X + b * K0 * K1, K0, K1, S);
   __syncthreads();
-  Acc4 acc;
-  acc_zero(acc);
-  const WaveA wa = wave_a(w, K0, sm.o1);
+  acc.zero();
   if (wa.on) phase_a<MODE>(S, slab_ldx(K1), sm.o1, wa, acc);
+  ib.prefetch(sm.o0);
   __syncthreads();
   const int LDT = slab_ldt(M1);
   if (wa.on) store_t<MODE>(S, LDT, sm.o1, wa, acc);
   __syncthreads();
+  if (!ib.on) return;
+  acc.zero();
+  phase_b<MODE>(S, LDT, sm.o0, ib, acc);
   double* Yb = Y + b * M0 * M1;
   const double* E = sm.epi == 3 ? sm.E + b * M0 * M1 : sm.E;
-  const int nit = items_b(sm.o0, M1);
-  for (int it = w; it < nit; it += NW) {
-    const ItemB ib = item_b(it, sm.o0, M1);
-    acc_zero(acc);
-    phase_b<MODE>(S, LDT, sm.o0, ib, acc);
-    each_b<MODE>(sm.o0, ib, M1, acc, [&](int m, int c, double v) {
-      const int i = m * M1 + c;
-      v *= sm.alpha;
-      if (sm.epi == 1)
-        v /= E[i];
-      else if (sm.epi)
-        v *= E[i];
-      if (sm.accum) v += Yb[i];
-      Yb[i] = v;
-    });
-  }
+  each_b<MODE>(sm.o0, ib, M1, acc, [&](int m, int c, double v) {
+    const int i = m * M1 + c;
+    v *= sm.alpha;
+    if (sm.epi == 1)
+      v /= E[i];
+    else if (sm.epi)
+      v *= E[i];
+    if (sm.accum) v += Yb[i];
+    Yb[i] = v;
+  });
 }
 
 struct FdMap {
@@ -61,7 +63,7 @@ struct FdMap {
   const double *E, *scale;  // scale: one factor per slab, or null
 };
 
-template <int NW>
+template <int NW, int JW>
 __global__ __launch_bounds__(64 * NW) void plane_fd_par_kernel(const double* __restrict__ X, double* __restrict__ Y,
                                                                FdMap fm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -70,47 +72,54 @@ __global__ __launch_bounds__(64 * NW) void plane_fd_par_kernel(const double* __r
   const int n0 = fm.w0.K, n1 = fm.w1.K;
   const long long b = blockIdx.x;
   const int LDX = slab_ldx(n1), LDT = slab_ldt(n1);
+  WaveA<JW> wa;
+  ItemB<JW> ib;
+  Acc<JW> acc;
+  wa.init(w, n0, fm.w1);
+  ib.init(w, fm.w0, n1);
+  wa.prefetch(fm.w1);
   slab_stage<64 * NW>(X + b * n0 * n1, n0, n1, S);
   __syncthreads();
-  Acc4 acc;
-  const WaveA wa = wave_a(w, n0, fm.w1);
-  const bool onb = w < items_b(fm.w0, n1);  // NW covers every item
-  const ItemB ib = item_b(w, fm.w0, n1);
-  acc_zero(acc);
+  acc.zero();
   if (wa.on) phase_a<MODE_MIX>(S, LDX, fm.w1, wa, acc);
+  ib.prefetch(fm.w0);
   __syncthreads();
   if (wa.on) store_t<MODE_MIX>(S, LDT, fm.w1, wa, acc);
   __syncthreads();
-  acc_zero(acc);
-  if (onb) phase_b<MODE_MIX>(S, LDT, fm.w0, ib, acc);
+  acc.zero();
+  if (ib.on) phase_b<MODE_MIX>(S, LDT, fm.w0, ib, acc);
+  wa.prefetch(fm.v1);
   __syncthreads();
   // G / E back into LDS as the second pass's input, zero padded like a staged slab
-  if (onb)
+  if (ib.on)
     each_b<MODE_MIX>(fm.w0, ib, n1, acc, [&](int m, int c, double v) { S[m * LDX + c] = v / fm.E[m * n1 + c]; });
   slab_zero_pad<64 * NW>(n0, n1, S);
   __syncthreads();
-  acc_zero(acc);
+  acc.zero();
   if (wa.on) phase_a<MODE_MIX>(S, LDX, fm.v1, wa, acc);
+  ib.prefetch(fm.v0);
   __syncthreads();
   if (wa.on) store_t<MODE_MIX>(S, LDT, fm.v1, wa, acc);
   __syncthreads();
-  acc_zero(acc);
-  if (onb) {
-    phase_b<MODE_MIX>(S, LDT, fm.v0, ib, acc);
-    double* Yb = Y + b * n0 * n1;
-    const double f = fm.scale ? fm.scale[b] : 1.0;
-    each_b<MODE_MIX>(fm.v0, ib, n1, acc, [&](int m, int c, double v) { Yb[m * n1 + c] = v * f; });
-  }
+  if (!ib.on) return;
+  acc.zero();
+  phase_b<MODE_MIX>(S, LDT, fm.v0, ib, acc);
+  double* Yb = Y + b * n0 * n1;
+  const double f = fm.scale ? fm.scale[b] : 1.0;
+  each_b<MODE_MIX>(fm.v0, ib, n1, acc, [&](int m, int c, double v) { Yb[m * n1 + c] = v * f; });
 }
 
 bool par_op(const double* frag, int M, int K, int mode, int sgn, int bp, int bq, ParOp& o);
 
-// waves that phase A of (K0 rows) x (operator o1) needs, 4 or 16
-int slab_waves(int K0, const ParOp& o0, const ParOp& o1) {
-  const int a = (slab_pad(K0) / 16) * ((o1.nrb + 1) / 2), b = o0.nrb * ((slab_pad(o1.M) / 16 + 1) / 2);
-  const int n = a > b ? a : b;
-  return n <= 4 ? 4 : n <= 8 ? 8 : 16;
-}
+// More than three slabs per CU of more than 32 rows: four waves with two blocks
+// each (six workgroups a CU overlap each other, and a wave's operator fragments
+// serve two blocks).  Fewer slabs, and slabs up to 32 x 32 whose workgroup is four
+// waves anyway: one block a wave, fragments loaded ahead.  us, two blocks / one:
+// 62 x 62 -> 64 x 64: 256 slabs 11.5 / 9.5, 768 20.7 / 20.8, 4096 75.7 / 81.7;
+// 48 x 48 solves: 256 15.6 / 11.1, 768 25.2 / 25.2, 4096 102 / 112;
+// 30 x 30 solves: 256 12.0 / 8.4, 4096 59.7 / 33.5.
+static bool slab_many(long long B, int items) { return items > 4 && B > 3 * 256; }
+static bool slab_small(const ParOp& o) { return o.M <= 64 && o.K <= 64; }
 
 template <typename K>
 static int slab_shm(K kern, size_t shm) {
@@ -119,31 +128,36 @@ static int slab_shm(K kern, size_t shm) {
   return JFX_OK;
 }
 
-template <int MODE, int NW>
+template <int MODE, int NW, int JW>
 static int launch_plane(const double* X, double* Y, const SlabMap& sm, long long B, hipStream_t st) {
   const size_t shm = (size_t)slab_lds(sm.o0.K, sm.o1.K, sm.o1.M) * sizeof(double);
-  const int rc = slab_shm(plane_par_kernel<MODE, NW>, shm);
+  const int rc = slab_shm(plane_par_kernel<MODE, NW, JW>, shm);
   if (rc) return rc;
-  hipLaunchKernelGGL((plane_par_kernel<MODE, NW>), dim3((unsigned)B), dim3(64 * NW), shm, st, X, Y, sm);
+  hipLaunchKernelGGL((plane_par_kernel<MODE, NW, JW>), dim3((unsigned)B), dim3(64 * NW), shm, st, X, Y, sm);
   JFX_LAUNCH_CHECK();
   return JFX_OK;
 }
 
 template <int MODE>
 static int launch_plane_w(const double* X, double* Y, const SlabMap& sm, long long B, hipStream_t st) {
-  switch (slab_waves(sm.o0.K, sm.o0, sm.o1)) {
-    case 4: return launch_plane<MODE, 4>(X, Y, sm, B, st);
-    case 8: return launch_plane<MODE, 8>(X, Y, sm, B, st);
-    default: return launch_plane<MODE, 16>(X, Y, sm, B, st);
+  if (slab_small(sm.o0) && slab_small(sm.o1)) {
+    const int n = slab_items<1>(sm.o0.K, sm.o0, sm.o1);
+    if (slab_many(B, n)) return launch_plane<MODE, 4, 2>(X, Y, sm, B, st);
+    if (n <= 2) return launch_plane<MODE, 2, 1>(X, Y, sm, B, st);
+    if (n <= 4) return launch_plane<MODE, 4, 1>(X, Y, sm, B, st);
+    if (n <= 6) return launch_plane<MODE, 6, 1>(X, Y, sm, B, st);
+    return launch_plane<MODE, 8, 1>(X, Y, sm, B, st);
   }
+  const int n = slab_items<2>(sm.o0.K, sm.o0, sm.o1);
+  return n <= 8 ? launch_plane<MODE, 8, 2>(X, Y, sm, B, st) : launch_plane<MODE, 16, 2>(X, Y, sm, B, st);
 }
 
-template <int NW>
+template <int NW, int JW>
 static int launch_fd(const double* X, double* Y, const FdMap& fm, long long B, hipStream_t st) {
   const size_t shm = (size_t)slab_lds(fm.w0.K, fm.w1.K, fm.w1.M) * sizeof(double);
-  const int rc = slab_shm(plane_fd_par_kernel<NW>, shm);
+  const int rc = slab_shm(plane_fd_par_kernel<NW, JW>, shm);
   if (rc) return rc;
-  hipLaunchKernelGGL(plane_fd_par_kernel<NW>, dim3((unsigned)B), dim3(64 * NW), shm, st, X, Y, fm);
+  hipLaunchKernelGGL((plane_fd_par_kernel<NW, JW>), dim3((unsigned)B), dim3(64 * NW), shm, st, X, Y, fm);
   JFX_LAUNCH_CHECK();
   return JFX_OK;
 }
@@ -188,11 +202,16 @@ int jfx_plane_fd_par(const double* W0, const double* W1, const double* V0, const
   if (B == 0) return JFX_OK;
   fm.E = E;
   fm.scale = scale;
-  switch (slab_waves(n0, fm.w0, fm.w1)) {
-    case 4: return launch_fd<4>(X, Y, fm, B, stream);
-    case 8: return launch_fd<8>(X, Y, fm, B, stream);
-    default: return launch_fd<16>(X, Y, fm, B, stream);
+  if (slab_small(fm.w0) && slab_small(fm.w1)) {
+    const int n = slab_items<1>(n0, fm.w0, fm.w1);
+    if (slab_many(B, n)) return launch_fd<4, 2>(X, Y, fm, B, stream);
+    if (n <= 2) return launch_fd<2, 1>(X, Y, fm, B, stream);
+    if (n <= 4) return launch_fd<4, 1>(X, Y, fm, B, stream);
+    if (n <= 6) return launch_fd<6, 1>(X, Y, fm, B, stream);
+    return launch_fd<8, 1>(X, Y, fm, B, stream);
   }
+  return slab_items<2>(n0, fm.w0, fm.w1) <= 8 ? launch_fd<8, 2>(X, Y, fm, B, stream)
+                                              : launch_fd<16, 2>(X, Y, fm, B, stream);
 }
 
 }  // extern "C"

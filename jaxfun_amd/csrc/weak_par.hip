@@ -20,7 +20,7 @@ struct WeakMap {
   ParOp b, d, tb, td;
 };
 
-template <int NW>
+template <int NW, int JW>
 __global__ __launch_bounds__(64 * NW) void weak_par_kernel(const double* __restrict__ U, const double* __restrict__ kq,
                                                            double* __restrict__ Y, WeakMap wm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -30,51 +30,65 @@ __global__ __launch_bounds__(64 * NW) void weak_par_kernel(const double* __restr
   const long long b = blockIdx.x;
   const double* kb = kq + b * Q * Q;
   const int LXn = slab_ldx(n), LXq = slab_ldx(Q), LTn = slab_ldt(n), LTq = slab_ldt(Q);
-  Acc4 acc, sum;
-  acc_zero(sum);
-  const WaveA we = wave_a(w, n, wm.b), wp = wave_a(w, Q, wm.tb);
-  const bool one = w < items_b(wm.b, Q), onp = w < items_b(wm.tb, n);
-  const ItemB ie = item_b(w, wm.b, Q), ip = item_b(w, wm.tb, n);
+  Acc<JW> acc, sum;
+  sum.zero();
+  WaveA<JW> we, wp;
+  ItemB<JW> ie, ip;
+  we.init(w, n, wm.b);
+  wp.init(w, Q, wm.tb);
+  ie.init(w, wm.b, Q);
+  ip.init(w, wm.tb, n);
+  we.prefetch(wm.b);
+#pragma unroll 1
   for (int t = 0; t < 2; ++t) {
     const ParOp &e0 = t ? wm.b : wm.d, &e1 = t ? wm.d : wm.b, &p0 = t ? wm.tb : wm.td, &p1 = t ? wm.td : wm.tb;
-    slab_stage<64 * NW>(U + b * n * n, n, n, S);
+    // opaque copies: without them the loads and addresses that both halves share
+    // are hoisted out of the loop and held in 150 registers
+    const double *Ut = U + b * n * n, *kt = kb;
+    asm volatile("" : "+s"(Ut), "+s"(kt));
+    slab_stage<64 * NW>(Ut, n, n, S);
     __syncthreads();
-    acc_zero(acc);
+    acc.zero();
     if (we.on) phase_a<MODE_EVAL>(S, LXn, e1, we, acc);
+    ie.prefetch(e0);
     __syncthreads();
     if (we.on) store_t<MODE_EVAL>(S, LTq, e1, we, acc);
     __syncthreads();
-    acc_zero(acc);
-    if (one) phase_b<MODE_EVAL>(S, LTq, e0, ie, acc);
+    acc.zero();
+    if (ie.on) phase_b<MODE_EVAL>(S, LTq, e0, ie, acc);
+    wp.prefetch(p1);
     __syncthreads();
-    if (one) each_b<MODE_EVAL>(e0, ie, Q, acc, [&](int m, int c, double v) { S[m * LXq + c] = v * kb[m * Q + c]; });
+    if (ie.on) each_b<MODE_EVAL>(e0, ie, Q, acc, [&](int m, int c, double v) { S[m * LXq + c] = v * kt[m * Q + c]; });
     slab_zero_pad<64 * NW>(Q, Q, S);
     __syncthreads();
-    acc_zero(acc);
+    acc.zero();
     if (wp.on) phase_a<MODE_PROJ>(S, LXq, p1, wp, acc);
+    ip.prefetch(p0);
     __syncthreads();
     if (wp.on) store_t<MODE_PROJ>(S, LTn, p1, wp, acc);
     __syncthreads();
-    if (onp) phase_b<MODE_PROJ>(S, LTn, p0, ip, sum);
-    __syncthreads();
+    if (ip.on) phase_b<MODE_PROJ>(S, LTn, p0, ip, sum);
+    if (t == 0) {
+      we.prefetch(wm.d);
+      __syncthreads();
+    }
   }
-  if (onp) {
+  if (ip.on) {
     double* Yb = Y + b * n * n;
     each_b<MODE_PROJ>(wm.tb, ip, n, sum, [&](int m, int c, double v) { Yb[m * n + c] = v; });
   }
 }
 
 bool par_op(const double* frag, int M, int K, int mode, int sgn, int bp, int bq, ParOp& o);
-int slab_waves(int K0, const ParOp& o0, const ParOp& o1);
 
-template <int NW>
+template <int NW, int JW>
 static int launch_weak(const double* U, const double* kq, double* Y, const WeakMap& wm, long long B, hipStream_t st) {
   const int a = slab_lds(wm.b.K, wm.b.K, wm.b.M), c = slab_lds(wm.b.M, wm.b.M, wm.b.K);
   const size_t shm = (size_t)(a > c ? a : c) * sizeof(double);
   if (shm > 64 * 1024)
-    JFX_CHECK_HIP(hipFuncSetAttribute((const void*)weak_par_kernel<NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    JFX_CHECK_HIP(hipFuncSetAttribute((const void*)weak_par_kernel<NW, JW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       (int)shm));
-  hipLaunchKernelGGL(weak_par_kernel<NW>, dim3((unsigned)B), dim3(64 * NW), shm, st, U, kq, Y, wm);
+  hipLaunchKernelGGL((weak_par_kernel<NW, JW>), dim3((unsigned)B), dim3(64 * NW), shm, st, U, kq, Y, wm);
   JFX_LAUNCH_CHECK();
   return JFX_OK;
 }
@@ -94,12 +108,14 @@ int jfx_weak_par(const double* FB, int sB, const double* FD, int sD, const doubl
       n > SLAB_MAX || Q > SLAB_MAX || B < 0 || B > 0x7fffffffLL)
     return set_error("weak_par: %lld slabs, n = %d, Q = %d", B, n, Q), JFX_ESHAPE;
   if (B == 0) return JFX_OK;
-  const int a = slab_waves(n, wm.b, wm.b), c = slab_waves(Q, wm.tb, wm.tb);
-  switch (a > c ? a : c) {
-    case 4: return launch_weak<4>(U, k, Y, wm, B, stream);
-    case 8: return launch_weak<8>(U, k, Y, wm, B, stream);
-    default: return launch_weak<16>(U, k, Y, wm, B, stream);
+  if (Q <= 64 && n <= 64) {
+    const int a = slab_items<1>(n, wm.b, wm.b), c = slab_items<1>(Q, wm.tb, wm.tb), m = a > c ? a : c;
+    return m <= 2   ? launch_weak<2, 1>(U, k, Y, wm, B, stream)
+           : m <= 4 ? launch_weak<4, 1>(U, k, Y, wm, B, stream)
+                    : launch_weak<8, 1>(U, k, Y, wm, B, stream);
   }
+  const int a = slab_items<2>(n, wm.b, wm.b), c = slab_items<2>(Q, wm.tb, wm.tb);
+  return (a > c ? a : c) <= 8 ? launch_weak<8, 2>(U, k, Y, wm, B, stream) : launch_weak<16, 2>(U, k, Y, wm, B, stream);
 }
 
 }  // extern "C"

@@ -265,12 +265,13 @@ def pcg(apply, b: torch.Tensor, precond, x0: torch.Tensor | None = None, rtol: f
     z = precond(r)
     p = K.lincomb([(1.0, z)])
     rz = batched_dot(r, z)
-    # left[i]: systems still active after iteration i.  The host reads it while the
-    # next iteration's operator and update are queued, so the device never waits for
-    # the host; systems that have stopped do not change, so a queued iteration too
-    # many changes nothing.
+    # left[i]: systems still active after iteration i, which the device stores to
+    # pinned memory.  The host reads it while the next iteration's operator and update
+    # are queued, so the device never waits for the host; systems that have stopped do
+    # not change, so a queued iteration too many changes nothing.
     left = torch.zeros(_LEFT_SLOTS, dtype=torch.int32, device=b.device)
     host = torch.empty(2, dtype=torch.int32, pin_memory=True)
+    seen = host.numpy()
     ev = [torch.cuda.Event(), torch.cuda.Event()]
     for it in range(maxiter):
         slot = it % _LEFT_SLOTS
@@ -278,17 +279,18 @@ def pcg(apply, b: torch.Tensor, precond, x0: torch.Tensor | None = None, rtol: f
             left.zero_()
         q = apply(p)
         _lib.call("jfx_pcg_step", K._p(x), K._p(r), K._p(p), K._p(q), K._p(rz), K._p(bb), rtol * rtol, K._p(active),
-                  K._p(iters), left.data_ptr() + 4 * slot, B, n, K._s())
-        host[it % 2].copy_(left[slot], non_blocking=True)
+                  K._p(iters), left.data_ptr() + 4 * slot, host.data_ptr() + 4 * (it % 2), B, n, K._s())
         ev[it % 2].record()
         if it and it % check_every == 0:  # after iteration it - 1
             ev[(it - 1) % 2].synchronize()
-            if int(host[(it - 1) % 2]) == 0:
+            if seen[(it - 1) % 2] == 0:
                 break
         if snap_out is not None and it + 1 in snapshots:
             snap_out[it + 1] = (x.clone(), r.clone())
         z = precond(r)
         _lib.call("jfx_pcg_direction", K._p(p), K._p(z), K._p(r), K._p(rz), K._p(active), B, n, K._s())
+    if maxiter > 0:
+        ev[it % 2].synchronize()  # the last store to `host`, which is freed on return
     if breakdown == "raise":
         nbad = int((iters < 0).sum().item())
         if nbad:

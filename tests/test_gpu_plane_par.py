@@ -44,6 +44,27 @@ def test_plane(dev, mode, s0, s1):
             assert np.all(np.abs(y - ref) <= (K0 + K1 + 10) * 2 * EPS * bound + 1e-300), (M0, K0, M1, K1, epi, acc)
 
 
+def test_many_slabs(dev):
+    """More than three slabs per CU above 32 x 32 take the four-wave kernels: the same
+    values as a batch that does not, up to the order of sums."""
+    import torch
+
+    from jaxfun_amd import kernels as K
+
+    rng = np.random.default_rng(2)
+    for n, N in ((62, 64), (33, 40), (30, 32)):
+        A, W = _structured(rng, N, n, 1, 1), _structured(rng, n, n, 3, 1)
+        op, w = K.AxisOperator(torch.tensor(A, device=dev), K.evaluates_parity()), \
+            K.AxisOperator(torch.tensor(W, device=dev), K.mixes_parity())
+        X = torch.tensor(rng.standard_normal((800, n, n)), device=dev)
+        E = torch.tensor(rng.uniform(0.5, 2, (n, n)), device=dev)
+        for f in (lambda x: K.plane(op, op, x), lambda x: K.plane_fd(w, w, w, w, x, E)):
+            many, few = f(X), f(X[:700].contiguous())
+            scale = float(few.abs().max())
+            assert float((many[:700] - few).abs().max()) <= 1e-13 * n * scale
+            assert float((f(X[700:].contiguous()) - many[700:]).abs().max()) <= 1e-13 * n * scale
+
+
 @pytest.mark.parametrize("n0,n1", [(1, 1), (2, 5), (16, 16), (31, 33), (62, 62), (64, 64), (97, 40), (62, 126), (128, 128)])
 def test_plane_fd(dev, n0, n1):
     import torch

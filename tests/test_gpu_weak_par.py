@@ -60,15 +60,18 @@ def test_pcg_steps(dev, n):
     T = lambda a: torch.tensor(a, device=dev)  # noqa: E731
     xd, rd, pd, qd, zd, rzd, bbd, ad, itd = (T(a) for a in (x, r, p, q, z, rz, bb, act, it))
     left = torch.zeros(1, dtype=torch.int32, device=dev)
+    host = torch.full((1,), -7, dtype=torch.int32).pin_memory()
     _lib.call("jfx_pcg_step", K._p(xd), K._p(rd), K._p(pd), K._p(qd), K._p(rzd), K._p(bbd), 1e-20, K._p(ad), K._p(itd),
-              K._p(left), Bt, n, K._s())
+              K._p(left), host.data_ptr(), Bt, n, K._s())
+    torch.cuda.synchronize()
     a = rz / np.sum(p * q, axis=1)
     x1, r1 = x + a[:, None] * p, r - a[:, None] * q
     x1[0], r1[0] = x[0], r[0]
     eps = 1e-15 * n + 1e-14
     np.testing.assert_allclose(xd.cpu().numpy()[:4], x1[:4], rtol=eps, atol=eps)
     np.testing.assert_allclose(rd.cpu().numpy()[:4], r1[:4], rtol=eps, atol=eps)
-    assert ad.cpu().tolist() == [0, 0, 1, 1, 0] and itd.cpu().tolist() == [7, 3, 3, 3, -1] and int(left) == 2
+    assert ad.cpu().tolist() == [0, 0, 1, 1, 0] and itd.cpu().tolist() == [7, 3, 3, 3, -1] and int(left) == (Bt << 16) + 2
+    assert int(host[0]) == 2
     rnow, p0 = rd.cpu().numpy(), pd.clone()
     _lib.call("jfx_pcg_direction", K._p(pd), K._p(zd), K._p(rd), K._p(rzd), K._p(ad), Bt, n, K._s())
     s = np.sum(rnow * z, axis=1)
