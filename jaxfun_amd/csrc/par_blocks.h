@@ -3,8 +3,8 @@
 //
 // One workgroup of NW waves holds a slab in LDS and applies one operator along
 // each axis:  T = X A1^T (rows x M1),  Y = A0 T (M0 x M1).
-//   phase A  a wave owns 16 rows of X and JW half column blocks of T, even and odd
-//            part: all of T sits in the workgroup's registers, so T overwrites X
+//   phase A  a wave owns JW 16-row blocks of X and a half column block of T, even and
+//            odd part: all of T sits in the workgroup's registers, so T overwrites X
 //   phase B  a wave owns a half row block of Y and JW column blocks
 // Up to 64 x 64 (JW = 1) a wave loads all its fragments of a phase before the
 // barrier in front of it: with one slab per CU a phase is as long as its loads
@@ -110,6 +110,30 @@ __device__ __forceinline__ void slab_stage(const double* __restrict__ X, int K0,
   slab_zero_pad<NT>(K0, K1, Xs);
 }
 
+// The same in two halves: the loads of a slab into registers (at most 8 pairs a
+// thread: 16384 values for 1024 threads; K1 even, X 16-byte aligned), and later
+// the stores into LDS.
+template <int NT>
+__device__ __forceinline__ void slab_load8(const double* __restrict__ X, int K0, int K1, d2 (&v)[8]) {
+  const int tid = own_tid(), n2 = K0 * (K1 / 2);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int e = tid + NT * u;
+    v[u] = *(const d2*)(X + 2 * (e < n2 ? e : n2 - 1));  // unconditional: v is not live through branches
+  }
+}
+template <int NT>
+__device__ __forceinline__ void slab_put8(const d2 (&v)[8], int K0, int K1, double* Xs) {
+  const int tid = own_tid(), n2 = K0 * (K1 / 2), LDX = slab_ldx(K1);
+  const unsigned kh = K1 / 2;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const unsigned e = tid + NT * u, i = e / kh, k = e - i * kh;
+    if ((int)e < n2) *(d2*)&Xs[i * LDX + 2 * k] = v[u];
+  }
+  slab_zero_pad<NT>(K0, K1, Xs);
+}
+
 // even and odd operand of k-step s from a row of X (element stride 1)
 template <int MODE>
 __device__ __forceinline__ void row_operands(const double* row, int s, int kk, int K, double sg, double& e, double& o) {
@@ -211,40 +235,44 @@ struct Frag {
 template <int JW>
 constexpr int frag_steps() { return JW == 1 ? 8 : 2; }
 
-// A wave's share of phase A: a row block and JW half column blocks.
+// A wave's share of phase A: a half column block and JW row blocks, which share
+// the operator's fragments (the other way round, JW column blocks of one row block,
+// the fragments of a 128 x 128 pass are 512 KB from L2 instead of 256: 250 against
+// 238 us for 2048 slabs).
 template <int JW>
 struct WaveA {
-  int rb, cb[JW];
+  int cb, rb[JW];
   bool on, ok[JW];
-  Frag<JW, frag_steps<JW>()> f;
+  Frag<1, frag_steps<JW>()> f;
 
   __device__ __forceinline__ void init(int w, int K0, const ParOp& o) {
-    const int ncg = (o.nrb + JW - 1) / JW, nrow = slab_pad(K0) >> 4;
-    rb = w / ncg;
-    const int cg = w - rb * ncg;
-    on = rb < nrow;
+    const int nrow = slab_pad(K0) >> 4, rg = w / o.nrb;
+    cb = w - rg * o.nrb;
+    on = JW * rg < nrow;
 #pragma unroll
     for (int j = 0; j < JW; ++j) {
-      ok[j] = JW * cg + j < o.nrb;
-      cb[j] = ok[j] ? JW * cg + j : JW * cg;  // a copy whose results are not stored
+      ok[j] = JW * rg + j < nrow;
+      rb[j] = ok[j] ? JW * rg + j : 0;  // a copy whose results are not stored
     }
   }
-  __device__ __forceinline__ void prefetch(const ParOp& o) { f.init(o, cb); }
+  __device__ __forceinline__ void prefetch(const ParOp& o) {
+    const int c[1] = {cb};
+    f.init(o, c);
+  }
 };
 
 template <int MODE, int JW>
 __device__ __forceinline__ void phase_a(const double* Xs, int LDX, const ParOp& o, WaveA<JW>& wa, Acc<JW>& acc) {
   const int lane = own_lane(), kk = lane >> 4, cl = lane & 15;
-  const double* row = Xs + (16 * wa.rb + cl) * LDX;
   const double sg = o.sgn;
   const int K = o.K;
-  wa.f.each([&](int s, const double(&a)[2][JW]) {
-    double e, d;
-    row_operands<MODE>(row, s, kk, K, sg, e, d);
+  wa.f.each([&](int s, const double(&a)[2][1]) {
 #pragma unroll
     for (int j = 0; j < JW; ++j) {
-      acc.v[0][j] = mfma_f64(e, a[0][j], acc.v[0][j]);
-      acc.v[1][j] = mfma_f64(d, a[1][j], acc.v[1][j]);
+      double e, d;
+      row_operands<MODE>(Xs + (16 * wa.rb[j] + cl) * LDX, s, kk, K, sg, e, d);
+      acc.v[0][j] = mfma_f64(e, a[0][0], acc.v[0][j]);
+      acc.v[1][j] = mfma_f64(d, a[1][0], acc.v[1][j]);
     }
   });
 }
@@ -255,14 +283,14 @@ __device__ __forceinline__ void store_t(double* T, int LDT, const ParOp& o, cons
   const int lane = own_lane(), cl = lane & 15;
   const double sg = o.sgn;
   const int M = o.M, Mh = (M + 1) >> 1;
+  const int m = 16 * wa.cb + cl;
+  if (m >= Mh) return;
 #pragma unroll
   for (int j = 0; j < JW; ++j) {
     if (!wa.ok[j]) break;
-    const int m = 16 * wa.cb[j] + cl;
-    if (m >= Mh) continue;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      double* d = T + (16 * wa.rb + mfma16_row_f64(lane, r)) * LDT;
+      double* d = T + (16 * wa.rb[j] + mfma16_row_f64(lane, r)) * LDT;
       const double e = acc.v[0][j][r], q = acc.v[1][j][r];
       if constexpr (MODE == MODE_EVAL) {
         d[m] = e + q;
@@ -322,7 +350,7 @@ __device__ __forceinline__ void phase_b(const double* T, int LDT, const ParOp& o
 // waves that cover phase A of (K0 rows) x o1 and phase B of o0
 template <int JW>
 inline int slab_items(int K0, const ParOp& o0, const ParOp& o1) {
-  const int a = (slab_pad(K0) / 16) * ((o1.nrb + JW - 1) / JW), b = items_b<JW>(o0, o1.M);
+  const int a = (slab_pad(K0) / 16 + JW - 1) / JW * o1.nrb, b = items_b<JW>(o0, o1.M);
   return a > b ? a : b;
 }
 

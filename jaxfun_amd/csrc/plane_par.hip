@@ -58,6 +58,50 @@ __global__ __launch_bounds__(64 * NW) void plane_par_kernel(const double* __rest
   });
 }
 
+// Slabs of which one fills a CU's LDS, several per CU: a persistent workgroup loads
+// the next slab into registers while it multiplies the current one.  2048 slabs of
+// 128 x 128: 253 us one slab per workgroup, 238 us here (reading and writing take
+// 101 us, the FP64 products 119 us; 16 waves in step leave the matrix units idle
+// around the barriers: LDS stores of X and T and the stores of Y are 40% of a
+// slab's 28 us).  Where two workgroups fit, they overlap by themselves: 512 slabs
+// of 96 x 94 36 us, persistent 41 us.
+template <int MODE>
+__global__ __launch_bounds__(1024) void plane_par_stream_kernel(const double* __restrict__ X, double* __restrict__ Y,
+                                                                SlabMap sm, long long B) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  double* S = reinterpret_cast<double*>(smem);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int K0 = sm.o0.K, K1 = sm.o1.K, M0 = sm.o0.M, M1 = sm.o1.M, LDT = slab_ldt(M1);
+  WaveA<2> wa;
+  ItemB<2> ib;
+  Acc<2> acc;
+  wa.init(w, K0, sm.o1);
+  ib.init(w, sm.o0, M1);
+  d2 v[8];
+  slab_load8<1024>(X + blockIdx.x * (long long)K0 * K1, K0, K1, v);
+#pragma unroll 1
+  for (long long b = blockIdx.x; b < B; b += gridDim.x) {
+    wa.prefetch(sm.o1);
+    slab_put8<1024>(v, K0, K1, S);
+    __syncthreads();
+    const long long bn = b + gridDim.x;
+    slab_load8<1024>(X + (bn < B ? bn : b) * K0 * K1, K0, K1, v);
+    acc.zero();
+    if (wa.on) phase_a<MODE>(S, slab_ldx(K1), sm.o1, wa, acc);
+    ib.prefetch(sm.o0);
+    __syncthreads();
+    if (wa.on) store_t<MODE>(S, LDT, sm.o1, wa, acc);
+    __syncthreads();
+    acc.zero();
+    if (ib.on) {
+      phase_b<MODE>(S, LDT, sm.o0, ib, acc);
+      double* Yb = Y + b * M0 * M1;
+      each_b<MODE>(sm.o0, ib, M1, acc, [&](int m, int c, double y) { Yb[m * M1 + c] = y * sm.alpha; });
+    }
+    __syncthreads();  // T is free for the next slab
+  }
+}
+
 struct FdMap {
   ParOp w0, w1, v0, v1;
   const double *E, *scale;  // scale: one factor per slab, or null
@@ -149,6 +193,14 @@ static int launch_plane_w(const double* X, double* Y, const SlabMap& sm, long lo
     return launch_plane<MODE, 8, 1>(X, Y, sm, B, st);
   }
   const int n = slab_items<2>(sm.o0.K, sm.o0, sm.o1);
+  const size_t shm = (size_t)slab_lds(sm.o0.K, sm.o1.K, sm.o1.M) * sizeof(double);
+  if (n > 8 && B > 256 && shm > 80 * 1024 && !sm.epi && !sm.accum && sm.o1.K % 2 == 0 && ((uintptr_t)X & 15) == 0) {
+    const int rc = slab_shm(plane_par_stream_kernel<MODE>, shm);
+    if (rc) return rc;
+    hipLaunchKernelGGL(plane_par_stream_kernel<MODE>, dim3(256), dim3(1024), shm, st, X, Y, sm, B);
+    JFX_LAUNCH_CHECK();
+    return JFX_OK;
+  }
   return n <= 8 ? launch_plane<MODE, 8, 2>(X, Y, sm, B, st) : launch_plane<MODE, 16, 2>(X, Y, sm, B, st);
 }
 

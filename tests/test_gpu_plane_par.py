@@ -65,6 +65,26 @@ def test_many_slabs(dev):
             assert float((f(X[700:].contiguous()) - many[700:]).abs().max()) <= 1e-13 * n * scale
 
 
+@pytest.mark.parametrize("mode", [1, 2, 3])
+@pytest.mark.parametrize("M0,K0,M1,K1", [(128, 128, 127, 126), (100, 118, 128, 120), (97, 101, 99, 110)])
+def test_streamed_slabs(dev, mode, M0, K0, M1, K1):
+    """More than one slab per CU, each filling its LDS: the persistent kernel."""
+    import torch
+
+    from jaxfun_amd import kernels as K
+
+    rng = np.random.default_rng(M0 + mode)
+    A0, A1 = _structured(rng, M0, K0, mode, 1), _structured(rng, M1, K1, mode, 1)
+    op0, op1 = (K.AxisOperator(torch.tensor(a, device=dev), (mode, 1, -1, -1)) for a in (A0, A1))
+    for B in (257, 600):
+        X = torch.tensor(rng.standard_normal((B, K0, K1)), device=dev)
+        y = K.plane(op0, op1, X, alpha=0.5)
+        for b in (0, 1, 255, 256, B - 1):
+            x = X[b].cpu().numpy()
+            bound = 0.5 * np.abs(A0) @ np.abs(x) @ np.abs(A1).T
+            assert np.all(np.abs(y[b].cpu().numpy() - 0.5 * A0 @ x @ A1.T) <= (K0 + K1 + 10) * 2 * EPS * bound + 1e-300)
+
+
 @pytest.mark.parametrize("n0,n1", [(1, 1), (2, 5), (16, 16), (31, 33), (62, 62), (64, 64), (97, 40), (62, 126), (128, 128)])
 def test_plane_fd(dev, n0, n1):
     import torch
