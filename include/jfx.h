@@ -120,6 +120,16 @@ int jfx_plane_fd_par(const double* W0, const double* W1, const double* V0, const
 int jfx_weak_par(const double* FB, int sB, const double* FD, int sD, const double* FTB, int sTB, const double* FTD,
                  int sTD, int n, int Q, const double* U, const double* k, double* Y, long long B, hipStream_t stream);
 
+/* Y[b] = S0 w S1^T with w = c0 u u + c1 u ux + c2 u uy + c3 ux ux + c4 ux uy + c5 uy uy,
+ * u = B0 U[b] B1^T, ux = D0 U[b] B1^T, uy = B0 U[b] D1^T: the quadratic term of a 2D
+ * Galerkin right-hand side on a padded mesh, one launch, FP64 arithmetic, U and Y
+ * (n0 x n1) in FP64 (dtype 0) or FP32 (1).  F (host array): fragments of B0, D0 (Q0 x n0),
+ * B1, D1 (Q1 x n1) (mode 1) and S0 (n0 x Q0), S1 (n1 x Q1) (mode 2, S0's sign 1); sgn, c:
+ * host arrays of 6.  jfx_quad_par_ok: whether the sizes are taken. */
+int jfx_quad_par_ok(int n0, int Q0, int n1, int Q1);
+int jfx_quad_par(int dtype, const double* const* F, const int* sgn, const double* c, int n0, int Q0, int n1, int Q1,
+                 const void* U, void* Y, long long B, hipStream_t stream);
+
 /* Fused PCG steps over `batch` systems of n values, FP64.  jfx_pcg_step: for active
  * systems a = rz / (p, q), x += a p, r -= a q, then the stopping test of jfx_pcg_check
  * with count = 1; *left (a zeroed int) counts the systems that stay active in its low

@@ -45,6 +45,8 @@ SIGNATURES: dict[str, tuple] = {
     "jfx_plane_fd_par": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_ll, c_int, c_int, c_vp]),
     "jfx_weak_par": (c_int, [c_vp, c_int, c_vp, c_int, c_vp, c_int, c_vp, c_int, c_int, c_int, c_vp, c_vp, c_vp, c_ll,
                              c_vp]),
+    "jfx_quad_par_ok": (c_int, [c_int, c_int, c_int, c_int]),
+    "jfx_quad_par": (c_int, [c_int, c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_vp]),
     "jfx_pcg_step": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_dbl, c_vp, c_vp, c_vp, c_vp, c_int, c_ll, c_vp]),
     "jfx_pcg_direction": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_ll, c_vp]),
     "jfx_contract_bf16x": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll, c_vp]),

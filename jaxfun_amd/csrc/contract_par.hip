@@ -447,6 +447,15 @@ bool par_op(const double* frag, int M, int K, int mode, int sgn, int bp, int bq,
   return true;
 }
 
+// k-steps and row blocks per part of an operator's fragments
+bool par_shape(int M, int K, int mode, int& S, int& nrb) {
+  ParDims d;
+  if (!par_dims(M, K, mode, d)) return false;
+  S = d.S;
+  nrb = d.nrb;
+  return true;
+}
+
 template <typename T, int MODE, bool QONE, int NB, int JB>
 static int launch_par3(const T* Af, const T* X, T* Y, const ParMap& pm, hipStream_t st) {
   const int kz = par_kz(MODE, pm.K, pm.S);

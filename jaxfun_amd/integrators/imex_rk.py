@@ -18,6 +18,8 @@ accumulation and FP32 state.
 
 from __future__ import annotations
 
+import math
+
 import sympy as sp
 import torch
 
@@ -136,6 +138,45 @@ class IMEXRungeKutta:
     def apply_linear(self, U):
         return self.linear(U, self.precision) if self.linear is not None else None
 
+    _QUAD_FIELDS = ((0, 0), (1, 0), (0, 1))  # u, u_x, u_y
+
+    def _quad_coefficients(self) -> list[float]:
+        """Coefficients of u u, u u_x, u u_y, u_x u_x, u_x u_y, u_y u_y."""
+        out = [0.0] * 6
+        pos = {(0, 0): 0, (0, 1): 1, (0, 2): 2, (1, 1): 3, (1, 2): 4, (2, 2): 5}
+        for c, o1, o2 in self.nonlinear:
+            i, j = sorted((self._QUAD_FIELDS.index(o1), self._QUAD_FIELDS.index(o2)))
+            out[pos[i, j]] += c
+        return out
+
+    def _quad_operators(self):
+        """Operators of the fused nonlinear term, or None where it does not apply:
+        2D terms in u, u_x and u_y on parity bases, FP64 or mixed precision."""
+        if "quad" not in self._stage_ops:
+            T, ops = self.testspace, None
+            if len(T) == 2 and self.precision in ("f64", "bf16x6") and len(self.nonlinear) <= 4 and \
+                    all(o in self._QUAD_FIELDS for _, o1, o2 in self.nonlinear for o in (o1, o2)):
+                ops = [T[ax].backward_operator(self.Np[ax], k) for ax in (0, 1) for k in (0, 1)]
+                ops += [T[ax].scalar_product_operator(self.Np[ax]) for ax in (0, 1)]
+            self._stage_ops["quad"] = ops if ops is not None and K.quad_ok(*ops) else None
+        return self._stage_ops["quad"]
+
+    def _quad_pays(self, nbatch: int) -> bool:
+        """Whether the fused term is the faster one.  A problem is one workgroup's
+        work, so its time goes by rounds of one problem per CU; the separate launches
+        spread over the chip but cost 70 us at least.  Up to 128 mesh points an axis a
+        round takes 15 to 40 us: always.  Beyond, FP64 from 90 problems on (192 x 192:
+        100 problems 161 us fused, 174 separate; 20 problems 155 / 105); mixed precision
+        too, except that meshes in multiples of 64 points, which the separate bf16x6
+        contractions read best, need rounds that are nearly full (256 problems on 192 x
+        192 185 / 189 us alone and 25 us less in a step, 160 problems 172 / 148)."""
+        if max(self.Np) <= 128:
+            return True
+        cus = K.num_cus()
+        if self.precision != "f64" and all(q % 64 == 0 for q in self.Np):
+            return nbatch >= 0.9 * cus * -(-nbatch // cus)
+        return nbatch >= 0.35 * cus
+
     def nonlinear_rhs_scalar_product(self, U):
         """(v, N(u)) with N evaluated on the padded mesh (integrators/base.py:238-248)."""
         if not self.nonlinear:
@@ -143,6 +184,9 @@ class IMEXRungeKutta:
         T = self.testspace
         prec = self.precision
         nb = U.ndim - 2
+        ops = self._quad_operators()
+        if ops is not None and nb >= 0 and not U.is_complex() and self._quad_pays(math.prod(U.shape[:nb])):
+            return K.quadratic_term(*ops, self._quad_coefficients(), U.contiguous())
         fields = {}
         needed = set()
         for _, o1, o2 in self.nonlinear:

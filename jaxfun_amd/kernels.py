@@ -680,6 +680,37 @@ def weak_laplacian(B: AxisOperator, D: AxisOperator, TB: AxisOperator, TD: AxisO
     return Y
 
 
+def quad_ok(B0, D0, B1, D1, S0, S1) -> bool:
+    """Whether the fused quadratic term (csrc/quad_par.hip) takes these operators:
+    B, D evaluate a parity basis and its derivative, S projects, per axis."""
+    ops = (B0, D0, B1, D1, S0, S1)
+    if any(type(o) is not AxisOperator or o.parity is None for o in ops):
+        return False
+    n0, Q0, n1, Q1 = B0.K, B0.M, B1.K, B1.M
+    if any((o.M, o.K, o.parity[0]) != want for o, want in zip(ops, (
+            (Q0, n0, PAR_EVAL), (Q0, n0, PAR_EVAL), (Q1, n1, PAR_EVAL), (Q1, n1, PAR_EVAL), (n0, Q0, PAR_PROJ),
+            (n1, Q1, PAR_PROJ)))) or S0.parity[1] != 1:
+        return False
+    return _lib.load().jfx_quad_par_ok(n0, Q0, n1, Q1) == 1 and all(o.fragments("f64") is not None for o in ops)
+
+
+def quadratic_term(B0, D0, B1, D1, S0, S1, coefficients, U: torch.Tensor) -> torch.Tensor:
+    """``S0 w S1^T`` over the last two axes of U (FP64 or FP32, FP64 arithmetic) with
+    w = c0 u u + c1 u u_x + c2 u u_y + c3 u_x u_x + c4 u_x u_y + c5 u_y u_y on the mesh
+    (operators as :func:`quad_ok` takes them)."""
+    _req(U, torch.float32 if U.dtype == torch.float32 else torch.float64, "U")
+    if tuple(U.shape[-2:]) != (B0.K, B1.K):
+        raise ValueError(f"quadratic_term: U {tuple(U.shape)} does not end with {(B0.K, B1.K)}")
+    fr = [o.fragments("f64") for o in (B0, D0, B1, D1, S0, S1)]
+    F = (ctypes.c_void_p * 6)(*[f[0].data_ptr() for f in fr])
+    sgn = (ctypes.c_int * 6)(*[f[2] for f in fr])
+    c = (ctypes.c_double * 6)(*[float(v) for v in coefficients])
+    Y = torch.empty_like(U)
+    _lib.call("jfx_quad_par", 0 if U.dtype == torch.float64 else 1, F, sgn, c, B0.K, B0.M, B1.K, B1.M, _p(U), _p(Y),
+              math.prod(U.shape[:-2]), _s())
+    return Y
+
+
 PLANE_PRECISIONS = ("f64", "bf16x6", "i8x5", "i8x6")
 
 
