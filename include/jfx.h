@@ -398,13 +398,14 @@ int jfx_cast(int direction, const void* x, void* y, long long n, hipStream_t str
  *   float-split slices each ([3][AP][AP] per table at 3*voff) in mode 1, or
  *   as the fp16 high and low terms of V_p * 2^texp ([2][AP][AP] at 2*voff,
  *   texp in the item, max |V_p| 2^texp < 2^14) in mode 2.  lam at loff.
- * mode 0: FP64 MFMA (fp64 I/O); mode 1: 3-term BF16 split MFMA with FP32
- *   accumulation/storage and FP64 tridiagonal recurrences whose sweep values
- *   and multipliers are stored in FP32 (io_f32 selects float or double F/U).
+ * mode 0: FP64 MFMA (fp64 I/O; one 8-wave kernel for nwaves 4 and 8).
+ * mode 1: 3-term BF16 split MFMA with FP32 accumulation/storage and FP64
+ *   tridiagonal recurrences whose sweep values and multipliers are stored in
+ *   FP32 (io_f32 selects float or double F/U).
  *   nwaves 4 or 8 (mode 1: 4 = two 4-wave workgroups per CU, one column
  *   parity at a time; 8 = one 8-wave workgroup per CU, both column parities
- *   at once with whole-row F reads and U writes); scratch holds
- *   nblocks * jfx_helm_scratch_doubles_per_block() doubles (mode 0 only).
+ *   at once with whole-row F reads and U writes); mode 0
+ *   wants scratch of nblocks * jfx_helm_scratch_doubles_per_block() doubles.
  * mode 2: as mode 1 with a 2-term fp16 split (three MFMA products instead of
  *   six): each operand block is scaled by a power of two from its largest
  *   entry before the split and the products are scaled back exactly; nwaves 4

@@ -16,11 +16,11 @@
 // queue g mod nq -- workgroups are dispatched round-robin over the XCDs, so a
 // queue's tables stay in one XCD's L2 -- and moves on to the next queues when
 // its own is drained; every workgroup loops until all queues are empty.
-//   MODE 0: FP64 MFMA, FP64 storage
-//   MODE 1: BF16 3-term float split (6 products) MFMA, FP32 accumulation and
-//           storage, FP64 tridiagonal solve.
+//   mode 0 (helm64_kernel): FP64 MFMA, FP64 storage
+//   mode 1 (compact and pair kernels): BF16 3-term float split (6 products) MFMA,
+//           FP32 accumulation and storage, FP64 tridiagonal solve.
 //   mode 2 (compact kernel only): FP16 2-term split (3 products) of operands
-//           scaled by powers of two, otherwise as MODE 1.
+//           scaled by powers of two, otherwise as mode 1.
 #include <mutex>
 #include <type_traits>
 
@@ -37,17 +37,6 @@ struct HelmItem {
 };
 
 constexpr int HMAXA = 128;  // a, b <= 128  (n <= 256)
-
-template <int MODE>
-struct HelmTypes;
-template <>
-struct HelmTypes<0> {
-  typedef double TS;
-};
-template <>
-struct HelmTypes<1> {
-  typedef float TS;
-};
 
 __global__ void helm_reset(int* counters, int nq) {
   if ((int)threadIdx.x < nq) counters[threadIdx.x] = 0;
@@ -100,179 +89,6 @@ __device__ __forceinline__ double rcp64(double x) {
   return fma(r, e, r);
 }
 
-template <int MODE>
-struct HelmLDS;
-template <>
-struct HelmLDS<0> {  // FP64: work block 128 x 129 doubles, V slab 16 x 129 doubles; multipliers in global scratch
-  static constexpr int LDW = 129, KS = 16;
-  static constexpr size_t WK = (size_t)HMAXA * LDW * 8, U1 = (size_t)KS * (HMAXA + 1) * 8;
-};
-template <>
-struct HelmLDS<1> {  // bf16 split: work block 128 x 130 floats; V slab (3 bf16 slices of 128 x 32) shares
-                     // its space with the 128 x 128 FP32 tridiagonal multipliers
-  static constexpr int LDW = 130, KS = 32, VLD = 40;
-  static constexpr size_t WK = (size_t)HMAXA * LDW * 4, U1 = (size_t)HMAXA * HMAXA * 4;
-};
-constexpr size_t HTAB = 3 * HMAXA * 8;
-
-// One GEMM phase (a x b block):   C = A * Wk   with A an (AP x AP) table applied by rows
-//   phase 1: A = V^T, result back into Wk (each wave owns its column panels)
-//   phase 3: A = V,   result scattered to U
-// The next k-slab of A is prefetched into registers while the current one is multiplied.
-template <int MODE, int NW, typename TIO, bool TO_GLOBAL>
-__device__ __forceinline__ void helm_gemm_phase(const HelmItem& I, int q, int b, const double* __restrict__ tabd,
-                                                const unsigned short* __restrict__ tabs,
-                                                typename HelmTypes<MODE>::TS* Wk, unsigned char* vslab,
-                                                TIO* __restrict__ Ub) {
-  typedef typename HelmTypes<MODE>::TS TS;
-  constexpr int LDW = HelmLDS<MODE>::LDW, KS = HelmLDS<MODE>::KS, NT = NW * 64;
-  constexpr int PPW = 8 / NW;  // column panels per wave (b <= 128 -> <= 8 panels)
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int a = I.a, AP = I.AP, n = I.n;
-  const int npanel = (b + 15) >> 4, nrb = (a + 15) >> 4;  // output row blocks
-  typedef typename std::conditional<MODE == 0, v4d, v4f>::type vacc;
-  vacc acc[PPW][8];
-#pragma unroll
-  for (int pp = 0; pp < PPW; ++pp)
-#pragma unroll
-    for (int rb = 0; rb < 8; ++rb) acc[pp][rb] = vacc{0, 0, 0, 0};
-
-  // register prefetch of one k-slab
-  constexpr int NPRE = (MODE == 0) ? (KS * HMAXA / NT) : (3 * HMAXA * 4 / NT);
-  typedef typename std::conditional<MODE == 0, double, v8u16>::type PT;
-  PT pre[NPRE];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < NPRE; ++u) {
-      const int e = tid + u * NT;
-      if constexpr (MODE == 0) {
-        if (e < KS * AP) {
-          const int kk = e / AP, m = e - kk * AP;
-          pre[u] = tabd[I.voff + (long long)(k0 + kk) * AP + m];
-        }
-      } else {
-        if (e < 3 * AP * 4) {
-          const int sl = e / (AP * 4), rem = e - sl * AP * 4, m = rem >> 2, part = rem & 3;
-          pre[u] = *(const v8u16*)(tabs + 3 * I.voff + (long long)sl * AP * AP + (long long)m * AP + k0 + part * 8);
-        }
-      }
-    }
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int u = 0; u < NPRE; ++u) {
-      const int e = tid + u * NT;
-      if constexpr (MODE == 0) {
-        if (e < KS * AP) {
-          const int kk = e / AP, m = e - kk * AP;
-          reinterpret_cast<double*>(vslab)[kk * (HMAXA + 1) + m] = pre[u];
-        }
-      } else {
-        constexpr int VLD = HelmLDS<1>::VLD;
-        if (e < 3 * AP * 4) {
-          const int sl = e / (AP * 4), rem = e - sl * AP * 4, m = rem >> 2, part = rem & 3;
-          *(v8u16*)&reinterpret_cast<unsigned short*>(vslab)[(sl * HMAXA + m) * VLD + part * 8] = pre[u];
-        }
-      }
-    }
-  };
-
-  fetch(0);
-  for (int k0 = 0; k0 < AP; k0 += KS) {
-    store();
-    __syncthreads();
-    if (k0 + KS < AP) fetch(k0 + KS);
-#pragma unroll
-    for (int pp = 0; pp < PPW; ++pp) {
-      const int pc = w + pp * NW;
-      if (pc < npanel) {
-        const int col = pc * 16 + (lane & 15);
-        const bool cok = col < b;
-        if constexpr (MODE == 0) {
-          const double* Vs0 = reinterpret_cast<const double*>(vslab);
-#pragma unroll
-          for (int ks = 0; ks < KS; ks += 4) {
-            const int k = k0 + ks + (lane >> 4);
-            double bv = (cok && k < a) ? (double)Wk[k * LDW + col] : 0.0;
-#pragma unroll
-            for (int rb = 0; rb < 8; ++rb)
-              if (rb < nrb)
-                acc[pp][rb] = mfma_f64(Vs0[(ks + (lane >> 4)) * (HMAXA + 1) + rb * 16 + (lane & 15)], bv,
-                                       acc[pp][rb]);
-          }
-        } else {
-          constexpr int VLD = HelmLDS<1>::VLD;
-          const unsigned short* Vsl = reinterpret_cast<const unsigned short*>(vslab);
-          v8u16 bh, bm, bl;
-          float xv[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int k = k0 + 8 * (lane >> 4) + e;
-            xv[e] = (cok && k < a) ? (float)Wk[k * LDW + col] : 0.f;
-          }
-          split3_pk8(xv, bh, bm, bl);
-#pragma unroll
-          for (int rb = 0; rb < 8; ++rb) {
-            if (rb < nrb) {
-              const int row = rb * 16 + (lane & 15), ko = 8 * (lane >> 4);
-              v8u16 ah = *(const v8u16*)&Vsl[(0 * HMAXA + row) * VLD + ko];
-              v8u16 am = *(const v8u16*)&Vsl[(1 * HMAXA + row) * VLD + ko];
-              v8u16 al = *(const v8u16*)&Vsl[(2 * HMAXA + row) * VLD + ko];
-              // products ordered small to large
-              acc[pp][rb] = mfma_bf16(al, bh, acc[pp][rb]);
-              acc[pp][rb] = mfma_bf16(am, bm, acc[pp][rb]);
-              acc[pp][rb] = mfma_bf16(ah, bl, acc[pp][rb]);
-              acc[pp][rb] = mfma_bf16(am, bh, acc[pp][rb]);
-              acc[pp][rb] = mfma_bf16(ah, bm, acc[pp][rb]);
-              acc[pp][rb] = mfma_bf16(ah, bh, acc[pp][rb]);
-            }
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int pp = 0; pp < PPW; ++pp) {
-    const int pc = w + pp * NW;
-    if (pc >= npanel) continue;
-    const int col = pc * 16 + (lane & 15);
-    if (col >= b) continue;
-#pragma unroll
-    for (int rb = 0; rb < 8; ++rb) {
-      if (rb >= nrb) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = rb * 16 + ((MODE == 0) ? mfma16_row_f64(lane, r) : mfma16_row_f32(lane, r));
-        if (m >= a) continue;
-        if constexpr (TO_GLOBAL)
-          Ub[(long long)(I.p + 2 * m) * n + q + 2 * col] = (TIO)acc[pp][rb][r];
-        else
-          Wk[m * LDW + col] = (TS)acc[pp][rb][r];
-      }
-    }
-  }
-}
-
-// Multiplier storage of the row solves: FP32 LDS (mixed) or FP64 global scratch.
-template <int MODE>
-struct CPStore {
-  float* lds;
-  double* glob;
-  __device__ __forceinline__ void put(int j, int r, double v) const {
-    if constexpr (MODE == 1)
-      lds[j * HMAXA + r] = (float)v;
-    else
-      glob[(long long)j * HMAXA + r] = v;
-  }
-  __device__ __forceinline__ double get(int j, int r) const {
-    if constexpr (MODE == 1)
-      return (double)lds[j * HMAXA + r];
-    else
-      return glob[(long long)j * HMAXA + r];
-  }
-};
-
 // Rescale a continuant pair by the same power of two (exact).
 __device__ __forceinline__ void renorm(double& P1, double& P2) {
   const int e = ilogb(P1);
@@ -313,141 +129,345 @@ __device__ __forceinline__ void helm_gather(const TIO* __restrict__ Fb, int n, i
   }
 }
 
-template <int MODE, int NW, typename TIO>
-__global__ __launch_bounds__(NW * 64) void helm_ragged_kernel(
-    const HelmItem* __restrict__ items, int nitems, HelmQueues Q,
-    const double* __restrict__ Vd, const double* __restrict__ VTd,
-    const unsigned short* __restrict__ Vs, const unsigned short* __restrict__ VTs,
-    const double* __restrict__ lam, const TIO* __restrict__ F, TIO* __restrict__ U,
-    double* __restrict__ mult_scratch) {
-  typedef typename HelmTypes<MODE>::TS TS;
-  constexpr int LDW = HelmLDS<MODE>::LDW, NT = NW * 64;
+// FP64 kernel: one workgroup of 8 waves per CU walks the work queues.
+//   Wk : 128 x 129 FP64 work block (odd stride: the row solves read 32 rows at once)
+//   H  : h_{q+2j} = 2 / (2(q+2j) + 1), j = 0..b, and h_{q+2j} + h_{q+2j+2}
+// What bounds it: the FP64 products (129 us of matrix time for 1000 solves of
+// N = 32..256 at the card's 72 TFLOP/s) behind four dependent phases per block with
+// one workgroup per CU.  So: the products read the tables from L2 straight into
+// registers, two k-steps ahead (128-byte runs of the row-major tables), in tiles of 4
+// x 2 blocks per wave (2 x 1 up to 64 x 64) with no barriers inside; the row solves keep
+// their multipliers in registers; the next block of F is loaded while the second
+// product's results are stored.  With tables staged through LDS (two barriers per 16
+// rows), multipliers in global memory and F read between blocks: 632 us; now 475 us.  Of a 127 x 127 block's 55 us the products take 30 (27 at
+// the matrix units' rate), the row solves 6, stores and loads of half-used lines 12.
+struct Helm64 {
+  static constexpr int LDW = 129, NT = 512;
+  static constexpr size_t WK = (size_t)HMAXA * LDW * 8, HT = 2 * (HMAXA + 2) * 8, DUMMY = (HMAXA + 2) * 8;
+  static constexpr size_t BYTES = WK + HT + DUMMY;
+};
+
+// A wave's tiles of C = A Wk: TC column panels and TR row blocks.
+template <int TR, int TC>
+struct Tile64 {
+  int c0, rb0, nr, nc;
+  v4d acc[TC][TR];
+  __device__ __forceinline__ void init(int w, int a, int b) {
+    // panels over four groups as evenly as they go, rows over two
+    const int npanel = (b + 15) >> 4, nrb = (a + 15) >> 4, rh = (nrb + 1) >> 1;
+    const int rg = w >> 2, pg = w & 3, base = npanel >> 2, rem = npanel & 3;
+    c0 = pg * base + (pg < rem ? pg : rem);
+    nc = base + (pg < rem ? 1 : 0);
+    rb0 = rg * rh;
+    nr = nrb - rb0 < rh ? nrb - rb0 : rh;
+#pragma unroll
+    for (int c = 0; c < TC; ++c)
+#pragma unroll
+      for (int r = 0; r < TR; ++r) acc[c][r] = v4d{0, 0, 0, 0};
+  }
+  // T: (AP x AP) table whose row k holds column k of A; rows past a are zero in T and Wk
+  __device__ __forceinline__ void multiply(const double* __restrict__ T, int a, int AP, const double* Wk) {
+    if (nc <= 0 || nr <= 0) return;
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // addresses are not shared between the phases
+    const int kk = lane >> 4, cl = lane & 15, S = (a + 3) >> 2;
+    const double* at = T + kk * AP + 16 * rb0 + cl;
+    const double* bt = Wk + kk * Helm64::LDW + 16 * c0 + cl;
+    // two k-steps at a time, the next two steps' table entries on their way
+    double av[2][TR], an[2][TR];
+    auto ld = [&](int s, double(&v)[2][TR]) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < TR; ++r)
+          v[u][r] = at[4 * (s + u < S ? s + u : S - 1) * AP + 16 * (r < nr ? r : nr - 1)];
+    };
+    ld(0, av);
+    for (int s = 0; s < S; s += 2) {
+      ld(s + 2, an);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (s + u < S) {  // uniform
+          double bv[TC];
+#pragma unroll
+          for (int c = 0; c < TC; ++c) bv[c] = bt[4 * (s + u) * Helm64::LDW + 16 * (c < nc ? c : 0)];
+#pragma unroll
+          for (int r = 0; r < TR; ++r)
+            if (r < nr) {
+#pragma unroll
+              for (int c = 0; c < TC; ++c) acc[c][r] = mfma_f64(av[u][r], bv[c], acc[c][r]);
+            }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < TR; ++r) av[u][r] = an[u][r];
+    }
+  }
+  // f(row m, column, value) for the entries inside the a x b block
+  template <typename F>
+  __device__ __forceinline__ void each(int a, int b, F&& f) const {
+    if (nc <= 0 || nr <= 0) return;
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+#pragma unroll
+    for (int c = 0; c < TC; ++c) {
+      const int col = 16 * (c0 + c) + (lane & 15);
+      if (c < nc && col < b) {
+#pragma unroll
+        for (int r = 0; r < TR; ++r)
+          if (r < nr) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int m = 16 * (rb0 + r) + mfma16_row_f64(lane, e);
+              if (m < a) f(m, col, acc[c][r][e]);
+            }
+          }
+      }
+    }
+  }
+};
+
+// A block of F in flight in registers: rows w + 8 i, columns lane and lane + 64.
+struct Gather64 {
+  double v[16][2];
+  __device__ __forceinline__ void load(const double* __restrict__ F, int n, int p, int q, int a, int b) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, w = tid >> 6;
+    // clamped: every load is valid; a running 32-bit offset (< n^2) keeps one address
+    const int c0 = 2 * (lane < b ? lane : b - 1), d1 = 2 * (lane + 64 < b ? lane + 64 : b - 1) - c0;
+    int off = (p + 2 * (w < a ? w : a - 1)) * n + q + c0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      v[i][0] = F[off];
+      v[i][1] = F[off + d1];
+      off += w + 8 * (i + 1) < a ? 16 * n : 0;
+      asm volatile("" : "+v"(off));
+    }
+  }
+  __device__ __forceinline__ void store(double* Wk, int a, int b) const {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, w = tid >> 6;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = w + 8 * i;
+      if (r < a) {
+        if (lane < b) Wk[r * Helm64::LDW + lane] = v[i][0];
+        if (lane + 64 < b) Wk[r * Helm64::LDW + lane + 64] = v[i][1];
+      }
+    }
+  }
+};
+
+// Row r of G: T u = g, T = s M_q + diag(4c + 6), c = q + 2j, s = alpha - lambda_r:
+// d_j = s Hs_j + 4c + 6, T[j][j+1] = -s H_{j+1}.  Twisted elimination by two lanes,
+// (r, 0) downwards and (r, 1) upwards over len = b / 2 rows each; pivots are ratios
+// of continuants P_j = d_j P_{j-1} - o_{j-1}^2 P_{j-2}, whose serial dependence is
+// one FMA a step, reciprocals off that chain; the halves meet in the middle row (odd
+// b) or in a 2 x 2 system (even b).  FP64 throughout, multipliers in registers.
+__device__ __forceinline__ void helm64_rows(const HelmItem& I, int q, int b, const double* __restrict__ lam, double* Wk,
+                                            const double* H, const double* Hs, double* dummy) {
+  int t2 = threadIdx.x;
+  asm volatile("" : "+v"(t2));
+  const int r = t2 >> 1, side = t2 & 1;
+  const bool act = r < I.a;
+  const double s = act ? I.alpha - lam[I.loff + r] : 1.0;
+  const int rb = act ? r * Helm64::LDW : (int)(dummy - Wk);  // idle lanes leave the zero rows alone
+  const int len = b >> 1;
+  const int j0 = side ? b - 1 : 0, dj = side ? -1 : 1;
+  const int ho_off = side ? 0 : 1;  // coupling towards the middle = -s H[j + ho_off]
+  const double dg0 = fma(8.0, (double)j0, 4.0 * q + 6.0), ddg = 8.0 * dj;
+  double cm[64];
+  double P1 = 1.0, P2 = 0.0, yprev = 0.0, oprev = 0.0, cl = 0.0;
+  // first index of a chunk of 8 steps, opaque: the row's 64 addresses are not kept
+  // in registers from the elimination to the back substitution
+  auto chunk = [&](int ch) {
+    int j = j0 + dj * 8 * ch;
+    asm volatile("" : "+v"(j));
+    return j;
+  };
+  auto fwd_v = [&](int i, int j, double g, double hs, double ho) {
+    const double d = fma(s, hs, fma((double)i, ddg, dg0));
+    const double on = -s * ho;
+    const double Pj = fma(d, P1, -(oprev * oprev) * P2);
+    const double rj = P1 * rcp64(Pj);
+    const double yj = fma(-oprev, yprev, g) * rj;
+    cl = on * rj;
+    cm[i] = cl;
+    Wk[rb + j] = yj;
+    P2 = P1;
+    P1 = Pj;
+    yprev = yj;
+    oprev = on;
+  };
+#pragma unroll
+  for (int ch = 0; ch < 8; ++ch) {
+    if (ch * 8 + 8 <= len) {
+      // half a chunk's loads issue before its arithmetic
+      const int jc = chunk(ch);
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        double g[4], hs[4], ho[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int j = jc + dj * (4 * hh + u);
+          g[u] = Wk[rb + j];
+          hs[u] = Hs[j];
+          ho[u] = H[j + ho_off];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) fwd_v(ch * 8 + 4 * hh + u, jc + dj * (4 * hh + u), g[u], hs[u], ho[u]);
+      }
+      renorm(P1, P2);
+    } else if (ch * 8 < len) {
+      const int jc = chunk(ch);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (ch * 8 + u < len) {
+          const int j = jc + dj * u;
+          fwd_v(ch * 8 + u, j, Wk[rb + j], Hs[j], H[j + ho_off]);
+        }
+    }
+  }
+  const double co = __shfl_xor(cl, 1), yo = __shfl_xor(yprev, 1);  // the partner's last step
+  const double ct = side == 0 ? cl : co, yt = side == 0 ? yprev : yo;  // rows above the middle
+  const double cb = side == 0 ? co : cl, yb = side == 0 ? yo : yprev;  // rows below
+  double own;
+  int start;
+  if (b & 1) {
+    const int m = len;
+    const double am = (m > 0) ? -s * H[m] : 0.0;
+    const double cmm = (m < b - 1) ? -s * H[m + 1] : 0.0;
+    const double dm = fma(s, Hs[m], fma(8.0, (double)m, 4.0 * q + 6.0));
+    own = (Wk[rb + m] - am * yt - cmm * yb) / (dm - am * ct - cmm * cb);
+    start = len - 1;
+    if (side == 0) Wk[rb + m] = own;  // both lanes have read it above
+  } else {
+    const double ut = (yt - ct * yb) / (1.0 - ct * cb);  // u_t = y_t - c_t u_b, u_b = y_b - c_b u_t
+    own = side == 0 ? ut : yb - cb * ut;
+    start = len - 2;
+    Wk[rb + j0 + dj * (len - 1)] = own;
+  }
+  // back substitution outwards, i = start .. 0
+  double uprev = own;
+  auto bwd = [&](int i, int j, double y) {
+    const double v = fma(-cm[i], uprev, y);
+    Wk[rb + j] = v;
+    uprev = v;
+  };
+#pragma unroll
+  for (int ch = 7; ch >= 0; --ch) {
+    if (ch * 8 + 7 <= start) {
+      const int jc = chunk(ch);
+      double y[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) y[u] = Wk[rb + jc + dj * u];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 7; u >= 0; --u) bwd(ch * 8 + u, jc + dj * u, y[u]);
+    } else if (ch * 8 <= start) {
+      const int jc = chunk(ch);
+#pragma unroll
+      for (int u = 7; u >= 0; --u)
+        if (ch * 8 + u <= start) bwd(ch * 8 + u, jc + dj * u, Wk[rb + jc + dj * u]);
+    }
+  }
+}
+
+// One column parity q of work item I; F_pq is in Wk.  The next block (In, qn) is
+// loaded around the stores of this one and left in Wk.
+template <int TR, int TC>
+__device__ __forceinline__ void helm64_pass(const HelmItem& I, int q, const HelmItem& In, int qn, bool has_next,
+                                            const double* __restrict__ Vd, const double* __restrict__ VTd,
+                                            const double* __restrict__ lam, const double* __restrict__ F,
+                                            double* __restrict__ U, double* Wk, double* H, double* dummy) {
+  constexpr int LDW = Helm64::LDW, NT = Helm64::NT;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int a = I.a, AP = I.AP, b = (I.n - q + 1) >> 1;
+  double* Hs = H + HMAXA + 2;
+  for (int e = tid; e < (((a + 3) & ~3) - a) * 128; e += NT) Wk[(a + (e >> 7)) * LDW + (e & 127)] = 0.0;
+  for (int j = tid; j <= b; j += NT) {
+    const double hj = 2.0 / (2 * (q + 2 * j) + 1);
+    H[j] = hj;
+    Hs[j] = hj + 2.0 / (2 * (q + 2 * j) + 5);
+  }
+  __syncthreads();
+  Tile64<TR, TC> t;
+  t.init(w, a, b);
+  t.multiply(Vd + I.voff, a, AP, Wk);  // G = V_p^T F_pq: row k of V_p is column k of V_p^T
+  __syncthreads();
+  t.each(a, b, [&](int m, int c, double v) { Wk[m * LDW + c] = v; });
+  __syncthreads();
+  if (w * 32 < a) helm64_rows(I, q, b, lam, Wk, H, Hs, dummy);
+  __syncthreads();
+  t.init(w, a, b);
+  t.multiply(VTd + I.voff, a, AP, Wk);
+  Gather64 G;
+  const int bn = (In.n - qn + 1) >> 1;
+  if (has_next) G.load(F + In.foff, In.n, In.p, qn, In.a, bn);
+  double* Ub = U + I.foff + q;
+  t.each(a, b, [&](int m, int c, double v) { Ub[(I.p + 2 * m) * I.n + 2 * c] = v; });
+  __syncthreads();  // Wk is free
+  if (has_next) G.store(Wk, In.a, bn);
+}
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void helm64_kernel(
+    const HelmItem* __restrict__ items, int nitems, HelmQueues Q, const double* __restrict__ Vd,
+    const double* __restrict__ VTd, const double* __restrict__ lam, const double* __restrict__ F,
+    double* __restrict__ U) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  TS* Wk = reinterpret_cast<TS*>(smem_raw);
-  unsigned char* u1 = smem_raw + HelmLDS<MODE>::WK;
-  double* Hs = reinterpret_cast<double*>(smem_raw + HelmLDS<MODE>::WK + HelmLDS<MODE>::U1);  // h_c + h_{c+2}
-  double* H2 = Hs + HMAXA;                                                                 // h_{c+2}
-  double* Dg = H2 + HMAXA;                                                                 // 4c + 6
+  double* Wk = reinterpret_cast<double*>(smem_raw);
+  double* H = reinterpret_cast<double*>(smem_raw + Helm64::WK);
+  double* dummy = reinterpret_cast<double*>(smem_raw + Helm64::WK + Helm64::HT);
   __shared__ int s_nx[2];
   const int tid = threadIdx.x;
-  CPStore<MODE> cps{reinterpret_cast<float*>(u1), mult_scratch + (long long)blockIdx.x * HMAXA * HMAXA};
-
-  // the next item's index is claimed at the start of the current one, so the
-  // counter round trip overlaps the work (two slots: slot k is rewritten only
-  // after every thread has passed the barriers of the item in between)
   int qi = blockIdx.x % Q.nq;
   if (tid < 64) {
     const int first = Q.claim(qi);
     if (tid == 0) s_nx[0] = first;
   }
   __syncthreads();
-  int it = s_nx[0], slot = 1;
-  while (it < nitems) {
-    const HelmItem I = items[it];
+  const int it0 = __builtin_amdgcn_readfirstlane(s_nx[0]);
+  if (it0 >= nitems) return;
+  HelmItem I = items[it0];
+  {
+    Gather64 G;
+    const int b = (I.n + 1) >> 1;
+    G.load(F + I.foff, I.n, I.p, 0, I.a, b);
+    G.store(Wk, I.a, b);
+  }
+  int slot = 1;
+  for (;;) {
+    // the next item is claimed now; its index is published after this item's
+    // first pass (two slots: slot k is rewritten only after every thread has
+    // passed the barriers of the passes in between)
     int nxt = 0;
     if (tid < 64) nxt = Q.claim(qi);
-    const int n = I.n, p = I.p, a = I.a;
-    const TIO* Fb = F + I.foff;
-
-    // both column parities of this (solve, row parity) in turn: the second
-    // pass re-reads / re-writes the other half of the same lines from L2
-    for (int q = 0; q < 2; ++q) {
-      const int b = (n - q + 1) >> 1;
-      if (b == 0) continue;
-      // ---------------- phase 0: F_pq -> Wk, column constants
-      helm_gather<NW, LDW>(Fb, n, p, q, a, b, Wk);
-      for (int j = tid; j < b; j += NT) {
-        const int c = q + 2 * j;
-        const double hc = 2.0 / (2 * c + 1), hc2 = 2.0 / (2 * c + 5);
-        Hs[j] = hc + hc2;
-        H2[j] = hc2;
-        Dg[j] = 4.0 * c + 6.0;
-      }
-      __syncthreads();
-
-      // ---------------- phase 1: G = V_p^T F_pq (in place, column-owned)
-      helm_gemm_phase<MODE, NW, TIO, false>(I, q, b, Vd, VTs, Wk, u1, nullptr);
-      __syncthreads();
-
-      // ---------------- phase 2: FP64 tridiagonal solves, two lanes per row
-      // row r: T u = g, T = s M_q + diag(4c + 6), s = alpha - lambda_r, c = q + 2j:
-      //   d_j = T[j][j] = s (h_c + h_{c+2}) + 4c + 6,  o_j = T[j][j+1] = T[j+1][j] = -s h_{c+2}
-      // Twisted elimination: lane (r, 0) sweeps rows 0..m-1 down, lane (r, 1)
-      // rows b-1..m+1 up, m = b / 2.  The pivots are ratios of continuants
-      // P_j = d_j P_{j-1} - o_{j-1}^2 P_{j-2}  (P_{-1} = 1), so the serial
-      // dependence per step is one FMA; reciprocals run off that chain.
-      for (int t = tid; t < 2 * HMAXA; t += NT) {
-        const int r = t >> 1, side = t & 1;
-        const bool act = r < a;
-        const double s = act ? I.alpha - lam[I.loff + r] : 1.0;
-        TS* row = Wk + (act ? r : 0) * LDW;
-        const int m = b >> 1;
-        // both lanes of a pair run the same instruction stream; `side` only
-        // selects the direction: step i visits j = i (down) or j = b-1-i (up)
-        const int len = act ? (side ? b - 1 - m : m) : 0;
-        const int maxlen = b - m - 1 > m ? b - m - 1 : m;
-        double P1 = 1.0, P2 = 0.0, yprev = 0.0, oprev = 0.0, cl = 0.0;
-        for (int i = 0; i < maxlen; ++i) {
-          if (i < len) {
-            const int j = side ? b - 1 - i : i;
-            const int inext = side ? j - 1 : j;  // coupling towards the middle
-            const double on = -s * H2[inext];
-            const double Pj = fma(fma(s, Hs[j], Dg[j]), P1, -(oprev * oprev) * P2);
-            const double rj = P1 * rcp64(Pj);
-            const double yj = fma(-oprev, yprev, (double)row[j]) * rj;
-            cl = on * rj;
-            cps.put(j, r, cl);
-            row[j] = (TS)yj;
-            P2 = P1;
-            P1 = Pj;
-            yprev = yj;
-            oprev = on;
-            if ((i & 7) == 7) renorm(P1, P2);
-          }
-        }
-        const double dl = yprev;
-        // exchange with the partner lane (adjacent lane of the same wave)
-        const double co = __shfl_xor(cl, 1), dO = __shfl_xor(dl, 1);
-        if (act) {
-          const double ct = side == 0 ? cl : co, dt = side == 0 ? dl : dO;  // rows < m
-          const double fb = side == 0 ? co : cl, eb = side == 0 ? dO : dl;  // rows > m
-          const double am = (m > 0) ? -s * H2[m - 1] : 0.0;
-          const double cm = (m < b - 1) ? -s * H2[m] : 0.0;
-          const double um = ((double)row[m] - am * dt - cm * eb) / (fma(s, Hs[m], Dg[m]) - am * ct - cm * fb);
-          // back substitution outwards from m: j = m-1-i (down) or m+1+i (up)
-          double uprev = um;
-          int i = 0;
-          for (; i + 8 <= len; i += 8) {
-            double c8[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) c8[u] = cps.get(side ? m + 1 + i + u : m - 1 - i - u, r);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-              const int j = side ? m + 1 + i + u : m - 1 - i - u;
-              const double v = (double)row[j] - c8[u] * uprev;
-              row[j] = (TS)v;
-              uprev = v;
-            }
-          }
-          for (; i < len; ++i) {
-            const int j = side ? m + 1 + i : m - 1 - i;
-            const double v = (double)row[j] - cps.get(j, r) * uprev;
-            row[j] = (TS)v;
-            uprev = v;
-          }
-          if (side == 0) row[m] = (TS)um;
-        }
-      }
-      __syncthreads();
-
-      // ---------------- phase 3: U_pq = V_p U~ -> global
-      helm_gemm_phase<MODE, NW, TIO, true>(I, q, b, VTd, Vs, Wk, u1, U + I.foff);
-      __syncthreads();
+    const bool two = I.n > 1;  // n = 1 has one column parity
+    const bool small = I.n <= 128;
+    if (two) {
+      if (small)
+        helm64_pass<2, 1>(I, 0, I, 1, true, Vd, VTd, lam, F, U, Wk, H, dummy);
+      else
+        helm64_pass<4, 2>(I, 0, I, 1, true, Vd, VTd, lam, F, U, Wk, H, dummy);
     }
     if (tid == 0) s_nx[slot] = nxt;
     __syncthreads();
-    it = s_nx[slot];
+    const int itn = __builtin_amdgcn_readfirstlane(s_nx[slot]);
     slot ^= 1;
+    const bool has = itn < nitems;
+    const HelmItem In = items[has ? itn : it0];
+    if (small)
+      helm64_pass<2, 1>(I, two ? 1 : 0, In, 0, has, Vd, VTd, lam, F, U, Wk, H, dummy);
+    else
+      helm64_pass<4, 2>(I, 1, In, 0, has, Vd, VTd, lam, F, U, Wk, H, dummy);
+    if (!has) break;
+    I = In;
+    __syncthreads();
   }
 }
 
@@ -1484,18 +1504,13 @@ static int launch_helm_compact(const HelmItem* items, int nitems, HelmQueues Q, 
   return JFX_OK;
 }
 
-template <int MODE, int NW, typename TIO>
-static int launch_helm(const HelmItem* items, int nitems, HelmQueues Q, const double* Vd,
-                       const double* VTd, const unsigned short* Vs, const unsigned short* VTs,
-                       const double* lam, const TIO* F, TIO* U, double* mult_scratch, int nblocks,
-                       hipStream_t st) {
-  size_t shm = HelmLDS<MODE>::WK + HelmLDS<MODE>::U1 + HTAB;
-  auto kern = helm_ragged_kernel<MODE, NW, TIO>;
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+static int launch_helm64(const HelmItem* items, int nitems, HelmQueues Q, const double* Vd, const double* VTd,
+                         const double* lam, const double* F, double* U, int nblocks, hipStream_t st) {
+  hipError_t e = hipFuncSetAttribute((const void*)helm64_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)Helm64::BYTES);
   if (e != hipSuccess) return set_error("helm: hipFuncSetAttribute: %s", hipGetErrorString(e)), JFX_EHIP;
   hipLaunchKernelGGL(helm_reset, dim3(1), dim3(64), 0, st, Q.counters, Q.nq);
-  hipLaunchKernelGGL(kern, dim3(nblocks), dim3(NW * 64), shm, st, items, nitems, Q, Vd, VTd, Vs, VTs,
-                     lam, F, U, mult_scratch);
+  hipLaunchKernelGGL(helm64_kernel, dim3(nblocks), dim3(512), Helm64::BYTES, st, items, nitems, Q, Vd, VTd, lam, F, U);
   JFX_LAUNCH_CHECK();
   return JFX_OK;
 }
@@ -1579,7 +1594,7 @@ int jfx_helm_scratch_doubles_per_block(void) { return HMAXA * HMAXA; }
 // mode 2: FP16 2-term split (tables V 2^eA in two fp16 slices, eA in the
 //         item's pad field; blocks scaled by a power of two), nwaves 4
 // nwaves: 4 or 8 waves per workgroup; nblocks: persistent grid size
-//   (mult_scratch must hold nblocks * jfx_helm_scratch_doubles_per_block() doubles).
+//   (mult_scratch is not used; it must not be null).
 int jfx_helm_ragged(int mode, int io_f32, int nwaves, const void* items, int nitems, int* counters,
                     const int* qbounds, int nqueues, const double* Vd, const double* VTd, const unsigned short* Vs,
                     const unsigned short* VTs, const double* lam, const void* F, void* U,
@@ -1592,12 +1607,9 @@ int jfx_helm_ragged(int mode, int io_f32, int nwaves, const void* items, int nit
   const HelmQueues queues{counters, qbounds, nqueues};
   if (mode == 0) {
     if (!Vd || !VTd || io_f32) return set_error("helm_ragged: mode 0 needs fp64 tables and fp64 I/O"), JFX_EARG;
-    if (nwaves == 4)
-      return launch_helm<0, 4, double>(it, nitems, queues, Vd, VTd, Vs, VTs, lam, (const double*)F,
-                                       (double*)U, mult_scratch, nblocks, stream);
-    if (nwaves == 8)
-      return launch_helm<0, 8, double>(it, nitems, queues, Vd, VTd, Vs, VTs, lam, (const double*)F,
-                                       (double*)U, mult_scratch, nblocks, stream);
+    // one kernel of 8 waves whatever nwaves (4 or 8) says
+    if (nwaves == 4 || nwaves == 8)
+      return launch_helm64(it, nitems, queues, Vd, VTd, lam, (const double*)F, (double*)U, nblocks, stream);
   } else if (mode == 1) {
     if (!Vs || !VTs) return set_error("helm_ragged: mode 1 needs bf16 slice tables"), JFX_EARG;
     if (io_f32) {

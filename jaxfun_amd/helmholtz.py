@@ -72,7 +72,7 @@ class HelmholtzBatch:
         nwaves, blocks_per_cu: launch shape (see :func:`autotune`); in mixed mode
             nwaves 4 runs one column parity at a time (two workgroups fit a CU),
             nwaves 8 both at once with whole-row reads of F and writes of U
-            (one workgroup per CU).
+            (one workgroup per CU); fp64 mode runs one 8-wave kernel for both.
         queues: number of work queues (1..16); items sharing tables share a queue.
     """
 
@@ -388,10 +388,10 @@ def autotune(batch: HelmholtzBatch, F: torch.Tensor, candidates=None, reps: int 
     the shapes are the two kernels at their occupancy: (4, 2) two 4-wave
     workgroups per CU (one column parity at a time) and (8, 1) one 8-wave
     workgroup per CU (both column parities at once), plus (4, 1); mixed16
-    has the 4-wave kernel only."""
+    has the 4-wave kernel only and fp64 one 8-wave kernel."""
     if candidates is None:
         candidates = {"mixed": ((4, 2), (8, 1), (4, 1)), "mixed16": ((4, 2), (4, 1))}.get(
-            batch.mode, ((4, 1), (8, 1), (4, 2), (8, 2)))
+            batch.mode, ((8, 1), (8, 2)))
     U = torch.empty_like(F)
     best, best_t = None, float("inf")
     for nw, bpc in candidates:

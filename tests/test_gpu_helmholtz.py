@@ -218,3 +218,27 @@ def test_mixed16_launch_shapes_and_graph(dev):
         torch.cuda.synchronize()
         assert np.array_equal(U.cpu().numpy(), a)
         hb.solve(F)
+
+
+@pytest.mark.parametrize("Ns", [list(range(4, 13)), [33, 34, 35, 36, 64, 65, 66, 67], [128, 129, 130, 131, 132],
+                                [160, 161, 192, 193, 226, 255, 256, 257, 258]])
+def test_fp64_block_edges(dev, Ns):
+    """FP64 batches whose blocks sit at the edges of the 16-row blocks, of the small
+    and large tiles (n = 128) and of the largest size: residuals and both parities of
+    the size, several items per workgroup and none left over."""
+    import torch
+
+    from jaxfun_amd.helmholtz import HelmholtzBatch, legendre_dirichlet_pair
+
+    rng = np.random.default_rng(Ns[0])
+    alphas = 10.0 ** rng.uniform(-2, 4, len(Ns))
+    F = [rng.standard_normal((N - 2, N - 2)) / np.outer(1.0 + np.arange(N - 2), 1.0 + np.arange(N - 2))**2 for N in Ns]
+    for nwaves, bpc in ((4, 1), (8, 2)):
+        hb = HelmholtzBatch(Ns, alphas, mode="fp64", nwaves=nwaves, blocks_per_cu=bpc)
+        U = hb.unpack(hb.solve(hb.pack(F)))
+        for N, al, f, u in zip(Ns, alphas, F, U):
+            M, K = legendre_dirichlet_pair(N - 2)
+            r = al * M @ u @ M - K @ u @ M - M @ u @ K - f
+            # backward error of a stable solve: a few eps times the operator's norm, the size and |u|
+            scale = (al * np.linalg.norm(M, 2)**2 + 2 * np.linalg.norm(K, 2) * np.linalg.norm(M, 2)) * np.linalg.norm(u)
+            assert np.linalg.norm(r) <= 2.0**-52 * 20 * N * (scale + np.linalg.norm(f)), N
