@@ -139,8 +139,9 @@ __device__ __forceinline__ void helm_gather(const TIO* __restrict__ Fb, int n, i
 // x 2 blocks per wave (2 x 1 up to 64 x 64) with no barriers inside; the row solves keep
 // their multipliers in registers; the next block of F is loaded while the second
 // product's results are stored.  With tables staged through LDS (two barriers per 16
-// rows), multipliers in global memory and F read between blocks: 632 us; now 475 us.  Of a 127 x 127 block's 55 us the products take 30 (27 at
-// the matrix units' rate), the row solves 6, stores and loads of half-used lines 12.
+// rows), multipliers in global memory and F read between blocks: 632 us; now 475 us.
+// In a 127 x 127 block (one k-step ahead, cycles): products 2 x 46 k (33 k at the
+// matrix units' rate), row solves 15 k, loads of F 7 k, stores to half-used lines 24 k.
 struct Helm64 {
   static constexpr int LDW = 129, NT = 512;
   static constexpr size_t WK = (size_t)HMAXA * LDW * 8, HT = 2 * (HMAXA + 2) * 8, DUMMY = (HMAXA + 2) * 8;

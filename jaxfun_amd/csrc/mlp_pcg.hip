@@ -237,7 +237,7 @@ __device__ __forceinline__ double block_sum(double s, double* red) {
 // One PCG iteration's vector work, one workgroup per system: five launches
 // (two reductions, the update, the test, the count of systems left) in one, the
 // vectors read once from HBM and the second time from L2.  256 systems of 3844
-// values: 7.3 + 6.3 + 7.3 + 2.0 us and a 3-kernel count before, 10 us now.
+// values: 7.3 + 6.3 + 7.3 + 2.0 us and a 3-kernel count before, 9 us now.
 constexpr int PCG_W = 8;
 // One active system; returns (thread 0) whether it goes on.
 __device__ __forceinline__ int pcg_step_system(double* __restrict__ x, double* __restrict__ r,

@@ -10,7 +10,7 @@
 // halves (par_blocks.h).  U is staged again for the second half (from L2), so
 // that one LDS buffer serves every pass: 37 KB at 64 x 64, four workgroups per
 // CU.  256 slabs of 62 x 62 on a 64 x 64 mesh: 8 contractions, 2 products and a
-// sum in separate launches 115 us, here 33 us; the FP64 products alone take 8 us,
+// sum in separate launches 115 us, here 30 us; the FP64 products alone take 7 us,
 // so latency bounds it (eight phases with barriers between them per slab).
 #include "par_blocks.h"
 

@@ -158,7 +158,11 @@ class IMEXRungeKutta:
                     all(o in self._QUAD_FIELDS for _, o1, o2 in self.nonlinear for o in (o1, o2)):
                 ops = [T[ax].backward_operator(self.Np[ax], k) for ax in (0, 1) for k in (0, 1)]
                 ops += [T[ax].scalar_product_operator(self.Np[ax]) for ax in (0, 1)]
-            self._stage_ops["quad"] = ops if ops is not None and K.quad_ok(*ops) else None
+            if ops is not None and not K.quad_ok(*ops):
+                if torch.cuda.is_current_stream_capturing():
+                    return None  # unprepared operators: the next use decides
+                ops = None
+            self._stage_ops["quad"] = ops
         return self._stage_ops["quad"]
 
     def _quad_pays(self, nbatch: int) -> bool:

@@ -496,8 +496,10 @@ class AxisOperator:
             return None
         f = torch.empty(n, dtype=io_dtype(prec), device=self.A64.device)
         _lib.call("jfx_par_prepare", 0 if prec == "f64" else 1, _p(self.A64), self.M, self.K, mode, sgn, _p(f), _s())
-        self._prep[key] = (f, mode, sgn, p, q)
-        return self._prep[key]
+        # complete before they are published: the next use may be on another stream
+        torch.cuda.current_stream().synchronize()
+        fr = self._prep[key] = (f, mode, sgn, p, q)
+        return fr
 
     def _padded(self):
         """Zero-pad K to a multiple of 32 (the slice row stride the kernels read)."""

@@ -147,3 +147,27 @@ def test_first_use_inside_a_capture(dev):
         assert np.abs(y.cpu().numpy() - ref).max() < 1e-12 * np.abs(ref).max()
         eager = K.apply_along(op, x, 0).cpu().numpy()
         assert np.abs(eager - ref).max() < 1e-12 * np.abs(ref).max()
+
+
+def test_prepared_on_another_stream():
+    """An operator first used on a busy stream is ready for one that does not wait for it."""
+    import torch
+
+    from jaxfun_amd import kernels as K
+
+    rng = np.random.default_rng(5)
+    A = _structured(rng, 96, 64, 1, 1)
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    big = torch.ones((4096, 4096), device="cuda")
+    x = torch.tensor(rng.standard_normal((7, 64)), device="cuda")
+    op = K.AxisOperator(torch.tensor(A, device="cuda"), (1, 1, -1, -1))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        for _ in range(20):
+            big = big @ big * 2.0**-12
+        K.apply_along(op, x, 1, "f64")
+    with torch.cuda.stream(other):
+        y = K.apply_along(op, x, 1, "f64")
+    torch.cuda.synchronize()
+    bound = np.abs(x.cpu().numpy()) @ np.abs(A).T
+    assert np.all(np.abs(y.cpu().numpy() - x.cpu().numpy() @ A.T) <= 68 * EPS["f64"] * bound)
