@@ -237,7 +237,7 @@ __device__ __forceinline__ double block_sum(double s, double* red) {
 // One PCG iteration's vector work, one workgroup per system: five launches
 // (two reductions, the update, the test, the count of systems left) in one, the
 // vectors read once from HBM and the second time from L2.  256 systems of 3844
-// values: 7.3 + 6.3 + 7.3 + 2.0 us and a 3-kernel count before, 9 us now.
+// values: 7.3 + 6.3 + 7.3 + 2.0 us and a 3-kernel count before, 10 us now.
 constexpr int PCG_W = 8;
 // One active system; returns (thread 0) whether it goes on.
 __device__ __forceinline__ int pcg_step_system(double* __restrict__ x, double* __restrict__ r,
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(64 * PCG_W) void pcg_step_kernel(double* __restrict
                                red, n);
   // *left: workgroups that are done (high half) and systems that go on (low
   // half) in one atomic, so that the last workgroup knows the count without a
-  // fence (13 us with one, 9 us without)
+  // fence (13 us with one, 10 us without)
   if (threadIdx.x == 0) {
     const unsigned old = atomicAdd(left, 0x10000u | (unsigned)on);
     if (host_left && (old >> 16) == gridDim.x - 1)
