@@ -546,10 +546,9 @@ def _refine_eig(A: np.ndarray, B: np.ndarray, lam: np.ndarray, V: np.ndarray, W:
     R = _extended_product(A, Ve) - _extended_product(B, Ve) * lam.astype(np.longdouble)
     P = W @ R.astype(np.float64)
     gap = lam[None, :] - lam[:, None]
-    with np.errstate(divide="ignore", invalid="ignore"):
-        # pairs too close for a first-order correction keep their vectors
-        Q = np.where(np.abs(P) <= 1e-3 * np.abs(gap), P / gap, 0.0)
-    np.fill_diagonal(Q, 0.0)
+    # pairs too close for a first-order correction, equal eigenvalues among them,
+    # keep their vectors
+    Q = np.divide(P, gap, out=np.zeros_like(P), where=(gap != 0) & (np.abs(P) <= 1e-3 * np.abs(gap)))
     Ve = Ve + V @ Q
     V = Ve.astype(np.float64)
     W = np.linalg.inv(B @ V)

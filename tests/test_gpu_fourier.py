@@ -320,6 +320,35 @@ def test_fourier_poly_advection_diffusion(dev, poly):
     assert np.abs(uj - sp.lambdify((x, y), ue)(*xj)).max() < 1e-12
 
 
+@pytest.mark.parametrize("poly", ["legendre", "chebyshev"])
+def test_fourier_fast_diagonalisation(dev, poly):
+    # Fourier axes have pairs of equal eigenvalues (+-k): the fast-diagonalisation
+    # solve of 3D and 2D problems against the Kronecker matrix
+    from jaxfun_amd import Chebyshev, Div, Fourier, FunctionSpace, Grad, Legendre, TensorProduct, TestFunction, \
+        TrialFunction, inner
+    from jaxfun_amd.la import TPMatricesLUFactors, tpmats_to_kron
+
+    space = Legendre if poly == "legendre" else Chebyshev
+
+    def D(N):
+        return FunctionSpace(N, space, {"left": {"D": 0}, "right": {"D": 0}})
+
+    rng = np.random.default_rng(11)
+    for spaces in ((Fourier(20), D(9), D(8)), (Fourier(20), D(12)), (Fourier(8), Fourier(10))):
+        T = TensorProduct(*spaces)
+        v, u = TestFunction(T), TrialFunction(T)
+        A = inner(v * (u - Div(Grad(u))), sparse=True)
+        if len(spaces) == 3:
+            assert isinstance(A.lu_factor(), TPMatricesLUFactors)
+        shape = tuple(int(m.shape[0]) for m in A.tpmats[0].mats)
+        b = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+        M = tpmats_to_kron(A.tpmats)
+        ref = np.linalg.solve(M, b.ravel()).reshape(shape)
+        for f in (A.lu_factor(), A.fd_factor()):
+            err = np.abs(_np(f.solve(b)) - ref).max() / np.abs(ref).max()
+            assert err < 4 * np.linalg.cond(M) * np.finfo(float).eps, (poly, shape, err)
+
+
 def test_poisson1d_periodic_example(dev):
     # examples/poisson1D_periodic.py: complex manufactured solution, the k = 0
     # mode pinned

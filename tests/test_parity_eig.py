@@ -51,6 +51,35 @@ def test_parity_blocks(family, N):
     assert err <= 1.2 * whole + 4e-16  # no further off than the pair diagonalised as a whole
 
 
+def _degenerate_pairs():
+    n, rng = 12, np.random.default_rng(3)
+    k2 = np.fft.fftfreq(20, 1.0 / 20)**2
+    M, K = _pair("legendre", 16)
+    close = np.diag(np.repeat(np.arange(1.0, n // 4 + 1), 4)) + 1e-13 * np.diag(rng.standard_normal(n))
+    return {"identity": (np.eye(n), np.eye(n)),
+            "chebyshev mass": (np.diag(np.where(np.arange(n) == 0, np.pi, np.pi / 2)), np.eye(n)),
+            "fourier": (2 * np.pi * np.diag(k2), 2 * np.pi * np.eye(20)),
+            "fourier mass": (2 * np.pi * np.eye(20), np.eye(20)),
+            "mass against itself": (M, M),
+            "multiples on blocks": (np.kron(np.eye(2), K), np.kron(np.eye(2), M)),
+            "nearly equal": (close, np.eye(n))}
+
+
+@pytest.mark.parametrize("name", list(_degenerate_pairs()))
+def test_repeated_eigenvalues(name):
+    """Pairs with equal and nearly equal eigenvalues within one parity: finite
+    vectors that diagonalise the pair, to the rounding of n-term FP64 sums."""
+    A, B = _degenerate_pairs()[name]
+    lam, V, W = T.axis_eig(A, B)
+    assert np.isfinite(lam).all() and np.isfinite(V).all() and np.isfinite(W).all()
+    tol = 8 * len(lam) * np.finfo(float).eps
+    cond = np.linalg.norm(W) * np.linalg.norm(B @ V)
+    assert np.linalg.norm(W @ B @ V - np.eye(len(lam))) <= tol * cond
+    assert np.linalg.norm(W @ A @ V - np.diag(lam)) <= tol * cond * np.abs(lam).max()
+    ref = np.sort(T._axis_eig(A, B)[0])
+    np.testing.assert_allclose(lam, ref, rtol=tol * np.linalg.cond(B), atol=tol * np.abs(ref).max())
+
+
 def test_pairs_without_parity_are_left_whole():
     rng = np.random.default_rng(0)
     A = rng.standard_normal((7, 7))
