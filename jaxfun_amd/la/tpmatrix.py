@@ -211,8 +211,9 @@ class TPMatricesLUFactors:
             D = D + float(s) * t
         self.D_host = D
         self._D = {}
-        self.eigvecs_host = [np.asarray(v) for v in eigvecs]
-        self.lefts_host = [np.asarray(w) for w in lefts]
+        # in the order of D_host and of the operators
+        self.eigvecs_host = [np.asarray(v) if o is None else np.asarray(v)[:, o] for v, o in zip(eigvecs, orders)]
+        self.lefts_host = [np.asarray(w) if o is None else np.asarray(w)[o] for w, o in zip(lefts, orders)]
 
     def D(self, dtype) -> torch.Tensor:
         if dtype not in self._D:

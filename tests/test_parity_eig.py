@@ -4,6 +4,7 @@ extended precision."""
 
 import numpy as np
 import pytest
+import torch
 
 from jaxfun_amd.la import tpmatrix as T
 
@@ -88,3 +89,19 @@ def test_pairs_without_parity_are_left_whole():
     ref = T._axis_eig(A, np.eye(7))
     assert all(np.array_equal(a, b) for a, b in zip((lam, V, W), ref))
     assert T._parity_order(V, W) is None
+
+
+@pytest.mark.parametrize("family", ["legendre", "chebyshev"])
+def test_host_factors_follow_one_order(family, monkeypatch):
+    """eigvecs_host, lefts_host and D_host together solve the problem, as the
+    operators built from them do."""
+    monkeypatch.setattr(T.K, "device", lambda: torch.device("cpu"))
+    monkeypatch.setattr(T.K.AxisOperator, "fragments", lambda self, prec: None)
+    (M0, K0), (M1, K1) = _pair(family, 11), _pair(family, 16)
+    fd = T.tpmats_lu_factor([T.TPMatrix([T.Matrix(K0), T.Matrix(M1)]), T.TPMatrix([T.Matrix(M0), T.Matrix(K1)])])
+    F = np.random.default_rng(5).standard_normal(fd.shape)
+    (W0, W1), (V0, V1) = fd.lefts_host, fd.eigvecs_host
+    X = V0 @ ((W0 @ F @ W1.T) / fd.D_host) @ V1.T
+    assert np.linalg.norm(K0 @ X @ M1.T + M0 @ X @ K1.T - F) <= 1e-12 * np.linalg.norm(F)
+    for host, ops in ((fd.eigvecs_host, fd.V), (fd.lefts_host, fd.W)):
+        assert all(np.array_equal(h, o.A64.numpy()) for h, o in zip(host, ops))
