@@ -140,7 +140,7 @@ class Fourier(OrthogonalSpace):
         X = self.map_reference_domain(as_device(x).reshape(-1)).contiguous()
         E = self._basis(X.shape[0], 0, False, 1.0, X)
         c = as_device(c)
-        out = K.apply_along(K.ComplexAxisOperator(E), c, c.ndim - 1, "f64")
+        out = K.apply_along(K.ComplexAxisOperator(E, once=True), c, c.ndim - 1, "f64")
         return out.reshape(tuple(out.shape[:-1]) + tuple(shp))
 
     def derivative_coeffs(self, c, k: int = 0):
@@ -149,7 +149,7 @@ class Fourier(OrthogonalSpace):
             return as_device(c)
         m = self.wavenumbers(eliminate_highest_freq=k % 2 == 1).astype(np.complex128)
         f = torch.tensor((1j * m) ** k, dtype=torch.complex128, device=K.device())
-        return K.apply_along(K.ComplexAxisOperator(torch.diag(f)), as_device(c), as_device(c).ndim - 1)
+        return K.apply_along(K.ComplexAxisOperator(torch.diag(f), once=True), as_device(c), as_device(c).ndim - 1)
 
     # ------------------------------------------------------------ matrices
     def _matrices(self, i, trial, q=0):

@@ -111,7 +111,7 @@ def _quad_nodes(space, N):
 
 
 def _stencil_apply(space, z: torch.Tensor, axis: int) -> torch.Tensor:
-    S = space._stencil_dev() if not space.is_orthogonal else None
+    S = space._stencil_once() if not space.is_orthogonal else None
     return z if S is None else K.apply_along(S, z.contiguous(), axis, "f64")
 
 
@@ -154,7 +154,7 @@ def bilinear_1d(v, i: int, u, j: int, coeff, Nq: int, use_precomputed: bool, wei
     Pi = v.orthogonal.vandermonde(x, i)
     Pj = u.orthogonal.vandermonde(x, j)
     PiTw = K.scale_transpose(Pi.contiguous(), wq.contiguous())            # (Ni, Q)
-    z = K.apply_along(K.AxisOperator(PiTw), Pj.contiguous(), 0, "f64")   # (Ni, Nj)
+    z = K.apply_along(K.AxisOperator(PiTw, once=True), Pj.contiguous(), 0, "f64")   # (Ni, Nj)
     z = _stencil_apply(v, z, 0)
     z = _stencil_apply(u, z, 1)
     return Matrix(z)

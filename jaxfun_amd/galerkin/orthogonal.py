@@ -198,14 +198,26 @@ class OrthogonalSpace:
             self._ops[key] = ok and self.stencil is not None and all(o % 2 == 0 for o in self.stencil)
         return self._ops[key]
 
+    def _stencil_once(self):
+        """The stencil for the one product that builds an operator, None for an
+        orthogonal basis: read as it is (its structure costs more to find and to
+        cut into fragments than such a product takes)."""
+        key = "S once"
+        if key not in self._ops:
+            S = self.stencil_matrix()
+            if S is None:
+                return None
+            self._ops[key] = K.AxisOperator(torch.tensor(S, dtype=torch.float64, device=K.device()), once=True)
+        return self._ops[key]
+
     def _stencil_dev(self):
-        S = self.stencil_matrix()
-        if S is None:
-            return None
+        """The stencil for series and basis values, which are transformed again and again."""
         key = "S"
         if key not in self._ops:
-            self._ops[key] = K.AxisOperator(torch.tensor(S, dtype=torch.float64, device=K.device()),
-                                            K.host_structure(np.asarray(S)))
+            S = self._stencil_once()
+            if S is None:
+                return None
+            self._ops[key] = K.AxisOperator(S.A64, K.host_structure(np.asarray(self.stencil_matrix())))
         return self._ops[key]
 
     def _apply_stencil_cols(self, V: torch.Tensor) -> torch.Tensor:
@@ -225,8 +237,11 @@ class OrthogonalSpace:
         if key not in self._ops:
             X = self._points(kind, N)
             V = self.orthogonal._vander(X, k, float(self.domain_factor) ** k)
+            S = self._stencil_once()
+            if S is not None:
+                V = K.apply_along(S, V.contiguous(), 1, "f64")
             par = K.evaluates_parity((-1) ** k) if kind == MeshKind.QUADRATURE and self.has_parity() else None
-            self._ops[key] = K.AxisOperator(self._apply_stencil_cols(V), par)
+            self._ops[key] = K.AxisOperator(V, par)
         return self._ops[key]
 
     def _weighted_vt(self, N: int) -> torch.Tensor:
@@ -241,7 +256,7 @@ class OrthogonalSpace:
         key = ("sp", N)
         if key not in self._ops:
             WVt = self._weighted_vt(N)
-            S = self._stencil_dev()
+            S = self._stencil_once()
             self._ops[key] = K.AxisOperator(WVt if S is None else K.apply_along(S, WVt, 0, "f64"),
                                             K.projects_parity() if self.has_parity() else None)
         return self._ops[key]
@@ -285,7 +300,7 @@ class OrthogonalSpace:
         nc = int(np.shape(c)[-1])
         if self.is_orthogonal and nc < V.shape[1]:
             V = V[:, :nc]
-        out = _apply_1d(K.AxisOperator(V.contiguous()), c, "f64")
+        out = _apply_1d(K.AxisOperator(V.contiguous(), once=True), c, "f64")
         return out.reshape(tuple(out.shape[:-1]) + tuple(shp))
 
     def derivative_coeffs(self, c, k: int = 0):
@@ -305,12 +320,12 @@ class OrthogonalSpace:
         if key not in self._ops:
             x, _ = self.quad_points_and_weights(self.N)
             Vk = self._vander(x, k).contiguous()                                   # (N, N)
-            self._ops[key] = K.AxisOperator(
-                K.apply_along(self.forward_operator(self.N), Vk, 0, "f64").contiguous())
+            F = K.AxisOperator(self.forward_operator(self.N).A64, once=True)
+            self._ops[key] = K.AxisOperator(K.apply_along(F, Vk, 0, "f64").contiguous())
         D = self._ops[key]
         n = int(c.shape[-1])
         if n < self.N:  # a shorter series: its derivative stays in the first n modes
-            D = K.AxisOperator(D.A64[:n, :n].contiguous())
+            D = K.AxisOperator(D.A64[:n, :n].contiguous(), once=True)
         return K.apply_along(D, c, c.ndim - 1, "f64")
 
     def mass_matrix(self):

@@ -187,7 +187,7 @@ class TensorProductSpace:
         d = len(self)
         B = [self._point_basis(ax, xs[ax]) for ax in range(d)]
         c = as_device(c)
-        op = K.ComplexAxisOperator(B[-1]) if B[-1].is_complex() else K.AxisOperator(B[-1])
+        op = (K.ComplexAxisOperator if B[-1].is_complex() else K.AxisOperator)(B[-1], once=True)
         X = K.apply_along(op, c, c.ndim - 1)
         for ax in range(d - 2, -1, -1):
             Bt = B[ax].T.contiguous()
@@ -196,7 +196,7 @@ class TensorProductSpace:
                 X = K.cmul_bcast(X, Bt if Bt.is_complex() else K.to_complex(Bt))
             else:
                 X = mul_bcast(X, Bt)
-            ones = K.AxisOperator(torch.ones((1, Bt.shape[0]), dtype=torch.float64, device=X.device))
+            ones = K.AxisOperator(torch.ones((1, Bt.shape[0]), dtype=torch.float64, device=X.device), once=True)
             X = K.apply_along(ones, X, X.ndim - 2)
             X = X.reshape(X.shape[:-2] + X.shape[-1:])
         return X.reshape(X.shape[:-1] + tuple(shp))

@@ -453,7 +453,8 @@ class AxisOperator:
 
     ``parity``: its structure (:func:`evaluates_parity`, :func:`projects_parity`,
     :func:`mixes_parity`), which FP64 and FP32 contractions use to halve their
-    products; the caller vouches for it up to rounding.
+    products; the caller vouches for it up to rounding.  ``once``: for a single
+    product, nothing is prepared for later ones.
 
     ``f64`` uses the FP64 matrix; ``f32`` an FP32 copy; ``bf16x3``/``bf16x6``
     2/3 bf16 float slices; ``ozakiS`` S fixed-point digit slices with
@@ -462,12 +463,13 @@ class AxisOperator:
     reference caches factorizations on its matrix objects.
     """
 
-    def __init__(self, A: torch.Tensor, parity: tuple | None = None):
+    def __init__(self, A: torch.Tensor, parity: tuple | None = None, once: bool = False):
         if A.dtype != torch.float64:
             A = A.to(torch.float64)
         self.A64 = A.contiguous()
         self.M, self.K = self.A64.shape
         self.parity = parity
+        self.once = once
         self._prep: dict[str, tuple] = {}
 
     def t(self) -> "AxisOperator":
@@ -482,7 +484,9 @@ class AxisOperator:
         """MFMA fragments of ``csrc/contract_par.hip`` and their structure
         ``(fragments, mode, sgn, p, q)`` for ``prec`` f64 or f32, or None where
         the sizes are not taken.  A first use inside a graph capture gives None
-        too: the capture would record the preparation instead of running it."""
+        too: the capture would record the preparation instead of running it.
+        Those of a ``once`` operator serve the current stream's next product and
+        are not kept, so nothing waits for them."""
         key = PAR_KEYS[prec]
         fr = self._prep.get(key, 0)
         if fr != 0:
@@ -492,10 +496,12 @@ class AxisOperator:
         if n == 0:
             self._prep[key] = None
             return None
-        if torch.cuda.is_current_stream_capturing():
+        if not self.once and torch.cuda.is_current_stream_capturing():
             return None
         f = torch.empty(n, dtype=io_dtype(prec), device=self.A64.device)
         _lib.call("jfx_par_prepare", 0 if prec == "f64" else 1, _p(self.A64), self.M, self.K, mode, sgn, _p(f), _s())
+        if self.once:
+            return f, mode, sgn, p, q
         # complete before they are published: the next use may be on another stream
         torch.cuda.current_stream().synchronize()
         fr = self._prep[key] = (f, mode, sgn, p, q)
@@ -558,11 +564,11 @@ class ComplexAxisOperator:
 
     is_complex = True
 
-    def __init__(self, A: torch.Tensor):
+    def __init__(self, A: torch.Tensor, once: bool = False):
         A = A.to(torch.complex128)
         self.M, self.K = A.shape
         self.A = A.contiguous()
-        self.stacked = AxisOperator(torch.cat([A.real, A.imag], 0).contiguous())
+        self.stacked = AxisOperator(torch.cat([A.real, A.imag], 0).contiguous(), once=once)
 
     def prepared(self, prec: str):
         if prec != "f64":
@@ -590,9 +596,15 @@ def _apply_complex(op: ComplexAxisOperator, X: torch.Tensor, axis: int) -> torch
     return Y
 
 
-def _use_fragments(op: AxisOperator, Q: int) -> bool:
-    """Whether FP64/FP32 contractions of ``op`` run from MFMA fragments."""
-    return op.parity is not None or not (Q == 1 or Q % 64 == 0)
+def _use_fragments(op: AxisOperator, P: int, Q: int) -> bool:
+    """Whether FP64/FP32 contractions of ``op`` run from MFMA fragments.  For a
+    single product they have to be cut first, which pays from 32 columns a row on:
+    (us, as it is / cut and multiplied) 64 x 64 on 2048 columns 14.3 / 10.1; 256 x 64 on
+    2048 16.3 / 22.2, on 32768 50.7 / 38.9; 512 x 128 on 2048 28.7 / 63.7, on 32768
+    149 / 108; 1 x 50 on 1000 11.7 / 9.7, on 1e6 634 / 116."""
+    if op.parity is None and (Q == 1 or Q % 64 == 0):
+        return False
+    return not op.once or P * Q >= 32 * op.M
 
 
 def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
@@ -635,7 +647,7 @@ def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
         _req(out, dt, "out")
         if list(out.shape) != shape:
             raise ValueError("apply_along: bad out shape")
-    if prec in ("f64", "f32") and P * Q > 0 and _use_fragments(op, Q):
+    if prec in ("f64", "f32") and P * Q > 0 and _use_fragments(op, P, Q):
         fr = op.fragments(prec)
         if fr is not None:
             _lib.call("jfx_contract_par", 0 if prec == "f64" else 1, _p(fr[0]), op.M, K, fr[1], fr[2], fr[3], fr[4],

@@ -45,6 +45,7 @@ class BaseMatrix:
         self._host_data = _host(data).copy()
         self._dev = None
         self._op = None
+        self._op_t = None
         self._lu = None
 
     # ---------------------------------------------------------------- data
@@ -78,6 +79,12 @@ class BaseMatrix:
                 K.AxisOperator(self.todense(), K.host_structure(self._host_data))
         return self._op
 
+    def transposed_operator(self):
+        """The operator of A^T, for products from the right."""
+        if self._op_t is None:
+            self._op_t = self.T.operator()
+        return self._op_t
+
     def diagonal_or_none(self) -> np.ndarray | None:
         A = self._host_data
         if A.shape[0] != A.shape[1]:
@@ -104,7 +111,7 @@ class BaseMatrix:
         from ..galerkin.orthogonal import as_device
 
         x = as_device(_coefficients(other))
-        return K.apply_along(self.T.operator(), x, x.ndim - 1, "f64")
+        return K.apply_along(self.transposed_operator(), x, x.ndim - 1, "f64")
 
     @staticmethod
     def _combine(a, data, b=None):
