@@ -364,10 +364,24 @@ __global__ __launch_bounds__(PAR_NT) void contract_par_kernel(const T* __restric
 // Fragment of part h, row block rb, k-step s, lane l: the operator entry of
 // half-row 16 rb + (l & 15) and half-column 4 s + (l >> 4), zero outside.
 // Mirror images are averaged, so that the halves carry the rounding of both.
+// One operator per blockIdx.y.
+struct ParJob {
+  const double* A;
+  void* out;
+  int M, K, mode, sgn, nrb, S, nparts;
+};
+constexpr int PAR_JOBS = 16;
+struct ParJobs {
+  ParJob j[PAR_JOBS];
+};
+
 template <typename T>
-__global__ void par_prepare_kernel(const double* __restrict__ A, int M, int K, int mode, int sgn, int nrb, int S,
-                                   int nparts, T* __restrict__ out) {
-  const long long total = (long long)nparts * nrb * S * 64;
+__global__ void par_prepare_kernel(ParJobs jobs) {
+  const ParJob& J = jobs.j[blockIdx.y];
+  const double* __restrict__ A = J.A;
+  T* __restrict__ out = (T*)J.out;
+  const int M = J.M, K = J.K, mode = J.mode, sgn = J.sgn, nrb = J.nrb, S = J.S;
+  const long long total = (long long)J.nparts * nrb * S * 64;
   for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < total;
        e += (long long)gridDim.x * blockDim.x) {
     const int l = e & 63;
@@ -538,21 +552,42 @@ long long jfx_par_frag_elems(int M, int K, int mode) {
   return (long long)d.nparts * d.nrb * d.S * 64;
 }
 
-int jfx_par_prepare(int dtype, const double* A, int M, int K, int mode, int sgn, void* frag, hipStream_t stream) {
-  if (!A || !frag) return set_error("par_prepare: null pointer"), JFX_EARG;
-  ParDims d;
-  if (!par_dims(M, K, mode, d) || (sgn != 1 && sgn != -1) || (dtype != 0 && dtype != 1))
-    return set_error("par_prepare: bad arguments M=%d K=%d mode=%d", M, K, mode), JFX_ESHAPE;
-  const long long n = (long long)d.nparts * d.nrb * d.S * 64;
-  const unsigned grid = (unsigned)((n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024);
-  if (dtype == 0)
-    hipLaunchKernelGGL(par_prepare_kernel<double>, dim3(grid), dim3(256), 0, stream, A, M, K, mode, sgn, d.nrb, d.S,
-                       d.nparts, (double*)frag);
-  else
-    hipLaunchKernelGGL(par_prepare_kernel<float>, dim3(grid), dim3(256), 0, stream, A, M, K, mode, sgn, d.nrb, d.S,
-                       d.nparts, (float*)frag);
-  JFX_LAUNCH_CHECK();
+int jfx_par_prepare_many(int dtype, int n, const double* const* A, const int* shape, void* const* frag,
+                         hipStream_t stream) {
+  if (n < 0 || (n && (!A || !shape || !frag))) return set_error("par_prepare: null pointer"), JFX_EARG;
+  if (dtype != 0 && dtype != 1) return set_error("par_prepare: dtype must be 0 or 1"), JFX_ESHAPE;
+  for (int i = 0; i < n; ++i) {
+    const int* s = shape + 4 * i;
+    ParDims d;
+    if (!A[i] || !frag[i]) return set_error("par_prepare: null pointer"), JFX_EARG;
+    if (!par_dims(s[0], s[1], s[2], d) || (s[3] != 1 && s[3] != -1))
+      return set_error("par_prepare: bad arguments M=%d K=%d mode=%d", s[0], s[1], s[2]), JFX_ESHAPE;
+  }
+  for (int i0 = 0; i0 < n; i0 += PAR_JOBS) {
+    const int nj = n - i0 < PAR_JOBS ? n - i0 : PAR_JOBS;
+    ParJobs jobs = {};
+    long long most = 0;
+    for (int i = 0; i < nj; ++i) {
+      const int* s = shape + 4 * (i0 + i);
+      ParDims d;
+      par_dims(s[0], s[1], s[2], d);
+      jobs.j[i] = ParJob{A[i0 + i], frag[i0 + i], s[0], s[1], s[2], s[3], d.nrb, d.S, d.nparts};
+      const long long e = (long long)d.nparts * d.nrb * d.S * 64;
+      most = e > most ? e : most;
+    }
+    const dim3 grid((unsigned)((most + 255) / 256 < 1024 ? (most + 255) / 256 : 1024), (unsigned)nj);
+    if (dtype == 0)
+      hipLaunchKernelGGL(par_prepare_kernel<double>, grid, dim3(256), 0, stream, jobs);
+    else
+      hipLaunchKernelGGL(par_prepare_kernel<float>, grid, dim3(256), 0, stream, jobs);
+    JFX_LAUNCH_CHECK();
+  }
   return JFX_OK;
+}
+
+int jfx_par_prepare(int dtype, const double* A, int M, int K, int mode, int sgn, void* frag, hipStream_t stream) {
+  const int shape[4] = {M, K, mode, sgn};
+  return jfx_par_prepare_many(dtype, 1, &A, shape, &frag, stream);
 }
 
 int jfx_contract_par(int dtype, const void* frag, int M, int K, int mode, int sgn, int bp, int bq, const void* X,

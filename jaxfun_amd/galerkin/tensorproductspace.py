@@ -110,10 +110,10 @@ class TensorProductSpace:
         if fuse:
             # leading axes one by one, the last two in one fused pass
             for ax, op in enumerate(ops[:-2]):
-                X = K.apply_along(op, X, nb + ax, prec)
+                X = K.apply_along(op, X, nb + ax, prec, peers=ops)
             return K.plane(ops[-2], ops[-1], X.contiguous(), prec)
         for ax, op in enumerate(ops):
-            X = K.apply_along(op, X, nb + ax, prec)
+            X = K.apply_along(op, X, nb + ax, prec, peers=ops)
         return X
 
     def backward(self, c, N=None, precision: str | None = None):

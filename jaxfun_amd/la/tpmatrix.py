@@ -197,8 +197,7 @@ class TPMatricesLUFactors:
             for ops, m in ((self.V, v if o is None else v[:, o]), (self.W, w if o is None else w[o])):
                 ops.append(K.AxisOperator(torch.tensor(np.ascontiguousarray(m), device=K.device()),
                                           None if o is None else K.mixes_parity()))
-                if o is not None:
-                    ops[-1].fragments("f64")
+        K.prepare_fragments([op for op in (*self.V, *self.W) if op.parity is not None])
         per_term_eigenvalues = [[ev if o is None else np.asarray(ev)[o] for ev, o in zip(evals, orders)]
                                 for evals in per_term_eigenvalues]
         D = np.zeros(self.shape)

@@ -108,3 +108,49 @@ def test_evaluations_prepare_nothing_after_the_first(dev, calls):
     assert np.abs(ref[1] - E @ ch[:, 0]).max() <= 1e-12
     assert np.abs(ref[2] - (1j * m)**2 * ch[:, 0]).max() <= 1e-12
     assert np.abs(ref[3] - ch[0].real @ phi).max() <= 1e-12
+
+
+def test_one_preparation_for_a_pass(dev, calls):
+    """All operators of a transform, a solve or a nonlinear term in one launch."""
+    import torch
+
+    from jaxfun_amd import Div, Grad, TensorProduct, TestFunction, TrialFunction, inner
+
+    T = TensorProduct(_dirichlet("chebyshev", 20), _dirichlet("legendre", 31), _dirichlet("chebyshev", 26))
+    c = torch.randn(18, 29, 24, dtype=torch.float64, device="cuda")
+    u = T.backward(c)
+    assert _prepared(calls) == 1
+    assert torch.linalg.norm(T.forward(u) - c) <= 1e-11 * torch.linalg.norm(c)
+    assert _prepared(calls) == 2
+    T.forward(T.backward(c))
+    assert _prepared(calls) == 2
+    T = TensorProduct(_dirichlet("legendre", 20), _dirichlet("chebyshev", 31))
+    v, u = TestFunction(T), TrialFunction(T)
+    A = inner(v * Div(Grad(u)), sparse=True)
+    del calls[:]
+    f = A.fd_factor()
+    assert _prepared(calls) == 1
+    f.solve(torch.ones(18, 29, dtype=torch.float64, device="cuda"))
+    assert _prepared(calls) == 1
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_operators_cut_together_as_alone(dev, prec):
+    """More operators than one launch takes, of every structure and unequal sizes:
+    the same fragments bit for bit; sizes that are not taken are left out."""
+    import torch
+
+    from jaxfun_amd import kernels as K
+
+    rng = np.random.default_rng(7)
+    structures = [None, K.evaluates_parity(), K.evaluates_parity(-1), K.projects_parity(), K.mixes_parity(),
+                  K.mixes_parity(-1, 1, 3)]
+    sizes = [(1, 1), (17, 33), (128, 126), (5, 512), (512, 5), (2000, 3)]
+    ops = [(torch.tensor(rng.standard_normal(s), device="cuda"), p) for p in structures for s in sizes]
+    together, alone = ([K.AxisOperator(A, p) for A, p in ops] for _ in range(2))
+    K.prepare_fragments(together + together[:3], prec)
+    for a, b in zip(together, alone):
+        assert K.PAR_KEYS[prec] in a._prep
+        fa, fb = a.fragments(prec), b.fragments(prec)
+        assert (fa is None) == (fb is None) == (a.M == 2000)
+        assert fa is None or (fa[1:] == fb[1:] and torch.equal(fa[0], fb[0]))

@@ -96,7 +96,7 @@ def test_host_factors_follow_one_order(family, monkeypatch):
     """eigvecs_host, lefts_host and D_host together solve the problem, as the
     operators built from them do."""
     monkeypatch.setattr(T.K, "device", lambda: torch.device("cpu"))
-    monkeypatch.setattr(T.K.AxisOperator, "fragments", lambda self, prec: None)
+    monkeypatch.setattr(T.K, "prepare_fragments", lambda ops: None)
     (M0, K0), (M1, K1) = _pair(family, 11), _pair(family, 16)
     fd = T.tpmats_lu_factor([T.TPMatrix([T.Matrix(K0), T.Matrix(M1)]), T.TPMatrix([T.Matrix(M0), T.Matrix(K1)])])
     F = np.random.default_rng(5).standard_normal(fd.shape)
