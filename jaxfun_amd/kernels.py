@@ -470,6 +470,7 @@ class AxisOperator:
         self.M, self.K = self.A64.shape
         self.parity = parity
         self.once = once
+        self._made_on = _s() if self.A64.is_cuda else None  # the stream that A64 is ordered on
         self._prep: dict[str, tuple] = {}
 
     def t(self) -> "AxisOperator":
@@ -548,7 +549,7 @@ class AxisOperator:
 
 def prepare_fragments(ops, prec: str = "f64") -> None:
     """Cut the fragments of every operator in ``ops`` that has none yet, in one
-    launch with one wait (19 us for one operator, 22 for four; most of it is the
+    launch with one wait (22 us for one operator, 31 for four; most of it is the
     wait).  Inside a graph capture this does nothing, see
     :meth:`AxisOperator.fragments`."""
     key = PAR_KEYS[prec]
@@ -563,6 +564,9 @@ def prepare_fragments(ops, prec: str = "f64") -> None:
                 todo.append((op, par, n))
     if not todo or torch.cuda.is_current_stream_capturing():
         return
+    # what is kept must not be cut from a matrix that another stream is still computing
+    for raw in {op._made_on for op, _, _ in todo} - {_s()}:
+        torch.cuda.current_stream().wait_stream(torch.cuda.ExternalStream(raw) if raw else torch.cuda.default_stream())
     n = len(todo)
     frags = [torch.empty(m, dtype=io_dtype(prec), device=op.A64.device) for op, _, m in todo]
     A = (ctypes.c_void_p * n)(*[op.A64.data_ptr() for op, _, _ in todo])

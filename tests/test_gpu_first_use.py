@@ -154,3 +154,33 @@ def test_operators_cut_together_as_alone(dev, prec):
         fa, fb = a.fragments(prec), b.fragments(prec)
         assert (fa is None) == (fb is None) == (a.M == 2000)
         assert fa is None or (fa[1:] == fb[1:] and torch.equal(fa[0], fb[0]))
+
+
+@pytest.mark.parametrize("side", ["built", "used"])
+def test_operators_built_on_another_stream(dev, side):
+    """An operator whose matrix is still being computed on its own stream when a
+    product on another stream cuts it: the kept fragments are the finished matrix's."""
+    import torch
+
+    from jaxfun_amd import kernels as K
+
+    rng = np.random.default_rng(9)
+    A, X = rng.standard_normal((40, 40)), rng.standard_normal((3, 40, 24))
+    A *= np.add.outer(np.arange(40), np.arange(40)) % 2 == 0
+    src, x = torch.tensor(A, device="cuda"), torch.tensor(X, device="cuda")
+    dst, big = torch.zeros_like(src), torch.full((4096, 4096), 1e-4, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    other = torch.cuda.Stream()
+    build, use = (other, torch.cuda.current_stream()) if side == "built" else (torch.cuda.current_stream(), other)
+    with torch.cuda.stream(build):
+        for _ in range(8):  # some 15 ms ahead of the matrix
+            big = big @ big
+        dst.copy_(src)
+        op = K.AxisOperator(dst, K.mixes_parity())
+    with torch.cuda.stream(use):
+        first = K.apply_along(op, x, 1)
+    torch.cuda.synchronize()
+    second = K.apply_along(op, x, 1)
+    ref = np.einsum("mk,pkq->pmq", A, X)
+    for y in (first, second):
+        assert np.abs(y.cpu().numpy() - ref).max() <= 1e-13 * np.abs(ref).max()
