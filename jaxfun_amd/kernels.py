@@ -913,6 +913,8 @@ def plane(op0: AxisOperator, op1: AxisOperator, X: torch.Tensor, prec: str = "f6
             _lib.call("jfx_plane_par", md, _p(f0), op0.M, op0.K, s0, p0, q0, _p(f1), op1.M, op1.K, s1, p1, q1, _p(X),
                       _p(Y), _p(E), mode, float(alpha), acc, B, _s())
             return Y
+        if mode == 3:  # unprepared operators inside a graph capture
+            return lincomb([(1.0, mul_bcast(plane(op0, op1, X, prec, alpha=alpha), E))], Y, accumulate)
         _lib.call("jfx_plane_contract", 0, _p(op0.A64), _p(op1.A64), _p(None), _p(None), _p(X), _p(Y), _p(E),
                   mode, float(alpha), acc, B, op0.M, op0.K, op1.M, op1.K, _s())
     else:

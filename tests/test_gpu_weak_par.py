@@ -120,3 +120,41 @@ def test_pcg_stops_and_counts(dev):
         assert np.all(np.abs(it.cpu().numpy() - itr) <= (0 if limit < 9 else 2)) and int(it[2]) == 1 and int(it[5]) == 0
         np.testing.assert_allclose(x.cpu().numpy(), xr, rtol=1e-8, atol=1e-8)
         assert sorted(snaps) == [k for k in (1, 2) if k <= limit]
+
+
+@pytest.mark.parametrize("N", [20, 97])
+def test_first_use_inside_a_capture(dev, N):
+    """The scaled preconditioner whose operators are used for the first time inside
+    a graph capture (its solve before): every replay against the eager result."""
+    import torch
+
+    from jaxfun_amd import kernels as K
+    from jaxfun_amd.learned import VarCoeffPoisson2D
+
+    op, eager = VarCoeffPoisson2D(N, 4), VarCoeffPoisson2D(N, 4)
+    rng = np.random.default_rng(N)
+    batch = 130  # both ends of the slab kernel's rule take it
+    s = torch.tensor(rng.uniform(0.5, 2.0, (batch, N, N)), device=dev)
+    R = torch.tensor(rng.standard_normal((batch, N - 2, N - 2)), device=dev)
+    op.L.solve(R)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        z = op.scaled_precond(s)(R)
+    for _ in range(3):
+        R.copy_(torch.tensor(rng.standard_normal(R.shape), device=dev))
+        g.replay()
+        ref = eager.scaled_precond(s)(R)
+        torch.cuda.synchronize()
+        assert torch.linalg.norm(z - ref) <= 1e-13 * N * torch.linalg.norm(ref)
+    assert torch.equal(op.scaled_precond(s)(R), ref)  # prepared at the next use outside
+    # with a scale and added to an output, as the fused kernel does it
+    a, b = K.AxisOperator(op.B.A64, op.B.parity), K.AxisOperator(op.B.A64, op.B.parity)
+    out, want = torch.ones_like(s), torch.ones_like(s)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        K.plane(a, b, R, "f64", ("mul_each", s), 0.5, out, True)
+    g.replay()
+    K.plane(op.B, op.B, R, "f64", ("mul_each", s), 0.5, want, True)
+    torch.testing.assert_close(out, want, rtol=1e-12, atol=1e-12)
