@@ -190,7 +190,9 @@ class IMEXRungeKutta:
         nb = U.ndim - 2
         ops = self._quad_operators()
         if ops is not None and nb >= 0 and not U.is_complex() and self._quad_pays(math.prod(U.shape[:nb])):
-            return K.quadratic_term(*ops, self._quad_coefficients(), U.contiguous())
+            U = U.contiguous()
+            K._req(U, K.io_dtype(prec), "U")  # the kernel takes either; the integrator has one
+            return K.quadratic_term(*ops, self._quad_coefficients(), U)
         fields = {}
         needed = set()
         for _, o1, o2 in self.nonlinear:

@@ -82,3 +82,27 @@ def test_step_is_the_same_with_and_without(dev, family, N0, N1, batch, precision
         out.append(it.nonlinear_rhs_scalar_product(U).double())
     tol = 1e-13 if precision == "f64" else 2e-6
     assert float((out[0] - out[1]).norm() / out[1].norm()) < tol
+
+
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+def test_the_other_data_type_is_refused(dev, precision):
+    """Fused and separate alike."""
+    import torch
+
+    from jaxfun_amd import Div, FunctionSpace, Grad, Legendre, TensorProduct, TestFunction, TrialFunction
+    from jaxfun_amd.galerkin.arguments import t
+    from jaxfun_amd.integrators import ARS443, IMEXRungeKutta
+
+    D = FunctionSpace(12, Legendre, {"left": {"D": 0}, "right": {"D": 0}})
+    T = TensorProduct(D, D)
+    v, u = TestFunction(T), TrialFunction(T, transient=True)
+    x, y = T.system.base_scalars()
+    weak = v * (u.diff(t) + u * (u.diff(x) + u.diff(y)) - 1e-2 * Div(Grad(u)))
+    it = IMEXRungeKutta(weak, tableau=ARS443, initial=sp.S.Zero, precision=precision)
+    assert it._quad_operators() is not None
+    other = torch.float32 if it.dt_io == torch.float64 else torch.float64
+    for pays in (True, False):
+        it._quad_pays = lambda n, p=pays: p
+        with pytest.raises(TypeError):
+            it.nonlinear_rhs_scalar_product(torch.zeros((2, 10, 10), dtype=other, device=dev))
+        it.nonlinear_rhs_scalar_product(torch.zeros((2, 10, 10), dtype=it.dt_io, device=dev))
