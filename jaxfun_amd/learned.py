@@ -273,22 +273,27 @@ def pcg(apply, b: torch.Tensor, precond, x0: torch.Tensor | None = None, rtol: f
     host = torch.empty(2, dtype=torch.int32, pin_memory=True)
     seen = host.numpy()
     ev = [torch.cuda.Event(), torch.cuda.Event()]
-    for it in range(maxiter):
-        slot = it % _LEFT_SLOTS
-        if it and slot == 0:
-            left.zero_()
-        q = apply(p)
-        _lib.call("jfx_pcg_step", K._p(x), K._p(r), K._p(p), K._p(q), K._p(rz), K._p(bb), rtol * rtol, K._p(active),
-                  K._p(iters), left.data_ptr() + 4 * slot, host.data_ptr() + 4 * (it % 2), B, n, K._s())
-        ev[it % 2].record()
-        if it and it % check_every == 0:  # after iteration it - 1
-            ev[(it - 1) % 2].synchronize()
-            if seen[(it - 1) % 2] == 0:
-                break
-        if snap_out is not None and it + 1 in snapshots:
-            snap_out[it + 1] = (x.clone(), r.clone())
-        z = precond(r)
-        _lib.call("jfx_pcg_direction", K._p(p), K._p(z), K._p(r), K._p(rz), K._p(active), B, n, K._s())
+    stream = torch.cuda.current_stream()
+    try:
+        for it in range(maxiter):
+            slot = it % _LEFT_SLOTS
+            if it and slot == 0:
+                left.zero_()
+            q = apply(p)
+            _lib.call("jfx_pcg_step", K._p(x), K._p(r), K._p(p), K._p(q), K._p(rz), K._p(bb), rtol * rtol, K._p(active),
+                      K._p(iters), left.data_ptr() + 4 * slot, host.data_ptr() + 4 * (it % 2), B, n, K._s())
+            ev[it % 2].record()
+            if it and it % check_every == 0:  # after iteration it - 1
+                ev[(it - 1) % 2].synchronize()
+                if seen[(it - 1) % 2] == 0:
+                    break
+            if snap_out is not None and it + 1 in snapshots:
+                snap_out[it + 1] = (x.clone(), r.clone())
+            z = precond(r)
+            _lib.call("jfx_pcg_direction", K._p(p), K._p(z), K._p(r), K._p(rz), K._p(active), B, n, K._s())
+    except BaseException:
+        stream.synchronize()  # a queued step still stores to `host`
+        raise
     if maxiter > 0:
         ev[it % 2].synchronize()  # the last store to `host`, which is freed on return
     if breakdown == "raise":

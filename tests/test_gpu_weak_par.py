@@ -158,3 +158,31 @@ def test_first_use_inside_a_capture(dev, N):
     g.replay()
     K.plane(op.B, op.B, R, "f64", ("mul_each", s), 0.5, want, True)
     torch.testing.assert_close(out, want, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("where", ["apply", "precond"])
+def test_pcg_leaves_no_queued_store_behind(dev, where):
+    """A callback that raises: the steps queued so far, which store to a pinned
+    buffer of the call, are finished when the exception comes out."""
+    import torch
+
+    from jaxfun_amd.learned import pcg
+
+    b = torch.tensor(np.random.default_rng(2).standard_normal((3, 1, 20)), device=dev)
+    lam = torch.linspace(1.0, 50.0, 20, dtype=torch.float64, device=dev)
+    big = torch.full((4096, 4096), 1e-4, dtype=torch.float64, device=dev)
+    count = {"apply": 0, "precond": 0}
+
+    def step(name, y):
+        count[name] += 1
+        if name == where and count[name] == 4:
+            raise RuntimeError("stop here")
+        if name == "apply":
+            for _ in range(4):  # some 8 ms of queued work ahead of the step
+                torch.mm(big, big)
+        return y
+
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError, match="stop here"):
+        pcg(lambda U: step("apply", lam * U), b, lambda R: step("precond", R.clone()), rtol=1e-14)
+    assert torch.cuda.current_stream().query()
