@@ -408,8 +408,8 @@ int jfx_cast(int direction, const void* x, void* y, long long n, hipStream_t str
  *   FP32 (io_f32 selects float or double F/U).
  *   nwaves 4 or 8 (mode 1: 4 = two 4-wave workgroups per CU, one column
  *   parity at a time; 8 = one 8-wave workgroup per CU, both column parities
- *   at once with whole-row F reads and U writes); mode 0
- *   wants scratch of nblocks * jfx_helm_scratch_doubles_per_block() doubles.
+ *   at once with whole-row F reads and U writes).
+ * scratch: nblocks * jfx_helm_scratch_doubles_per_block() doubles, now none; may be null.
  * mode 2: as mode 1 with a 2-term fp16 split (three MFMA products instead of
  *   six): each operand block is scaled by a power of two from its largest
  *   entry before the split and the products are scaled back exactly; nwaves 4

@@ -1588,19 +1588,20 @@ int jfx_helm_ragged_noalloc(int io_f32, int nwaves, const void* items, int nitem
 
 int jfx_helm_item_size(void) { return (int)sizeof(HelmItem); }
 
-int jfx_helm_scratch_doubles_per_block(void) { return HMAXA * HMAXA; }
+// Kept for callers that size the scratch argument: no mode needs any.
+int jfx_helm_scratch_doubles_per_block(void) { return 0; }
 
 // mode 0: FP64 (F, U double; Vd/VTd used)
 // mode 1: BF16 3-term split, FP32 storage (F, U float if io_f32 else double; Vs/VTs used)
 // mode 2: FP16 2-term split (tables V 2^eA in two fp16 slices, eA in the
 //         item's pad field; blocks scaled by a power of two), nwaves 4
 // nwaves: 4 or 8 waves per workgroup; nblocks: persistent grid size
-//   (mult_scratch is not used; it must not be null).
+//   (scratch is not used and may be null).
 int jfx_helm_ragged(int mode, int io_f32, int nwaves, const void* items, int nitems, int* counters,
                     const int* qbounds, int nqueues, const double* Vd, const double* VTd, const unsigned short* Vs,
                     const unsigned short* VTs, const double* lam, const void* F, void* U,
-                    double* mult_scratch, int nblocks, hipStream_t stream) {
-  if (!items || !counters || !qbounds || !lam || !F || !U || !mult_scratch || nitems < 0 || nblocks <= 0)
+                    double*, int nblocks, hipStream_t stream) {
+  if (!items || !counters || !qbounds || !lam || !F || !U || nitems < 0 || nblocks <= 0)
     return set_error("helm_ragged: bad arguments"), JFX_EARG;
   if (nqueues < 1 || nqueues > HMAXQ) return set_error("helm_ragged: nqueues must be in [1, 16]"), JFX_EARG;
   if (nitems == 0) return JFX_OK;

@@ -115,8 +115,6 @@ class HelmholtzBatch:
         self.nwaves, self.blocks_per_cu = nwaves, blocks_per_cu
         cus = torch.cuda.get_device_properties(self.dev).multi_processor_count
         self.nblocks = int(cus * blocks_per_cu)
-        per = _lib.load().jfx_helm_scratch_doubles_per_block()
-        self.scratch = torch.empty(self.nblocks * per, dtype=torch.float64, device=self.dev)
         self._graph = None
 
     # ------------------------------------------------------------------ set-up
@@ -236,7 +234,7 @@ class HelmholtzBatch:
                   self.nwaves, K._p(self.items), self.nitems, K._p(self.counter), K._p(self.qbounds),
                   self.nqueues, K._p(self.Vd),
                   K._p(self.VTd), K._p(self.Vs), K._p(self.VTs), K._p(self.lam), K._p(F), K._p(U),
-                  K._p(self.scratch), self.nblocks, K._s())
+                  K._p(None), self.nblocks, K._s())
 
     def _check_io(self, F: torch.Tensor, U: torch.Tensor | None) -> None:
         """F (and U) must be contiguous device tensors of the I/O dtype holding

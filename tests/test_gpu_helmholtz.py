@@ -242,3 +242,18 @@ def test_fp64_block_edges(dev, Ns):
             # backward error of a stable solve: a few eps times the operator's norm, the size and |u|
             scale = (al * np.linalg.norm(M, 2)**2 + 2 * np.linalg.norm(K, 2) * np.linalg.norm(M, 2)) * np.linalg.norm(u)
             assert np.linalg.norm(r) <= 2.0**-52 * 20 * N * (scale + np.linalg.norm(f)), N
+
+
+@pytest.mark.parametrize("mode", ["fp64", "mixed", "mixed16"])
+def test_launch_shapes_take_no_memory(dev, mode):
+    """A launch shape is a number of workgroups: choosing one allocates nothing."""
+    import torch
+
+    from jaxfun_amd import _lib
+    from jaxfun_amd.helmholtz import HelmholtzBatch
+
+    hb = HelmholtzBatch(np.array([10, 33]), np.array([1.0, 2.0]), mode=mode)
+    before = torch.cuda.memory_allocated()
+    hb.set_launch(4, 8)
+    assert torch.cuda.memory_allocated() <= before
+    assert _lib.load().jfx_helm_scratch_doubles_per_block() == 0
