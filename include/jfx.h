@@ -457,12 +457,6 @@ int jfx_adam(float* p, const float* g, float* m, float* v, long long n, float lr
  * no PCG; the operator is TensorMatrix's matvec (la/tensormatrix.py:54-56).
  * out[b] = <x_b, y_b> */
 int jfx_batched_dot(const double* x, const double* y, double* out, int batch, long long n, hipStream_t stream);
-/* x_b += (num_b/den_b) p_b, r_b -= (num_b/den_b) q_b for active b */
-int jfx_pcg_update_xr(double* x, double* r, const double* p, const double* q, const double* num,
-                      const double* den, const int* active, int batch, long long n, hipStream_t stream);
-/* p_b = z_b + (num_b/den_b) p_b for active b */
-int jfx_pcg_update_p(double* p, const double* z, const double* num, const double* den, const int* active,
-                     int batch, long long n, hipStream_t stream);
 /* active_b &= rr_b > tol2 bb_b, counting iters_b for systems active on entry when count != 0;
  * a non-finite rr_b stops system b with iters_b = -1 (breakdown) */
 int jfx_pcg_check(const double* rr, const double* bb, double tol2, int* active, int* iters, int batch, int count,

@@ -180,29 +180,6 @@ __global__ void batched_dot_kernel(const double* __restrict__ x, const double* _
   if (threadIdx.x == 0) out[b] = red[0];
 }
 
-// x += a p, r -= a q with a = num[b] / den[b] for active systems
-__global__ void pcg_xr_kernel(double* __restrict__ x, double* __restrict__ r, const double* __restrict__ p,
-                              const double* __restrict__ q, const double* __restrict__ num,
-                              const double* __restrict__ den, const int* __restrict__ active, long long n) {
-  const long long b = blockIdx.y;
-  if (!active[b]) return;
-  const double a = num[b] / den[b];
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    x[b * n + i] += a * p[b * n + i];
-    r[b * n + i] -= a * q[b * n + i];
-  }
-}
-
-// p = z + (num[b] / den[b]) p for active systems
-__global__ void pcg_p_kernel(double* __restrict__ p, const double* __restrict__ z, const double* __restrict__ num,
-                             const double* __restrict__ den, const int* __restrict__ active, long long n) {
-  const long long b = blockIdx.y;
-  if (!active[b]) return;
-  const double beta = num[b] / den[b];
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    p[b * n + i] = z[b * n + i] + beta * p[b * n + i];
-}
-
 // active[b] &= rr[b] > tol2 * bb[b]; iters[b] += (was active)
 __global__ void pcg_check_kernel(const double* __restrict__ rr, const double* __restrict__ bb, double tol2,
                                  int* __restrict__ active, int* __restrict__ iters, int batch, int count) {
@@ -399,28 +376,6 @@ int jfx_batched_dot(const double* x, const double* y, double* out, int batch, lo
   if (!x || !y || !out || batch < 0 || n < 0) return set_error("batched_dot: bad arguments"), JFX_EARG;
   if (batch == 0) return JFX_OK;
   hipLaunchKernelGGL(batched_dot_kernel, dim3(batch), dim3(256), 0, stream, x, y, out, n);
-  JFX_LAUNCH_CHECK();
-  return JFX_OK;
-}
-
-int jfx_pcg_update_xr(double* x, double* r, const double* p, const double* q, const double* num,
-                      const double* den, const int* active, int batch, long long n, hipStream_t stream) {
-  if (!x || !r || !p || !q || !num || !den || !active || batch < 0 || batch > 65535)
-    return set_error("pcg_update_xr: bad arguments"), JFX_EARG;
-  if (batch == 0 || n == 0) return JFX_OK;
-  dim3 g((unsigned)((n + 255) / 256 > 64 ? 64 : (n + 255) / 256), batch);
-  hipLaunchKernelGGL(pcg_xr_kernel, g, dim3(256), 0, stream, x, r, p, q, num, den, active, n);
-  JFX_LAUNCH_CHECK();
-  return JFX_OK;
-}
-
-int jfx_pcg_update_p(double* p, const double* z, const double* num, const double* den, const int* active,
-                     int batch, long long n, hipStream_t stream) {
-  if (!p || !z || !num || !den || !active || batch < 0 || batch > 65535)
-    return set_error("pcg_update_p: bad arguments"), JFX_EARG;
-  if (batch == 0 || n == 0) return JFX_OK;
-  dim3 g((unsigned)((n + 255) / 256 > 64 ? 64 : (n + 255) / 256), batch);
-  hipLaunchKernelGGL(pcg_p_kernel, g, dim3(256), 0, stream, p, z, num, den, active, n);
   JFX_LAUNCH_CHECK();
   return JFX_OK;
 }
