@@ -28,8 +28,8 @@
 //   Q > 1   LDS tile Bs[k][c]; a 16x16 result block has rows m and columns c.
 //   Q == 1  LDS tile Xs[c][k]; the operands swap roles, so that result blocks
 //           have rows c and columns m and stores run along the contiguous axis.
-// LDS strides keep the reads of a wave on distinct banks: 4 rows (8 apart in
-// the parity order) times 16 columns, see lds_stride().
+// A wave reads 4 rows times 16 columns of the tile; strides: lds_stride_cols(),
+// lds_stride_rows().
 // `band`: operators with A[m, k] = 0 outside -bp <= k - m <= bq skip the k-steps
 // a row block does not touch (mass matrices: 5 of 16; triangular stiffness: half).
 #include "par_blocks.h"
@@ -49,11 +49,11 @@ struct ParMap {
   short lo[2][PAR_MAXRB], hi[2][PAR_MAXRB];  // k-steps (even counts) of each part's row block
 };
 
-// Elements between LDS rows.  Q > 1: 16 columns of rows 2 apart (EVAL, MIX) or
-// 1 apart (DENSE, PROJ) must fall on distinct banks: 2 * stride or stride = 16
-// mod 32 doubles (FP32: mod 64 words).  Q == 1: rows c, stride twice (FP32: four
-// times) an odd number.
-template <typename T, int MODE, int NB>
+// Elements between LDS rows.  Q > 1: EVAL and MIX read rows 2 apart, and 2 * stride
+// = 16 (mod 32 doubles, for FP32 mod 64 words) puts their 16 columns on distinct
+// banks.  DENSE and PROJ read neighbouring rows, stride = 8 or 24 apart, which share
+// half their banks.  Q == 1: rows c, stride twice (FP32: four times) an odd number.
+template <int NB>
 __host__ __device__ constexpr int lds_stride_cols() {
   return 16 * NB + 8;
 }
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(PAR_NT) void contract_par_kernel(const T* __restric
   typedef typename ParT<T>::V V;
   typedef typename ParT<T>::T2 T2;
   constexpr int TN = 16 * NB;
-  constexpr int LDC = lds_stride_cols<T, MODE, NB>();
+  constexpr int LDC = lds_stride_cols<NB>();
   constexpr bool PARIN = MODE == MODE_EVAL || MODE == MODE_MIX;
   constexpr int NPART = MODE == MODE_DENSE ? 1 : 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -474,7 +474,7 @@ template <typename T, int MODE, bool QONE, int NB, int JB>
 static int launch_par3(const T* Af, const T* X, T* Y, const ParMap& pm, hipStream_t st) {
   const int kz = par_kz(MODE, pm.K, pm.S);
   const size_t rows = QONE ? (size_t)16 * NB * lds_stride_rows(kz, sizeof(T))
-                           : (size_t)kz * lds_stride_cols<T, MODE, NB>();
+                           : (size_t)kz * lds_stride_cols<NB>();
   const size_t shm = (rows * sizeof(T) + 15) & ~(size_t)15;
   auto kern = pm.nt ? contract_par_kernel<T, MODE, QONE, NB, JB, true> : contract_par_kernel<T, MODE, QONE, NB, JB, false>;
   if (shm > 64 * 1024) JFX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
