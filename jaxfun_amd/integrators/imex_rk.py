@@ -169,16 +169,23 @@ class IMEXRungeKutta:
         """Whether the fused term is the faster one.  A problem is one workgroup's
         work, so its time goes by rounds of one problem per CU; the separate launches
         spread over the chip but cost 70 us at least.  Up to 128 mesh points an axis a
-        round takes 15 to 40 us: always.  Beyond, FP64 from 90 problems on (192 x 192:
-        100 problems 161 us fused, 174 separate; 20 problems 155 / 105); mixed precision
-        too, except that meshes in multiples of 64 points, which the separate bf16x6
-        contractions read best, need rounds that are nearly full (256 problems on 192 x
-        192 185 / 189 us alone and 25 us less in a step, 160 problems 172 / 148)."""
+        round takes 15 to 70 us: always.  Beyond, from 90 problems on (us, fused /
+        separate, FP64: 144 x 144 64 problems 100 / 100, 90 99 / 110; 192 x 192 64 160 /
+        138, 90 158 / 176; 176 points on axis 1 are six strips as 192 are, and the lines
+        cross at 100 problems there).  Mixed precision too, but 192 points on axis 1 are
+        the layout that the separate bf16x6 contractions read best (192 x 192: 200
+        problems 163 / 169, 256 163 / 181, 300 317 / 222, 512 323 / 315; 129 x 192: 160
+        131 / 114, 200 132 / 147, 300 254 / 174; 96 x 192: 90 77 / 82, 300 147 / 131, 512
+        151 / 167).  There more than 96 points on axis 0 want one round that is three
+        quarters full, 65 to 96 a second round that is nearly full, fewer nothing."""
         if max(self.Np) <= 128:
             return True
         cus = K.num_cus()
-        if self.precision != "f64" and all(q % 64 == 0 for q in self.Np):
-            return nbatch >= 0.9 * cus * -(-nbatch // cus)
+        if self.precision != "f64" and self.Np[0] > 64 and self.Np[1] % 64 == 0 and self.testspace[1].dim <= 128 < self.Np[1]:
+            if self.Np[0] > 96:
+                return 0.75 * cus <= nbatch <= cus
+            if nbatch > cus:
+                return nbatch >= 0.9 * cus * -(-nbatch // cus)
         return nbatch >= 0.35 * cus
 
     def nonlinear_rhs_scalar_product(self, U):
