@@ -491,8 +491,10 @@ static int launch_par2(const T* Af, const T* X, T* Y, const ParMap& pm, hipStrea
   // wave takes both column blocks of a row block, so that the operator is read
   // once for both, unless that leaves waves idle.  (Single column blocks also
   // where five or six row blocks would come out more even: slower, 274 against
-  // 257 us at M = 160, K = 158, 256000 columns.)
-  const bool two = pm.K <= (sizeof(T) == 8 ? 192 : 384), thin = pm.nrb <= 2;
+  // 257 us at M = 160, K = 158, 256000 columns.)  Dense FP64 operators keep all K rows
+  // of a full-size product: 16 columns beyond K = 160 (128 x 192 on 2^20 columns 2072
+  // -> 1628 us, plain matrix 1770; 192 x 192 2910 -> 2308).
+  const bool two = pm.K <= (sizeof(T) == 8 ? (MODE == MODE_DENSE ? 160 : 192) : 384), thin = pm.nrb <= 2;
   if (pm.Q == 1)
     return !two   ? launch_par3<T, MODE, true, 1, 1>(Af, X, Y, pm, st)
            : thin ? launch_par3<T, MODE, true, 2, 1>(Af, X, Y, pm, st)

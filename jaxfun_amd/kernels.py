@@ -625,14 +625,32 @@ def _apply_complex(op: ComplexAxisOperator, X: torch.Tensor, axis: int) -> torch
     return Y
 
 
-def _use_fragments(op: AxisOperator, P: int, Q: int) -> bool:
-    """Whether FP64/FP32 contractions of ``op`` run from MFMA fragments.  For a
-    single product they have to be cut first, which pays from 32 columns a row on:
-    (us, as it is / cut and multiplied) 64 x 64 on 2048 columns 14.3 / 10.1; 256 x 64 on
-    2048 16.3 / 22.2, on 32768 50.7 / 38.9; 512 x 128 on 2048 28.7 / 63.7, on 32768
-    149 / 108; 1 x 50 on 1000 11.7 / 9.7, on 1e6 634 / 116."""
-    if op.parity is None and (Q == 1 or Q % 64 == 0):
-        return False
+def _use_fragments(op: AxisOperator, P: int, Q: int, prec: str) -> bool:
+    """Whether FP64/FP32 contractions of ``op`` run from MFMA fragments.
+
+    Operators with a structure: always.  Others: in layouts that the kernels for the
+    plain matrix read badly, where (us, plain / fragments) the fragments are the
+    faster ones.  A workgroup takes all rows of its columns, so many rows want many
+    columns; K beyond ``kmax`` leaves room for 16 columns and little overlap, which
+    few columns do not mind.  FP64, 65536 columns: 128 x 192 142 / 138, 200 x 200 213 /
+    210, 224 x 222 243 / 340, 100 x 400 284 / 394, 512 x 100 295 / 193; 4096 columns: 224
+    x 222 47 / 41, 100 x 400 76 / 44, 512 x 100 27 / 48, 512 x 256 58 / 103.  FP32, 65536:
+    256 x 254 150 / 143, 300 x 298 213 / 250, 100 x 400 122 / 189, 512 x 256 300 / 261;
+    4096: 100 x 400 59 / 27, 400 x 200 35 / 41.
+
+    For a single product they have to be cut first, which pays from 32 columns a row
+    on: 64 x 64 on 2048 columns 14.3 / 10.1; 256 x 64 on 2048 16.3 / 22.2, on 32768
+    50.7 / 38.9; 512 x 128 on 2048 28.7 / 63.7, on 32768 149 / 108; 1 x 50 on 1000 11.7 /
+    9.7, on 1e6 634 / 116."""
+    if op.parity is None:
+        if Q == 1 or Q % 64 == 0:
+            return False
+        kmax, few = (208, 8192) if prec == "f64" else (256, 16384)
+        if op.M <= 320:
+            if op.K > kmax and P * Q > min(2 * few, 320 * few // op.M):
+                return False
+        elif op.K > kmax or P * Q <= few:
+            return False
     return not op.once or P * Q >= 32 * op.M
 
 
@@ -676,7 +694,7 @@ def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
         _req(out, dt, "out")
         if list(out.shape) != shape:
             raise ValueError("apply_along: bad out shape")
-    if prec in ("f64", "f32") and P * Q > 0 and _use_fragments(op, P, Q):
+    if prec in ("f64", "f32") and P * Q > 0 and _use_fragments(op, P, Q, prec):
         fr = op.fragments(prec, peers)
         if fr is not None:
             _lib.call("jfx_contract_par", 0 if prec == "f64" else 1, _p(fr[0]), op.M, K, fr[1], fr[2], fr[3], fr[4],

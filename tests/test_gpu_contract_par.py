@@ -171,3 +171,21 @@ def test_prepared_on_another_stream():
     torch.cuda.synchronize()
     bound = np.abs(x.cpu().numpy()) @ np.abs(A).T
     assert np.all(np.abs(y.cpu().numpy() - x.cpu().numpy() @ A.T) <= 68 * EPS["f64"] * bound)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("M,Kd,pre,post", [(33, 160, (2,), (37,)), (33, 161, (2,), (37,)), (65, 176, (3,), (18,)),
+                                           (17, 192, (1,), (70,)), (40, 193, (2,), (5,)), (512, 5, (821,), (10,)),
+                                           (321, 161, (1639,), (10,)), (300, 256, (1,), (33,)), (9, 400, (2,), (15,))])
+def test_dense_operators_in_ragged_layouts(dev, prec, M, Kd, pre, post):
+    """Around the K at which a workgroup takes 16 columns instead of 32, and the
+    ends of the ranges that go by fragments."""
+    import torch
+
+    from jaxfun_amd import kernels as K
+
+    rng = np.random.default_rng(M + Kd)
+    A = rng.standard_normal((M, Kd))
+    op = K.AxisOperator(torch.tensor(A, device="cuda"))
+    _check(op, A, rng.standard_normal(pre + (Kd,) + post), len(pre), prec)
+    assert (op._prep.get(K.PAR_KEYS[prec]) is not None) == K._use_fragments(op, int(np.prod(pre)), int(np.prod(post)), prec)
