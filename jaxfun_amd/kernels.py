@@ -815,13 +815,15 @@ def _slab_fragments(ops):
 def slab_pays(op0, op1, nslabs: int) -> bool | None:
     """Whether ``nslabs`` slabs run faster through the fused FP64 slab kernel than
     axis by axis; None where that kernel does not take the operators.  A slab is
-    one workgroup's work: up to 64 x 64 always (256 slabs 12.0 us, per axis
-    16.5 us; one 10.2 / 14.9 us), larger ones when they occupy half the CUs
-    (128 x 128: 256 slabs 36 us, per axis 47 us; 64 slabs 28 us, per axis 20 us)."""
+    one workgroup's work: up to 64 x 128 values always (us, slab / per axis: one of 64
+    x 64 10.2 / 14.9, 256 12.0 / 16.5; one of 128 x 64 14.1 / 16.5, one of 128 x 20
+    10.2 / 16.1, 100 of 80 x 80 16.8 / 16.8), larger ones when they occupy half the CUs
+    (96 x 96: 16 slabs 18.4 / 16.3, 128 20.0 / 23.3; 128 x 128: 16 27 / 17, 128 29 / 34,
+    256 33 / 44)."""
     if any(type(o) is not AxisOperator or o.parity is None or max(o.M, o.K) > 128 for o in (op0, op1)) or \
             op0.parity[0] != op1.parity[0]:
         return None
-    return max(op0.M, op0.K, op1.M, op1.K) <= 64 or 2 * nslabs >= num_cus()
+    return max(op0.M, op0.K) * max(op1.M, op1.K) <= 64 * 128 or 2 * nslabs >= num_cus()
 
 
 def plane_fd_par_ok(ops) -> bool:

@@ -1,10 +1,12 @@
-"""The choice between MFMA fragments and the plain matrix for unstructured
-operators in ragged layouts (kernels._use_fragments) against both times, us,
-measured on a card of 256 CUs."""
+"""Choices of kernels by size against the times of both sides, us, measured on a
+card of 256 CUs: MFMA fragments or the plain matrix for unstructured operators in
+ragged layouts (kernels._use_fragments), slab kernel or one launch per axis
+(kernels.slab_pays)."""
 
 from types import SimpleNamespace
 
 import pytest
+import torch
 
 from jaxfun_amd import kernels as K
 
@@ -28,3 +30,18 @@ def test_the_faster_one_is_chosen(prec, M, Kd, P, Q, plain, fragments):
     op = SimpleNamespace(M=M, K=Kd, parity=None, once=False)
     assert K._use_fragments(op, P, Q, prec) == (fragments < plain)
     assert K._use_fragments(SimpleNamespace(M=M, K=Kd, parity=K.evaluates_parity(), once=False), P, Q, prec)
+
+
+# M0, K0, M1, K1, slabs, slab kernel, per axis
+SLABS = [(64, 62, 64, 62, 1, 10, 15), (66, 64, 66, 64, 16, 13, 16), (80, 78, 80, 78, 1, 15.3, 16.2),
+         (64, 62, 128, 126, 100, 15.4, 18.1), (126, 128, 62, 64, 1, 15.5, 16.5), (20, 18, 128, 126, 1, 9.4, 16.8),
+         (94, 96, 31, 33, 100, 11, 17), (2, 3, 126, 128, 16, 9.9, 17.7), (96, 94, 96, 94, 1, 17.8, 16.3),
+         (96, 94, 96, 94, 128, 20, 23), (128, 126, 128, 126, 16, 27, 17), (128, 126, 128, 126, 200, 31, 43)]
+
+
+@pytest.mark.parametrize("M0,K0,M1,K1,slabs,fused,separate", SLABS)
+def test_the_faster_slab_pass_is_chosen(monkeypatch, M0, K0, M1, K1, slabs, fused, separate):
+    monkeypatch.setattr(K, "num_cus", lambda: 256)
+    ops = [K.AxisOperator(torch.zeros(s, dtype=torch.float64), K.evaluates_parity()) for s in ((M0, K0), (M1, K1))]
+    assert K.slab_pays(*ops, slabs) == (fused < separate)
+    assert K.slab_pays(ops[0], K.AxisOperator(ops[1].A64), slabs) is None
