@@ -100,8 +100,8 @@ int jfx_split_matrix(const double* A, int M, int K, int mode, int nslices, unsig
 long long jfx_par_frag_elems(int M, int K, int mode);
 int jfx_par_prepare(int dtype, const double* A, int M, int K, int mode, int sgn, void* frag, hipStream_t stream);
 /* n operators in one launch; A, frag: host arrays of n device addresses; shape: host
- * array of n times (M, K, mode, sgn). */
-int jfx_par_prepare_many(int dtype, int n, const double* const* A, const int* shape, void* const* frag,
+ * array of n times (M, K, mode, sgn); wait: return when they are complete. */
+int jfx_par_prepare_many(int dtype, int n, const double* const* A, const int* shape, void* const* frag, int wait,
                          hipStream_t stream);
 int jfx_contract_par(int dtype, const void* frag, int M, int K, int mode, int sgn, int bp, int bq, const void* X,
                      void* Y, long long P, long long Q, hipStream_t stream);

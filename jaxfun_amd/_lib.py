@@ -38,7 +38,7 @@ SIGNATURES: dict[str, tuple] = {
     "jfx_split_matrix": (c_int, [c_vp, c_int, c_int, c_int, c_int, c_vp, c_vp, c_vp]),
     "jfx_par_frag_elems": (c_ll, [c_int, c_int, c_int]),
     "jfx_par_prepare": (c_int, [c_int, c_vp, c_int, c_int, c_int, c_int, c_vp, c_vp]),
-    "jfx_par_prepare_many": (c_int, [c_int, c_int, c_vp, c_vp, c_vp, c_vp]),
+    "jfx_par_prepare_many": (c_int, [c_int, c_int, c_vp, c_vp, c_vp, c_int, c_vp]),
     "jfx_contract_par": (c_int, [c_int, c_vp, c_int, c_int, c_int, c_int, c_int, c_int, c_vp, c_vp, c_ll, c_ll,
                                  c_vp]),
     "jfx_plane_par": (c_int, [c_int, c_vp, c_int, c_int, c_int, c_int, c_int, c_vp, c_int, c_int, c_int, c_int, c_int,

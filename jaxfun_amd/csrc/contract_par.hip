@@ -554,7 +554,7 @@ long long jfx_par_frag_elems(int M, int K, int mode) {
   return (long long)d.nparts * d.nrb * d.S * 64;
 }
 
-int jfx_par_prepare_many(int dtype, int n, const double* const* A, const int* shape, void* const* frag,
+int jfx_par_prepare_many(int dtype, int n, const double* const* A, const int* shape, void* const* frag, int wait,
                          hipStream_t stream) {
   if (n < 0 || (n && (!A || !shape || !frag))) return set_error("par_prepare: null pointer"), JFX_EARG;
   if (dtype != 0 && dtype != 1) return set_error("par_prepare: dtype must be 0 or 1"), JFX_ESHAPE;
@@ -584,12 +584,13 @@ int jfx_par_prepare_many(int dtype, int n, const double* const* A, const int* sh
       hipLaunchKernelGGL(par_prepare_kernel<float>, grid, dim3(256), 0, stream, jobs);
     JFX_LAUNCH_CHECK();
   }
+  if (wait) JFX_CHECK_HIP(hipStreamSynchronize(stream));
   return JFX_OK;
 }
 
 int jfx_par_prepare(int dtype, const double* A, int M, int K, int mode, int sgn, void* frag, hipStream_t stream) {
   const int shape[4] = {M, K, mode, sgn};
-  return jfx_par_prepare_many(dtype, 1, &A, shape, &frag, stream);
+  return jfx_par_prepare_many(dtype, 1, &A, shape, &frag, 0, stream);
 }
 
 int jfx_contract_par(int dtype, const void* frag, int M, int K, int mode, int sgn, int bp, int bq, const void* X,

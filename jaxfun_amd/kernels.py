@@ -572,9 +572,8 @@ def prepare_fragments(ops, prec: str = "f64") -> None:
     A = (ctypes.c_void_p * n)(*[op.A64.data_ptr() for op, _, _ in todo])
     F = (ctypes.c_void_p * n)(*[f.data_ptr() for f in frags])
     shape = (ctypes.c_int * (4 * n))(*[v for op, par, _ in todo for v in (op.M, op.K, par[0], par[1])])
-    _lib.call("jfx_par_prepare_many", 0 if prec == "f64" else 1, n, A, shape, F, _s())
     # complete before they are published: the next use may be on another stream
-    torch.cuda.current_stream().synchronize()
+    _lib.call("jfx_par_prepare_many", 0 if prec == "f64" else 1, n, A, shape, F, 1, _s())
     for (op, par, _), f in zip(todo, frags):
         op._prep[key] = (f, *par)
 
@@ -605,7 +604,7 @@ class ComplexAxisOperator:
         return self.stacked.prepared(prec)
 
 
-def _apply_complex(op: ComplexAxisOperator, X: torch.Tensor, axis: int) -> torch.Tensor:
+def _apply_complex(op: ComplexAxisOperator, X: torch.Tensor, axis: int, peers=()) -> torch.Tensor:
     axis = axis % X.ndim
     if X.shape[axis] != op.K:
         raise ValueError(f"apply_along: axis {axis} has length {X.shape[axis]}, operator expects {op.K}")
@@ -616,11 +615,11 @@ def _apply_complex(op: ComplexAxisOperator, X: torch.Tensor, axis: int) -> torch
     Y = torch.empty(shape, dtype=torch.complex128, device=X.device)
     if X.is_complex():
         _req(X, torch.complex128, "X")
-        Z = apply_along(op.stacked, torch.view_as_real(X).reshape(P, op.K, 2 * Q), 1)
+        Z = apply_along(op.stacked, torch.view_as_real(X).reshape(P, op.K, 2 * Q), 1, peers=peers)
         _lib.call("jfx_cplx_combine", _p(Z), _p(Y), P, op.M, Q, 0, _s())
     else:
         _req(X, torch.float64, "X")
-        Z = apply_along(op.stacked, X.reshape(P, op.K, Q), 1)
+        Z = apply_along(op.stacked, X.reshape(P, op.K, Q), 1, peers=peers)
         _lib.call("jfx_cplx_combine", _p(Z), _p(Y), P, op.M, Q, 1, _s())
     return Y
 
@@ -665,7 +664,7 @@ def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
     if getattr(op, "is_complex", False):
         if prec != "f64" or out is not None:
             raise ValueError("complex operators are applied in f64 without an out= tensor")
-        return _apply_complex(op, X, axis)
+        return _apply_complex(op, X, axis, peers)
     if X.is_complex():
         if prec != "f64":
             raise ValueError("complex arrays are transformed in f64 only")
@@ -674,7 +673,7 @@ def apply_along(op: AxisOperator, X: torch.Tensor, axis: int, prec: str = "f64",
         shape = list(X.shape)
         shape[axis] = op.M
         Y = torch.empty(shape, dtype=torch.complex128, device=X.device) if out is None else out
-        apply_along(op, torch.view_as_real(X), axis, "f64", out=torch.view_as_real(Y))
+        apply_along(op, torch.view_as_real(X), axis, "f64", out=torch.view_as_real(Y), peers=peers)
         return Y
     dt = io_dtype(prec)
     _req(X, dt, "X")

@@ -114,7 +114,7 @@ def test_one_preparation_for_a_pass(dev, calls):
     """All operators of a transform, a solve or a nonlinear term in one launch."""
     import torch
 
-    from jaxfun_amd import Div, Grad, TensorProduct, TestFunction, TrialFunction, inner
+    from jaxfun_amd import Div, Fourier, Grad, TensorProduct, TestFunction, TrialFunction, inner
 
     T = TensorProduct(_dirichlet("chebyshev", 20), _dirichlet("legendre", 31), _dirichlet("chebyshev", 26))
     c = torch.randn(18, 29, 24, dtype=torch.float64, device="cuda")
@@ -124,6 +124,10 @@ def test_one_preparation_for_a_pass(dev, calls):
     assert _prepared(calls) == 2
     T.forward(T.backward(c))
     assert _prepared(calls) == 2
+    del calls[:]
+    T = TensorProduct(Fourier(12), _dirichlet("legendre", 33))
+    T.backward(torch.randn(3, 12, 31, dtype=torch.complex128, device="cuda"))
+    assert _prepared(calls) == 1
     T = TensorProduct(_dirichlet("legendre", 20), _dirichlet("chebyshev", 31))
     v, u = TestFunction(T), TrialFunction(T)
     A = inner(v * Div(Grad(u)), sparse=True)
