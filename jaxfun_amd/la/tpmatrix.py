@@ -521,6 +521,28 @@ def axis_eig(A: np.ndarray, B: np.ndarray):
     return _axis_eig(A, B)
 
 
+def _slices(X: np.ndarray, axis: int, bits: int) -> list[np.ndarray]:
+    """X (FP64 or extended) as a sum of three FP64 arrays, the first two multiples
+    of a power of two of at most ``bits`` bits along ``axis``."""
+    u = np.ldexp(1.0, np.frexp(np.abs(X).max(axis=axis, keepdims=True).astype(np.float64))[1] - bits)
+    a = np.rint(X / u) * u
+    r = X - a
+    u = u * 2.0**-bits
+    b = np.rint(r / u) * u
+    return [s.astype(np.float64) for s in (a, b, r - b)]
+
+
+def _sliced_product(X: np.ndarray, Y: np.ndarray) -> list[np.ndarray]:
+    """X Y as FP64 terms, largest first, whose sum is within 2^-62 of |X| |Y| (row
+    and column maxima): products of the leading slices are exact in FP64 sums.  Six
+    FP64 products, where numpy multiplies extended arrays element by element (a
+    Legendre pair of 1022: 2.1 s in all, 0.4 to 0.6 this way)."""
+    n = X.shape[1]
+    bits = (53 - int(n - 1).bit_length()) // 2
+    x, y = _slices(X, 1, bits), _slices(Y, 0, bits)
+    return [x[0] @ y[0], x[0] @ y[1], x[1] @ y[0], x[0] @ y[2] + x[1] @ (y[1] + y[2]) + x[2] @ (y[0] + y[1])]
+
+
 def _extended_product(A: np.ndarray, V: np.ndarray) -> np.ndarray:
     """A V in the host's extended precision, by diagonals where A is banded."""
     A = A.astype(np.longdouble)
@@ -543,17 +565,21 @@ def _refine_eig(A: np.ndarray, B: np.ndarray, lam: np.ndarray, V: np.ndarray, W:
     eigenvalues; on Dirichlet pairs the solve's error falls from 1e-13 (Chebyshev,
     N = 128) and 6e-12 (Legendre) to below 1e-15."""
     Ve = V.astype(np.longdouble)
-    R = _extended_product(A, Ve) - _extended_product(B, Ve) * lam.astype(np.longdouble)
+    BV = _extended_product(B, Ve)
+    R = _extended_product(A, Ve) - BV * lam.astype(np.longdouble)
     P = W @ R.astype(np.float64)
     gap = lam[None, :] - lam[:, None]
     # pairs too close for a first-order correction, equal eigenvalues among them,
     # keep their vectors
     Q = np.divide(P, gap, out=np.zeros_like(P), where=(gap != 0) & (np.abs(P) <= 1e-3 * np.abs(gap)))
-    Ve = Ve + V @ Q
+    dV = V @ Q
+    Ve, BV = Ve + dV, BV + B @ dV
     V = Ve.astype(np.float64)
     W = np.linalg.inv(B @ V)
-    BV = _extended_product(B, Ve)
-    W = W + W @ (np.eye(len(lam)) - BV @ W.astype(np.longdouble)).astype(np.float64)
+    E = np.eye(len(lam))
+    for term in _sliced_product(BV, W):
+        E = E - term
+    W = W + W @ E
     return lam + np.diag(P), V, W
 
 

@@ -2,6 +2,8 @@
 time (la/tpmatrix.py axis_eig), against the fast-diagonalisation solve refined in
 extended precision."""
 
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -105,3 +107,32 @@ def test_host_factors_follow_one_order(family, monkeypatch):
     assert np.linalg.norm(K0 @ X @ M1.T + M0 @ X @ K1.T - F) <= 1e-12 * np.linalg.norm(F)
     for host, ops in ((fd.eigvecs_host, fd.V), (fd.lefts_host, fd.W)):
         assert all(np.array_equal(h, o.A64.numpy()) for h, o in zip(host, ops))
+
+
+@pytest.mark.parametrize("n,spread", [(1, 0), (2, 3), (33, 6), (200, 2), (257, 0)])
+def test_sliced_product(n, spread):
+    """Products of slices against the extended product, entries of unequal sizes and
+    a zero row and column among them."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, n)).astype(np.longdouble) * 10.0**rng.uniform(-spread, spread, (n, n))
+    X = X + X * np.longdouble(2.0)**-60
+    Y = rng.standard_normal((n, n)) * 10.0**rng.uniform(-spread, spread, (n, n))
+    if n > 2:
+        X[1], Y[:, 2] = 0.0, 0.0
+    got = sum(t.astype(np.longdouble) for t in T._sliced_product(X, Y))
+    bound = np.abs(X).max(1)[:, None] * np.abs(Y).max(0) * n
+    assert np.all(np.abs(got - X @ Y.astype(np.longdouble)) <= 2.0**-60 * bound)
+
+
+def test_diagonalisation_time():
+    """The correction's extended arithmetic stays on the order of the eigenvalue
+    solve (twice it at this size; 7 times with extended matrix products)."""
+    M, K = _pair("legendre", 1200)
+
+    def seconds(f):
+        t = time.perf_counter()
+        f()
+        return time.perf_counter() - t
+
+    T.axis_eig(K[:64, :64], M[:64, :64])
+    assert any(seconds(lambda: T.axis_eig(K, M)) < 4 * seconds(lambda: T._axis_eig(K, M)) for _ in range(3))
