@@ -448,6 +448,11 @@ def host_structure(A: np.ndarray) -> tuple | None:
     return mixes_parity(-1 if odd.any() else 1, max(0, int(-d.min())), max(0, int(d.max())))
 
 
+def fragment_values(M: int, K: int, mode: int) -> int:
+    """Values of an (M x K) operator's fragments, 0 for sizes that are not taken."""
+    return _lib.load().jfx_par_frag_elems(M, K, mode)
+
+
 class AxisOperator:
     """A constant (M x K) matrix applied along one axis, prepared per precision.
 
@@ -497,7 +502,7 @@ class AxisOperator:
             prepare_fragments((self, *(o for o in peers if type(o) is AxisOperator and o.parity is not None)), prec)
             return self._prep.get(key)
         mode, sgn, p, q = self.parity or (PAR_DENSE, 1, -1, -1)
-        n = _lib.load().jfx_par_frag_elems(self.M, self.K, mode)
+        n = fragment_values(self.M, self.K, mode)
         if n == 0:
             return None
         f = torch.empty(n, dtype=io_dtype(prec), device=self.A64.device)
@@ -557,7 +562,7 @@ def prepare_fragments(ops, prec: str = "f64") -> None:
     for op in ops:
         if type(op) is AxisOperator and not op.once and key not in op._prep and all(op is not o for o, _, _ in todo):
             par = op.parity or (PAR_DENSE, 1, -1, -1)
-            n = _lib.load().jfx_par_frag_elems(op.M, op.K, par[0])
+            n = fragment_values(op.M, op.K, par[0])
             if n == 0:
                 op._prep[key] = None
             else:

@@ -75,8 +75,13 @@ class BaseMatrix:
 
     def operator(self):
         if self._op is None:
-            self._op = K.ComplexAxisOperator(self.todense()) if self.is_complex else \
-                K.AxisOperator(self.todense(), K.host_structure(self._host_data))
+            if self.is_complex:
+                self._op = K.ComplexAxisOperator(self.todense())
+            else:
+                # sizes beyond the kernels that use a structure: not worth looking for
+                # one (0.1 s in a banded 4096 x 4096 matrix)
+                par = K.host_structure(self._host_data) if K.fragment_values(*self.shape, K.PAR_MIX) else None
+                self._op = K.AxisOperator(self.todense(), par)
         return self._op
 
     def transposed_operator(self):

@@ -136,3 +136,16 @@ def test_diagonalisation_time():
 
     T.axis_eig(K[:64, :64], M[:64, :64])
     assert any(seconds(lambda: T.axis_eig(K, M)) < 4 * seconds(lambda: T._axis_eig(K, M)) for _ in range(3))
+
+
+def test_structure_is_looked_for_where_it_is_used(monkeypatch):
+    """A matrix finds its structure for its operator up to the sizes that kernels
+    take, 1024 x 512, and never beyond."""
+    looked = []
+    structure = T.K.host_structure
+    monkeypatch.setattr(T.K, "device", lambda: torch.device("cpu"))
+    monkeypatch.setattr(T.K, "host_structure", lambda A: looked.append(A.shape) or structure(A))
+    for shape, taken in (((6, 6), True), ((1024, 512), True), ((1025, 512), False), ((40, 513), False)):
+        op = T.Matrix(np.eye(*shape)).operator()
+        assert op.parity == (T.K.mixes_parity(1, 0, 0) if taken else None)
+        assert (shape in looked) == taken
