@@ -16,8 +16,8 @@
 //   4  Y += s S1^T, accumulated in registers over the strips
 // U comes from L2 in every strip.  What bounds it: FP64 products (the strip's four
 // steps are 584 MFMAs per SIMD, 93 us for that problem) with four barriers a strip;
-// measured 194 us for 256 problems, axis by axis 354 us (FP32 in and out, with
-// bf16x6 contractions axis by axis: 185 against 189-196 us).
+// measured 173 us for 256 problems, axis by axis 328 us (FP32 in and out, with
+// bf16x6 contractions axis by axis: 163 against 181 us).
 #include "par_blocks.h"
 
 namespace jfx {
