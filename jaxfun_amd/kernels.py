@@ -41,6 +41,29 @@ def _s():
     return torch.cuda.current_stream().cuda_stream
 
 
+_stream_of = getattr(torch._C, "_cuda_getCurrentStream", None)
+
+
+def _stream_id() -> tuple:
+    """(stream id, device index, device type) of the current stream, from which
+    PyTorch's own streams can be named again later."""
+    if _stream_of is not None:
+        return _stream_of(torch.cuda.current_device())
+    s = torch.cuda.current_stream()
+    return s.stream_id, s.device_index, s.device_type
+
+
+def _wait_for(stream: tuple) -> None:
+    """The current stream's next work follows what ``stream`` (:func:`_stream_id`)
+    has been given so far.  Stream 0 and odd ids are PyTorch's streams, which it
+    never destroys; others are foreign handles that may be gone by now: the device."""
+    sid, index, kind = stream
+    if sid == 0 or sid & 1:
+        torch.cuda.current_stream().wait_stream(torch.cuda.Stream(stream_id=sid, device_index=index, device_type=kind))
+    else:
+        torch.cuda.synchronize()
+
+
 def _req(t: torch.Tensor, dtype: torch.dtype, name: str) -> None:
     if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous():
         return
@@ -475,7 +498,7 @@ class AxisOperator:
         self.M, self.K = self.A64.shape
         self.parity = parity
         self.once = once
-        self._made_on = _s() if self.A64.is_cuda else None  # the stream that A64 is ordered on
+        self._made_on = _stream_id() if self.A64.is_cuda else None  # the stream that A64 is ordered on
         self._prep: dict[str, tuple] = {}
 
     def t(self) -> "AxisOperator":
@@ -570,8 +593,8 @@ def prepare_fragments(ops, prec: str = "f64") -> None:
     if not todo or torch.cuda.is_current_stream_capturing():
         return
     # what is kept must not be cut from a matrix that another stream is still computing
-    for raw in {op._made_on for op, _, _ in todo} - {_s()}:
-        torch.cuda.current_stream().wait_stream(torch.cuda.ExternalStream(raw) if raw else torch.cuda.default_stream())
+    for stream in {op._made_on for op, _, _ in todo} - {_stream_id()}:
+        _wait_for(stream)
     n = len(todo)
     frags = [torch.empty(m, dtype=io_dtype(prec), device=op.A64.device) for op, _, m in todo]
     A = (ctypes.c_void_p * n)(*[op.A64.data_ptr() for op, _, _ in todo])

@@ -160,7 +160,7 @@ def test_operators_cut_together_as_alone(dev, prec):
         assert fa is None or (fa[1:] == fb[1:] and torch.equal(fa[0], fb[0]))
 
 
-@pytest.mark.parametrize("side", ["built", "used"])
+@pytest.mark.parametrize("side", ["built", "used", "foreign"])
 def test_operators_built_on_another_stream(dev, side):
     """An operator whose matrix is still being computed on its own stream when a
     product on another stream cuts it: the kept fragments are the finished matrix's."""
@@ -175,7 +175,9 @@ def test_operators_built_on_another_stream(dev, side):
     dst, big = torch.zeros_like(src), torch.full((4096, 4096), 1e-4, dtype=torch.float64, device="cuda")
     torch.cuda.synchronize()
     other = torch.cuda.Stream()
-    build, use = (other, torch.cuda.current_stream()) if side == "built" else (torch.cuda.current_stream(), other)
+    build, use = (torch.cuda.current_stream(), other) if side == "used" else (other, torch.cuda.current_stream())
+    if side == "foreign":
+        build = torch.cuda.ExternalStream(other.cuda_stream)
     with torch.cuda.stream(build):
         for _ in range(8):  # some 15 ms ahead of the matrix
             big = big @ big
