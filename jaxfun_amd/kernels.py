@@ -577,7 +577,7 @@ class AxisOperator:
 
 def prepare_fragments(ops, prec: str = "f64") -> None:
     """Cut the fragments of every operator in ``ops`` that has none yet, in one
-    launch with one wait (22 us for one operator, 31 for four; most of it is the
+    launch with one wait (20 us for one operator, 28 for four; most of it is the
     wait).  Inside a graph capture this does nothing, see
     :meth:`AxisOperator.fragments`."""
     key = PAR_KEYS[prec]
@@ -754,9 +754,8 @@ def weak_laplacian(B: AxisOperator, D: AxisOperator, TB: AxisOperator, TD: AxisO
     if max(n, Q) > 128 or any(o.parity is None or o.parity[0] != md or (o.M, o.K) != sz for o, md, sz in (
             (B, PAR_EVAL, (Q, n)), (D, PAR_EVAL, (Q, n)), (TB, PAR_PROJ, (n, Q)), (TD, PAR_PROJ, (n, Q)))):
         return None
-    prepare_fragments((B, D, TB, TD))
-    fr = [o.fragments("f64") for o in (B, D, TB, TD)]
-    if any(f is None for f in fr):
+    fr = _kept_fragments((B, D, TB, TD))
+    if fr is None:
         return None
     _req(U, torch.float64, "U")
     _req(k, torch.float64, "k")
@@ -825,6 +824,15 @@ def plane_ok(op0: AxisOperator, op1: AxisOperator, prec: str) -> bool:
     return prec in PLANE_PRECISIONS and max(op0.M, op0.K, op1.M, op1.K) <= 128
 
 
+def _kept_fragments(ops):
+    """FP64 fragments of every operator, cut together on first use; None if one has none."""
+    fr = [o._prep.get("par_f64") for o in ops]
+    if None in fr:
+        prepare_fragments(ops)
+        fr = [o._prep.get("par_f64") for o in ops]
+    return None if None in fr else fr
+
+
 def _slab_fragments(ops):
     """FP64 fragments of structured operators for the fused slab kernels
     (csrc/plane_par.hip): one structure, at most 128 rows and columns; else None."""
@@ -832,11 +840,7 @@ def _slab_fragments(ops):
         if type(o) is not AxisOperator or o.parity is None or o.M > 128 or o.K > 128 or \
                 o.parity[0] != ops[0].parity[0]:
             return None
-    out = [o._prep.get("par_f64") for o in ops]
-    if None in out:
-        prepare_fragments(ops)
-        out = [o._prep.get("par_f64") for o in ops]
-    return None if None in out else out
+    return _kept_fragments(ops)
 
 
 def slab_pays(op0, op1, nslabs: int) -> bool | None:
